@@ -417,7 +417,7 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
       }
     }
 
-  if (special) {
+  if (special && blockIdx.y == 0) {
     // bin M/2 (self-paired): gamma = e^{i pi dr/2}; its c2r pre-pass value is
     // conj(Ys) for every rate
     for (int j = tid; j < a.Nr; j += T) {
@@ -444,13 +444,15 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
     }
     // groups from the middle rates outwards, so that the rates k3 reads
     // first (Nr-1, 0, Nr-2, 1, ...) are the ones written last
-    const int g0 = ((npairs - 1) / NPG) * NPG;
+    const int ng = (npairs + NPG - 1) / NPG;
+    const int glo = group_first(ng, blockIdx.y, gridDim.y) * NPG;
+    const int g0 = (group_first(ng, blockIdx.y + 1, gridDim.y) - 1) * NPG;
 #pragma unroll
     for (int i = 0; i < PP; ++i)  // e^{2 pi i k r_g0/Nf}
       zp[i] = cis64f(static_cast<double>(kA[i]) * (a.hz0 + static_cast<double>(g0) * a.hd2));
     c32* cur = buf;
     c32* nxt = buf2;
-    for (int p0 = g0; p0 >= 0; p0 -= NPG) {
+    for (int p0 = g0; p0 >= glo; p0 -= NPG) {
       const int np = min(NPG, npairs - p0);
 #pragma unroll
       for (int i = 0; i < PP; ++i) zq[i] = zp[i];
@@ -515,11 +517,15 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
     }
   } else {
     // ---- chirp-Z for every rate, c2r pre-pass, inverse DFT_N1, store
+    constexpr int JG = ROWS / 2;
+    const int ng = (a.Nr + JG - 1) / JG;
+    const int jlo = group_first(ng, blockIdx.y, gridDim.y) * JG;
+    const int jhi = min(a.Nr, group_first(ng, blockIdx.y + 1, gridDim.y) * JG);
     c64 gam[PP], z[PP];
   #pragma unroll
     for (int i = 0; i < PP; ++i) {
       gam[i] = cis64f(static_cast<double>(kA[i]) * a.hd2);
-      z[i] = {1.0, 0.0};
+      z[i] = cis64f(static_cast<double>(kA[i]) * (static_cast<double>(jlo) * a.hd2));
     }
 
     // Rate groups of JG rates (2 JG rows: columns A and B of each rate).  The
@@ -527,14 +533,13 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
     // barrier per group (after the c2r pre-pass writes) also orders a group's
     // writes after the previous-but-one group's FFT reads.  Each wavefront
     // then runs the inverse DFT_N1 of its own rows in place and stores them.
-    constexpr int JG = ROWS / 2;
     constexpr int NW = T / 64;      // wavefronts
     constexpr int RPW = ROWS / NW;  // rows per wavefront
     static_assert(RPW * NW == ROWS && RPW * fft_max_nr<N1>() <= 64, "one butterfly per lane and pass");
     const int wv = tid >> 6, lane = tid & 63;
     c32* cur = buf;
     c32* nxt = buf2;
-    for (int j0 = 0; j0 < a.Nr; j0 += JG) {
+    for (int j0 = jlo; j0 < jhi; j0 += JG) {
       const int nj = min(JG, a.Nr - j0);
   #pragma unroll
       for (int jj = 0; jj < JG; ++jj) {
@@ -806,10 +811,19 @@ int launch_k1(const FastPlan* p, const float* spec, c32* G, int64_t Nt, hipStrea
 int fast_input(FastPlan* p, const float* spec, hipStream_t st) { return launch_k1(p, spec, p->G, p->Nt, st); }
 
 template <int N1, int N2>
-static int launch_k2(const K2Args& a, int NT, bool paired, hipStream_t st) {
-  constexpr unsigned grid = N2 / 2;
+static int launch_k2(const K2Args& a, int NT, bool paired, int64_t ncu, hipStream_t st) {
   constexpr unsigned TB = N1 < 512 ? N1 : 512;
   constexpr int RW = k2_rows(N1);
+  // rate groups over blockIdx.y.  Each part repeats the input phase, worth
+  // about three groups of rates, and the waves a CU holds are bounded by
+  // VGPRs (N1 <= 128) or LDS (256: 8, 512: 16).  At 129 rates, one part ->
+  // this rule: 2^16 channels 69.8 -> 29.5 us, 2^17 72.6 -> 36.6, 2^18
+  // 93.0 -> 61.7; a second part only costs at 2^19 (110.8 -> 128.3) and 2^20
+  // (181 -> 205), whose blocks fill the chip.
+  constexpr int WAVES = N1 >= 512 ? 16 : (N1 == 256 ? 8 : 12);
+  const int units = (paired && NT == 16) ? a.Nr / 2 + 1 : a.Nr;  // rate pairs or rates
+  const int per = (paired && NT == 16) ? RW / 4 : RW / 2;
+  const dim3 grid(N2 / 2, group_parts((units + per - 1) / per, N2 / 2, TB, WAVES, 3, ncu));
   if (paired && NT == 16) {
     k2_czt<N1, N2, 16, RW, true><<<grid, TB, 0, st>>>(a);
     ZDT_CHECK_LAUNCH("k2_czt");
@@ -869,28 +883,28 @@ int fast_run(FastPlan* p, float r0, int wkind, const float* window, float* dest,
     const int key = p->N1 * 2048 + p->N2;
     switch (key) {
       case 64 * 2048 + 512:
-        ZDT_TRY((launch_k2<64, 512>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<64, 512>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 64 * 2048 + 1024:
-        ZDT_TRY((launch_k2<64, 1024>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<64, 1024>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 128 * 2048 + 512:
-        ZDT_TRY((launch_k2<128, 512>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<128, 512>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 256 * 2048 + 512:
-        ZDT_TRY((launch_k2<256, 512>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<256, 512>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 512 * 2048 + 512:
-        ZDT_TRY((launch_k2<512, 512>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<512, 512>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 128 * 2048 + 1024:
-        ZDT_TRY((launch_k2<128, 1024>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<128, 1024>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 256 * 2048 + 1024:
-        ZDT_TRY((launch_k2<256, 1024>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<256, 1024>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       case 512 * 2048 + 1024:
-        ZDT_TRY((launch_k2<512, 1024>(a, p->NT, paired, st)));
+        ZDT_TRY((launch_k2<512, 1024>(a, p->NT, paired, p->resident_blocks / 2, st)));
         break;
       default:
         return fail(ZDT_ENOTSUP, "fused path: N1=%d N2=%d", p->N1, p->N2);

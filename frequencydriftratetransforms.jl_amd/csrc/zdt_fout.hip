@@ -267,7 +267,7 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
   const int64_t kA = cA + static_cast<int64_t>(N2) * k1A;
   const c32 WA = cis_rev(-static_cast<float>(kA) / static_cast<float>(a.Nf));
   const float h = 0.5f * a.oscale;
-  if (special) {
+  if (special && blockIdx.y == 0) {
     for (int j = tid; j < a.Nr; j += T) {
       const c32 y = a.Yc[static_cast<int64_t>(j) * a.M + HALF];  // bin M/2: k2 = 0, k1 = N1/2
       a.yhalf[j] = {y.x * a.oscale, -y.y * a.oscale};
@@ -296,8 +296,11 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
       }
     }
   };
-  load(0);
-  for (int j0 = 0; j0 < a.Nr; j0 += JG) {
+  const int ng = (a.Nr + JG - 1) / JG;
+  const int jlo = group_first(ng, blockIdx.y, gridDim.y) * JG;
+  const int jhi = min(a.Nr, group_first(ng, blockIdx.y + 1, gridDim.y) * JG);
+  load(jlo);
+  for (int j0 = jlo; j0 < jhi; j0 += JG) {
     const int nj = min(JG, a.Nr - j0);
 #pragma unroll
     for (int jj = 0; jj < JG; ++jj) {
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
       }
     }
     __syncthreads();
-    if (j0 + JG < a.Nr) load(j0 + JG);
+    if (j0 + JG < jhi) load(j0 + JG);
     const int nrw = min(RPW, max(0, 2 * nj - wv * RPW));
     wave_fft<N1, true, 1, true>(cur + wv * RPW * P, P, nrw, twl, lane, [&](int f, int jx, auto& v) {
       constexpr int RL = sizeof(v) / sizeof(c32);
@@ -621,7 +624,10 @@ __global__ __launch_bounds__(N1 < 1024 ? N1 : 1024) void k2_input(K2iArgs a) {
     twS1[i] = cis_rev(static_cast<float>((n1 * colB) & (a.M - 1)) * invM);
   }
 
-  for (int t0 = 0; t0 < a.Nt; t0 += TG) {
+  const int ng = (a.Nt + TG - 1) / TG;
+  const int tlo = group_first(ng, blockIdx.y, gridDim.y) * TG;
+  const int thi = min(a.Nt, group_first(ng, blockIdx.y + 1, gridDim.y) * TG);
+  for (int t0 = tlo; t0 < thi; t0 += TG) {
     const int nt = min(TG, a.Nt - t0);
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
@@ -743,9 +749,14 @@ int fast_out_create(int64_t Nf, int64_t Nr, int precision, FastPlan** out) {
 }
 
 template <int N1, int N2>
-static int launch_k2c(const K2cArgs& a, hipStream_t st) {
+static int launch_k2c(const K2cArgs& a, int64_t ncu, hipStream_t st) {
   if constexpr (N1 <= 512) {
-    k2_c2r<N1, N2, k2_rows(N1)><<<N2 / 2, N1, 0, st>>>(a);
+    // rate groups over blockIdx.y: at 257 rates, one part -> this rule, 2^16
+    // channels 79.6 -> 24.0 us, 2^17 86.8 -> 51, 2^18 123 -> 100, 2^19
+    // 227 -> 220; nothing at 2^20
+    constexpr int JG = k2_rows(N1) / 2;
+    const dim3 grid(N2 / 2, group_parts((a.Nr + JG - 1) / JG, N2 / 2, N1, 24, 2, ncu));
+    k2_c2r<N1, N2, k2_rows(N1)><<<grid, N1, 0, st>>>(a);
   } else {
     k2_c2r_wave<N1, N2><<<N2 / 2, 512, 0, st>>>(a);
   }
@@ -754,10 +765,15 @@ static int launch_k2c(const K2cArgs& a, hipStream_t st) {
 }
 
 template <int N1, int N2>
-static void launch_k2i(const K2iArgs& a, hipStream_t st) {
+static void launch_k2i(const K2iArgs& a, int64_t ncu, hipStream_t st) {
   // two ping-pong buffers of ~36 KB each: 8 rows up to N1 = 512, then 4, 2
   constexpr int ROWS = N1 <= 512 ? 8 : (N1 == 1024 ? 4 : 2);
-  k2_input<N1, N2, ROWS><<<N2 / 2, (N1 < 1024 ? N1 : 1024), 0, st>>>(a);
+  // groups of time steps over blockIdx.y up to 16 wavefronts a CU (the LDS
+  // rows bound them there from N1 = 512 on): 2^16 x 279 247 -> 33 us, 2^17 x
+  // 60 57.9 -> 20, 2^18 x 60 64.5 -> 28.9, 2^19 x 32 45.1 -> 32.4
+  constexpr int T = N1 < 1024 ? N1 : 1024;
+  const dim3 grid(N2 / 2, group_parts((a.Nt + ROWS / 2 - 1) / (ROWS / 2), N2 / 2, T, 16, 1, ncu));
+  k2_input<N1, N2, ROWS><<<grid, T, 0, st>>>(a);
 }
 
 int fast_out_input(FastPlan* p, const float* spec, int64_t Nt, c32* Ft, hipStream_t st) {
@@ -773,25 +789,25 @@ int fast_out_input(FastPlan* p, const float* spec, int64_t Nt, c32* Ft, hipStrea
   ProfScope ps(st, "k2_input", 16.0 * p->M * Nt);
   switch (p->N1 * 2048 + p->N2) {
     case 64 * 2048 + 512:
-      launch_k2i<64, 512>(a, st);
+      launch_k2i<64, 512>(a, p->resident_blocks / 2, st);
       break;
     case 64 * 2048 + 1024:
-      launch_k2i<64, 1024>(a, st);
+      launch_k2i<64, 1024>(a, p->resident_blocks / 2, st);
       break;
     case 128 * 2048 + 1024:
-      launch_k2i<128, 1024>(a, st);
+      launch_k2i<128, 1024>(a, p->resident_blocks / 2, st);
       break;
     case 256 * 2048 + 1024:
-      launch_k2i<256, 1024>(a, st);
+      launch_k2i<256, 1024>(a, p->resident_blocks / 2, st);
       break;
     case 512 * 2048 + 1024:
-      launch_k2i<512, 1024>(a, st);
+      launch_k2i<512, 1024>(a, p->resident_blocks / 2, st);
       break;
     case 1024 * 2048 + 1024:
-      launch_k2i<1024, 1024>(a, st);
+      launch_k2i<1024, 1024>(a, p->resident_blocks / 2, st);
       break;
     case 2048 * 2048 + 1024:
-      launch_k2i<2048, 1024>(a, st);
+      launch_k2i<2048, 1024>(a, p->resident_blocks / 2, st);
       break;
     default:
       return fail(ZDT_ENOTSUP, "fused output input: N1=%d N2=%d", p->N1, p->N2);
@@ -882,25 +898,25 @@ int fast_out_run(FastPlan* p, const c32* F, int64_t ldF, bool ftrans, int Nt, fl
     ProfScope ps(st, "k2_c2r", 16.0 * p->M * p->Nr);
     switch (p->N1 * 2048 + p->N2) {
       case 64 * 2048 + 512:
-        ZDT_TRY((launch_k2c<64, 512>(a, st)));
+        ZDT_TRY((launch_k2c<64, 512>(a, p->resident_blocks / 2, st)));
         break;
       case 64 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<64, 1024>(a, st)));
+        ZDT_TRY((launch_k2c<64, 1024>(a, p->resident_blocks / 2, st)));
         break;
       case 128 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<128, 1024>(a, st)));
+        ZDT_TRY((launch_k2c<128, 1024>(a, p->resident_blocks / 2, st)));
         break;
       case 256 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<256, 1024>(a, st)));
+        ZDT_TRY((launch_k2c<256, 1024>(a, p->resident_blocks / 2, st)));
         break;
       case 512 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<512, 1024>(a, st)));
+        ZDT_TRY((launch_k2c<512, 1024>(a, p->resident_blocks / 2, st)));
         break;
       case 1024 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<1024, 1024>(a, st)));
+        ZDT_TRY((launch_k2c<1024, 1024>(a, p->resident_blocks / 2, st)));
         break;
       case 2048 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<2048, 1024>(a, st)));
+        ZDT_TRY((launch_k2c<2048, 1024>(a, p->resident_blocks / 2, st)));
         break;
       default:
         return fail(ZDT_ENOTSUP, "fused output: N1=%d N2=%d", p->N1, p->N2);
