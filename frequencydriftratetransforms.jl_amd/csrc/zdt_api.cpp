@@ -297,7 +297,7 @@ int run_impl(zdt_ws* ws, float r0, int wkind, const float* window, float* dest) 
     return ZDT_OK;
   }
   if (ws->fout != nullptr) {
-    ZDT_TRY(fast_out_run(ws->fout, ws->Ft, ws->Nk, true, static_cast<int>(ws->Nt), r0, ws->dr, wkind, window, dest,
+    ZDT_TRY(fast_out_run(ws->fout, ws->Ft, static_cast<int>(ws->Nt), r0, ws->dr, wkind, window, dest,
                          out_scale(ws), ws->stream));
     ws->ys_fast = false;
     ws->ys_fout = (dest == nullptr);
@@ -478,7 +478,7 @@ int run_devstats(zdt_ws* ws, float r0, float* dest, double* colmean, double* col
   }
   if (ws->fout != nullptr) {
     RunMax rm_(ws->fout, smax);
-    ZDT_TRY(fast_out_run(ws->fout, ws->Ft, ws->Nk, true, static_cast<int>(ws->Nt), r0, ws->dr, ZDT_WINDOW_RECT,
+    ZDT_TRY(fast_out_run(ws->fout, ws->Ft, static_cast<int>(ws->Nt), r0, ws->dr, ZDT_WINDOW_RECT,
                          nullptr, dest, out_scale(ws), ws->stream, colmean, colvar));
     ws->ys_fast = false;
     ws->ys_fout = false;

@@ -34,15 +34,14 @@ int fast_plan_n2(const FastPlan* p);
 // doubles of k3's statistics partials (held by every fused plan)
 int64_t fast_stats_doubles(int64_t Nf, int64_t Nr);
 
-// Time steps the fused output takes (the chirp-Z runs in 64-step chunks
-// above 64; the input spectrum Ft holds Nk x Nt entries)
+// Time steps the fused output takes (the input spectrum Ft holds Nk x Nt
+// entries; at most FOLD_MAX_NT, czt_fold.h)
 constexpr int64_t FOUT_MAX_NT = 1024;
 
 // Fused output for power-of-two Nf in [2^16, 2^22] and Nt <= FOUT_MAX_NT: the chirp-Z
 // per bin from the input spectrum F, then the c2r through k2_c2r and k3
-// (fast_output).  F is either natural (Nk x Nt, column stride ldF) or, with
-// ftrans, the layout fast_out_input writes: (Nk-1) x Nt entries [t][k2][k1]
-// (bin k2 + N2 k1) followed by the Nt Nyquist bins.
+// (fast_output).  F is in the layout fast_out_input writes: (Nk-1) x Nt entries
+// [t][k2][k1] (bin k2 + N2 k1) followed by the Nt Nyquist bins.
 bool fast_out_supported(int64_t Nf, int64_t Nt, int64_t Nr);
 int64_t fast_out_bytes(int64_t Nf, int64_t Nr);
 // precision: as fast_create (the split modes change k1 and k3)
@@ -51,8 +50,7 @@ int fast_out_create(int64_t Nf, int64_t Nr, int precision, FastPlan** out);
 int fast_out_input(FastPlan* p, const float* spec, int64_t Nt, c32* Ft, hipStream_t st);
 // natural-layout F from Ft (for the step functions)
 int fast_out_unpack_F(FastPlan* p, const c32* Ft, int64_t Nt, c32* F, hipStream_t st);
-int fast_out_run(FastPlan* p, const c32* F, int64_t ldF, bool ftrans, int Nt, float r0, float dr, int wkind,
-                 const float* window, float* dest, double scale, hipStream_t st, double* colmean = nullptr,
-                 double* colvar = nullptr);
+int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkind, const float* window, float* dest,
+                 double scale, hipStream_t st, double* colmean = nullptr, double* colvar = nullptr);
 
 }  // namespace zdt

@@ -25,7 +25,7 @@
 // recurrence.  A thread owns a bin k and its Hermitian partner M-k, for which
 // gamma_{M-k}^j = e^{i pi dr j} conj(gamma_k^j), so the partner's powers cost
 // one multiply by a per-rate table.  Symmetric rate sets take the paired
-// evaluation of k2_czt<..., PAIRED> (reinsch2, zdt_fast_dev.h).
+// evaluation of k2_czt<..., PAIRED> (reinsch_quad, zdt_fast_dev.h).
 //
 // The device building blocks live in zdt_fast_dev.h, the plan in
 // zdt_fast_plan.h, and the fused output (Nt up to 64, Nf up to 2^22), which
@@ -246,7 +246,7 @@ struct K2Args {
 // rc = r0 + (Nr-1) dr/2 instead of r0, so that the remaining rates
 // r_j - rc = (j - (Nr-1)/2) dr are mirrored: rates j and Nr-1-j of a bin are
 // its sums at z = e^{2 pi i k (r_j - rc)/Nf} and conj(z) and come from one
-// reinsch2 (partner bin: z = e^{i pi (r_j - rc)} conj(z_k)); a group of
+// reinsch_quad (partner bin: z = e^{i pi (r_j - rc)} conj(z_k)); a group of
 // ROWS/2 rates holds the pairs (j, Nr-1-j), (j+1, Nr-2-j), ...
 template <int N1, int N2, int NT, int ROWS, bool PAIRED = false>
 __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_czt(K2Args a) {

@@ -2,7 +2,7 @@
 // where the chirp-Z coefficients of a bin do not fit k2's registers (Nt > 16)
 // or the rows do not fit its LDS (Nf > 2^20):
 //   k1_input + k2_input   input!: the four-step r2c into Ft[t][k2][k1]
-//   czt_reinsch_col       the chirp-Z per bin -> Yc[j][k2][k1]
+//   czt_fold_col          the chirp-Z per bin -> Yc[j][k2][k1]
 //   k2_c2r / k2_c2r_wave  c2r pre-pass and inverse DFT_N1 -> B (as k2)
 //   k3_output             as in the fused path (fast_output)
 #include <hip/hip_runtime.h>
@@ -19,217 +19,72 @@ namespace zdt {
 // ---------------------------------------------------------------- fused output for Nt > 16
 //
 // For power-of-two Nf with Nt up to FOUT_MAX_NT (more coefficients than k2
-// keeps in registers; above 64 the chirp-Z runs in 64-step chunks) the
-// chirp-Z runs per bin (czt_reinsch_col) and the output irfft reuses the
+// keeps in registers) the
+// chirp-Z runs per bin (czt_fold_col) and the output irfft reuses the
 // second half of k2 and k3:
-//   czt_reinsch_col  Ys[k, j] -> Yc[j][k2][k1] (k = k2 + N2 k1 < M), Ys[M, j] -> yM[j]
+//   czt_fold_col     Ys[k, j] -> Yc[j][k2][k1] (k = k2 + N2 k1 < M), Ys[M, j] -> yM[j]
 //   k2_c2r           per Hermitian column pair: c2r pre-pass, inverse DFT_N1
 //                    over k1 (one wavefront per row) -> B, bin M/2 -> yhalf
 //   k3_output        as in the fused path
 // which moves the spectra through HBM twice instead of once per FFT pass.
 
 struct CztColArgs {
-  const c32* F;  // Nk x Nt, natural layout (column stride ldF), or with ftrans
-                 // [Nt][N2][N1] (bin k2 + N2 k1 at [t][k2][k1]) then [Nt] bin M
-  int64_t ldF;
-  int ftrans;
+  const c32* F;  // [Nt][N2][N1] (bin k2 + N2 k1 at [t][k2][k1]) then [Nt] bin M
   c32* Yc;       // [Nr][N2][N1]
   c32* yM;       // [Nr]
   int64_t M, Nf;
   int logN1, logN2;
-  int Nt, Nr;
-  double hd2;    // dr/Nf
+  FoldRates r;
+  double r0, dr;
   int wkind;
   const float* wcustom;
   float scale;
-  double hc;     // czt_reinsch_col: rc/Nf, the coefficients' pre-rotation (centre rate rc)
-  double hz;     // czt_reinsch_col: (r0 - rc)/Nf
 };
 
-// The bin of a thread: one thread per bin; a block covers 16 columns k2 x 16
-// rows k1 (so the Nr stores of a wavefront are four 128-byte rows of Yc); the
-// last block's thread 0 takes the Nyquist bin M.  Returns false for the idle
-// threads of the last block.
-struct ColBin {
-  int64_t k;
-  c32* dst;
-  int64_t stride;  // between rates in dst
-  int64_t fo, fs;  // F offset of the bin and its step in t
-};
-
-__device__ __forceinline__ bool col_bin(const CztColArgs& a, ColBin& b) {
-  const int ntk1 = (1 << a.logN1) >> 4;
-  const int tile = blockIdx.x;
-  if (tile * 256 >= a.M) {
-    if (threadIdx.x != 0) return false;
-    b.k = a.M;
-    b.dst = a.yM;
-    b.stride = 1;
-    b.fo = a.ftrans ? a.M * a.Nt : a.M;
-    b.fs = a.ftrans ? 1 : a.ldF;
-  } else {
-    const int k2 = ((tile / ntk1) << 4) + (threadIdx.x >> 4);
-    const int k1 = ((tile % ntk1) << 4) + (threadIdx.x & 15);
-    b.k = k2 + (static_cast<int64_t>(k1) << a.logN2);
-    b.dst = a.Yc + (static_cast<int64_t>(k2) << a.logN1) + k1;
-    b.stride = a.M;
-    b.fo = a.ftrans ? (static_cast<int64_t>(k2) << a.logN1) + k1 : b.k;
-    b.fs = a.ftrans ? a.M : a.ldF;
-  }
-  return true;
-}
-
-// The chirp-Z of a bin for the rates in mirrored pairs: with the centre rate
-// rc = r0 + (Nr-1) dr/2 folded into the coefficients (c_t e^{2 pi i k t rc/Nf}),
-// rates j and Nr-1-j are the sums at z = e^{i theta} and conj(z),
-// theta = 2 pi k (r_j - rc)/Nf, and come from one Reinsch-modified Goertzel
-// recurrence (C. Reinsch, 1967; J. Oliver, "An error analysis of the modified
-// Clenshaw method", 1977) over the real and the imaginary parts of the
-// coefficients.  With s = sign(cos theta) and lambda = 2 (cos theta - s),
-//   D_t = a_t + lambda U_{t+1} + s D_{t+1},  U_t = D_t + s U_{t+1}  (t = Nt-1 .. 1),
-//   sum a_t cos(t theta) = a_0 + (lambda/2) U_1 + s D_1,  sum a_t sin(t theta) = U_1 sin theta:
-// three FMAs per term and part, six per term for both rates against eight
-// for two complex Horner evaluations.  lambda comes from the FP64 cos theta,
-// so no accuracy is lost near theta = 0 or pi (where Goertzel's rounded
-// 2 cos theta would lose it).  The middle rate of an odd Nr is its own
-// partner.
-template <int NT>
-__global__ __launch_bounds__(256) void czt_reinsch_col(CztColArgs a) {
-  ColBin bin;
-  if (!col_bin(a, bin)) return;
-  const double kd = static_cast<double>(bin.k);
-  const float w = fast_window(a.wkind, a.wcustom, bin.k, a.Nf) * a.scale;
-  float cr[NT], ci[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t < a.Nt) {
-      c32 f = a.F[bin.fo + static_cast<int64_t>(t) * bin.fs];
-      if (a.hc != 0.0) f = cmul(f, cis_nh(kd * static_cast<double>(t), a.hc));  // uniform
-      cr[t] = f.x * w;
-      ci[t] = f.y * w;
-    } else {
-      cr[t] = 0.0f;
-      ci[t] = 0.0f;
-    }
-  }
-  const c64 g = cis64f(kd * a.hd2);
-  c64 z = cis64f(kd * a.hz);  // e^{2 pi i k (r_0 - rc)/Nf}
-  const int npair = (a.Nr + 1) / 2;  // j < npair; partner Nr-1-j
-  // two rate pairs (j, j+1) per iteration: four independent recurrences
-  int j = 0;
-  for (; j + 1 < npair; j += 2) {
-    const c64 z1 = cmul(z, g);
-    c32 y0, y0c, y1, y1c;
-    reinsch_quad<NT>([&](int t) { return cr[t]; }, [&](int t) { return ci[t]; }, z, [&](int t) { return cr[t]; },
-                     [&](int t) { return ci[t]; }, z1, y0, y0c, y1, y1c);
-    const int jp = a.Nr - 1 - j;  // > j + 1: both partners are distinct
-    bin.dst[static_cast<int64_t>(j) * bin.stride] = y0;
-    bin.dst[static_cast<int64_t>(jp) * bin.stride] = y0c;
-    bin.dst[static_cast<int64_t>(j + 1) * bin.stride] = y1;
-    if (jp - 1 != j + 1) bin.dst[static_cast<int64_t>(jp - 1) * bin.stride] = y1c;
-    z = cmul(z1, g);
-  }
-  if (j < npair) {
-    const int jp = a.Nr - 1 - j;
-    c32 yz, yc;
-    reinsch_split<NT>(cr, ci, z, yz, yc);
-    bin.dst[static_cast<int64_t>(j) * bin.stride] = yz;
-    if (jp != j) bin.dst[static_cast<int64_t>(jp) * bin.stride] = yc;
-  }
-}
-
-// Nt > 64: the sum in chunks of 64 time steps, sum_t c_t z^t =
-// sum_q z^{64q} P_q(z), with NC (a power of two >= ceil(Nt/64)) adjacent
-// lanes per bin: lane q evaluates P_q for every rate pair (the recurrence of
-// czt_reinsch_col, two pairs at a time), scales it by z^{64q} (conj for the
-// partner rate; FP64 recurrence over the rates) and the NC partial sums are
-// added across the lanes (butterfly shuffles), so each Yc entry is written
-// once.  Bins are numbered g = 0 .. M (g = M: the Nyquist bin) in col_bin's
-// tile order.
-template <int NC>
-__global__ __launch_bounds__(256) void czt_reinsch_col_split(CztColArgs a) {
-  constexpr int NT = 64;
+// The chirp-Z of every bin, folded (czt_fold.h), for the rates in mirrored
+// pairs about the centre rate rc = r0 + (Nr-1) dr/2: rates j and Nr-1-j are
+// the sums at z = e^{2 pi i k (r_j - rc)/Nf} and conj(z) over the coefficients
+// c_t e^{2 pi i k t rc/Nf}.  NC adjacent lanes share a bin (1 up to 80 time
+// steps); bins g = 0 .. M-1 in the order of F and Yc (g = k1 + N1 k2), so that
+// a block's loads and stores are contiguous runs.  The
+// rate pairs are split over blockIdx.y.  VALU-bound from about 40 time steps
+// on: 235 operations per bin and pair of rates at 64 steps (28 of them FP64),
+// where the Reinsch recurrence it replaced took 395 and serialized its input
+// loads.  Three wavefronts per SIMD up to 64 steps.  Measured, before -> after:
+// 2^20 x 60 x 481 985 -> 705 us, 2^22 x 64 x 257 2229 -> 1556, 2^20 x 80 x 257
+// 1043 -> 480 (two lanes a bin -> one), 2^16 x 279 x 257 342 -> 171; below 40
+// steps the writes of Yc bound it (2^20 x 32 x 257 329 -> 258 us, 4.7 TB/s).
+template <int NB, int NC>
+__global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold_col(CztColArgs a) {
   constexpr int BPB = 256 / NC;  // bins per block
   const int q = threadIdx.x % NC;
-  const int64_t g = static_cast<int64_t>(blockIdx.x) * BPB + threadIdx.x / NC;
-  if (g > a.M) return;  // whole groups of NC lanes leave together
-  ColBin bin;
-  if (g == a.M) {
-    bin.k = a.M;
-    bin.dst = a.yM;
-    bin.stride = 1;
-    bin.fo = a.ftrans ? a.M * a.Nt : a.M;
-    bin.fs = a.ftrans ? 1 : a.ldF;
-  } else {
-    const int ntk1 = (1 << a.logN1) >> 4;
-    const int64_t tile = g >> 8, w = g & 255;
-    const int k2 = static_cast<int>(((tile / ntk1) << 4) + (w >> 4));
-    const int k1 = static_cast<int>(((tile % ntk1) << 4) + (w & 15));
-    bin.k = k2 + (static_cast<int64_t>(k1) << a.logN2);
-    bin.dst = a.Yc + (static_cast<int64_t>(k2) << a.logN1) + k1;
-    bin.stride = a.M;
-    bin.fo = a.ftrans ? (static_cast<int64_t>(k2) << a.logN1) + k1 : bin.k;
-    bin.fs = a.ftrans ? a.M : a.ldF;
-  }
-  const double kd = static_cast<double>(bin.k);
-  const float w = fast_window(a.wkind, a.wcustom, bin.k, a.Nf) * a.scale;
-  const int t0 = NT * q;
-  float cr[NT], ci[NT];
+  const int64_t g = static_cast<int64_t>(blockIdx.x) * BPB + threadIdx.x / NC;  // < M
+  const int64_t k = (g >> a.logN1) + ((g & ((int64_t(1) << a.logN1) - 1)) << a.logN2);
+  FoldBin b;
+  b.dst = a.Yc;
+  b.stride = a.M;
+  b.F = a.F;
+  b.fs = a.M;
+  b.o = static_cast<unsigned>(g);
+  b.kd = static_cast<double>(k);
+  b.w = fast_window(a.wkind, a.wcustom, k, a.Nf) * a.scale;
+  const int npair = (a.r.Nr + 1) / 2;
+  fold_rates<NB, NC>(b, a.r, q, 0, group_first(npair, blockIdx.y, gridDim.y),
+                     group_first(npair, blockIdx.y + 1, gridDim.y), false);
+  // the Nyquist bin, a wavefront per rate over all blocks (a block of its own
+  // would cost a whole round where the others fill the chip exactly)
+  const int lane = threadIdx.x & 63, nw = 4 * gridDim.x * gridDim.y;
+  for (int j = 4 * (blockIdx.y * gridDim.x + blockIdx.x) + (threadIdx.x >> 6); j < a.r.Nr; j += nw) {
+    const double rev = 0.5 * a.r0 + 0.5 * a.dr * static_cast<double>(j);  // e^{i pi t r_j}
+    c32 s = {0.0f, 0.0f};
+    for (int t = lane; t < a.r.Nt; t += 64) s = cfma(s, a.F[a.M * a.r.Nt + t], cis_nh(static_cast<double>(t), rev));
 #pragma unroll
-  for (int u = 0; u < NT; ++u) {
-    const int t = t0 + u;
-    if (t < a.Nt) {
-      c32 f = a.F[bin.fo + static_cast<int64_t>(t) * bin.fs];
-      if (a.hc != 0.0) f = cmul(f, cis_nh(kd * static_cast<double>(t), a.hc));  // uniform
-      cr[u] = f.x * w;
-      ci[u] = f.y * w;
-    } else {
-      cr[u] = 0.0f;
-      ci[u] = 0.0f;
+    for (int x = 32; x > 0; x >>= 1) {
+      s.x += __shfl_xor(s.x, x, 64);
+      s.y += __shfl_xor(s.y, x, 64);
     }
-  }
-  const c64 g1 = cis64f(kd * a.hd2);                              // z step between rates
-  const c64 gq = cis64f(kd * a.hd2 * static_cast<double>(t0));   // gamma^{t0}
-  c64 z = cis64f(kd * a.hz);                                      // e^{2 pi i k (r_0 - rc)/Nf}
-  c64 zq = cis64f(kd * a.hz * static_cast<double>(t0));           // z^{t0} of rate 0
-  auto reduce = [](c32 v) {
-#pragma unroll
-    for (int m = 1; m < NC; m <<= 1) {
-      v.x += __shfl_xor(v.x, m, 64);
-      v.y += __shfl_xor(v.y, m, 64);
-    }
-    return v;
-  };
-  auto store = [&](int j, c32 y) {
-    if (q == 0) bin.dst[static_cast<int64_t>(j) * bin.stride] = y;
-  };
-  const int npair = (a.Nr + 1) / 2;  // j < npair; partner Nr-1-j
-  int j = 0;
-  for (; j + 1 < npair; j += 2) {
-    const c64 z1 = cmul(z, g1);
-    const c64 zq1 = cmul(zq, gq);
-    c32 y0, y0c, y1, y1c;
-    reinsch_quad<NT>([&](int t) { return cr[t]; }, [&](int t) { return ci[t]; }, z, [&](int t) { return cr[t]; },
-                     [&](int t) { return ci[t]; }, z1, y0, y0c, y1, y1c);
-    const c32 s0 = {static_cast<float>(zq.x), static_cast<float>(zq.y)};
-    const c32 s1 = {static_cast<float>(zq1.x), static_cast<float>(zq1.y)};
-    const int jp = a.Nr - 1 - j;  // > j + 1
-    store(j, reduce(cmul(y0, s0)));
-    store(jp, reduce(cmulc(y0c, s0)));
-    store(j + 1, reduce(cmul(y1, s1)));
-    const c32 r1c = reduce(cmulc(y1c, s1));
-    if (jp - 1 != j + 1) store(jp - 1, r1c);
-    z = cmul(z1, g1);
-    zq = cmul(zq1, gq);
-  }
-  if (j < npair) {
-    const int jp = a.Nr - 1 - j;
-    c32 yz, yc;
-    reinsch_split<NT>(cr, ci, z, yz, yc);
-    const c32 s0 = {static_cast<float>(zq.x), static_cast<float>(zq.y)};
-    store(j, reduce(cmul(yz, s0)));
-    const c32 rc = reduce(cmulc(yc, s0));
-    if (jp != j) store(jp, rc);
+    const float w = fast_window(a.wkind, a.wcustom, a.M, a.Nf) * a.scale;
+    if (lane == 0) a.yM[j] = {s.x * w, s.y * w};
   }
 }
 
@@ -825,64 +680,40 @@ int fast_out_unpack_F(FastPlan* p, const c32* Ft, int64_t Nt, c32* F, hipStream_
   return ZDT_OK;
 }
 
-int fast_out_run(FastPlan* p, const c32* F, int64_t ldF, bool ftrans, int Nt, float r0, float dr, int wkind,
-                 const float* window, float* dest, double scale, hipStream_t st, double* colmean, double* colvar) {
+int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkind, const float* window, float* dest,
+                 double scale, hipStream_t st, double* colmean, double* colvar) {
   if (Nt < 1 || Nt > FOUT_MAX_NT) return fail(ZDT_ENOTSUP, "fused output: Nt=%d", Nt);
   CztColArgs c;
   c.F = F;
-  c.ldF = ldF;
-  c.ftrans = ftrans ? 1 : 0;
   c.Yc = p->Yc;
   c.yM = p->yM;
   c.M = p->M;
   c.Nf = p->Nf;
   c.logN1 = p->logN1;
   c.logN2 = p->logN2;
-  c.Nt = Nt;
-  c.Nr = static_cast<int>(p->Nr);
-  c.hd2 = static_cast<double>(dr) / static_cast<double>(p->Nf);
+  c.r0 = static_cast<double>(r0);
+  c.dr = static_cast<double>(dr);
   c.wkind = wkind;
   c.wcustom = window;
   c.scale = 1.0f;
   // rates in mirrored pairs around the centre rate (a single rate is its own partner)
   const double rc = static_cast<double>(r0) + 0.5 * static_cast<double>(p->Nr - 1) * static_cast<double>(dr);
-  c.hc = rc / static_cast<double>(p->Nf);
-  c.hz = (static_cast<double>(r0) - rc) / static_cast<double>(p->Nf);
-  if (Nt <= 64) {
-    const unsigned grid = static_cast<unsigned>(p->M / 256 + 1);
-    ProfScope ps(st, "czt_reinsch_col", 8.0 * (p->M + 1) * (Nt + p->Nr));  // F read, Yc written, once each
-    if (Nt <= 16) {
-      czt_reinsch_col<16><<<grid, 256, 0, st>>>(c);
-    } else if (Nt <= 32) {
-      czt_reinsch_col<32><<<grid, 256, 0, st>>>(c);
-    } else {
-      czt_reinsch_col<64><<<grid, 256, 0, st>>>(c);
-    }
-    ZDT_CHECK_LAUNCH("czt_reinsch_col");
-  } else {
-    // NC lanes per bin: the 64-step chunks, a power of two (FOUT_MAX_NT = 1024: at most 16)
-    int nc = 2;
-    while (nc * 64 < Nt) nc *= 2;
-    const int64_t bins = p->M + 1;
-    const unsigned grid = static_cast<unsigned>((bins + 256 / nc - 1) / (256 / nc));
-    ProfScope ps(st, "czt_reinsch_col_split", 8.0 * (p->M + 1) * (Nt + p->Nr));
-    switch (nc) {
-      case 2:
-        czt_reinsch_col_split<2><<<grid, 256, 0, st>>>(c);
-        break;
-      case 4:
-        czt_reinsch_col_split<4><<<grid, 256, 0, st>>>(c);
-        break;
-      case 8:
-        czt_reinsch_col_split<8><<<grid, 256, 0, st>>>(c);
-        break;
-      case 16:
-        czt_reinsch_col_split<16><<<grid, 256, 0, st>>>(c);
-        break;
-      default:
-        return fail(ZDT_ENOTSUP, "fused output: Nt=%d above %lld", Nt, (long long)FOUT_MAX_NT);
-    }
-    ZDT_CHECK_LAUNCH("czt_reinsch_col_split");
+  const double nf = static_cast<double>(p->Nf);
+  c.r = {Nt, static_cast<int>(p->Nr), static_cast<double>(dr) / nf, rc / nf, (static_cast<double>(r0) - rc) / nf};
+  {
+    int nb = 0, nc = 0;
+    fold_split(Nt, &nb, &nc);
+    const int per = 256 / nc;  // bins per block
+    const int nblk = static_cast<int>(p->M / per);
+    // rate pairs over blockIdx.y up to the wavefronts a CU holds (8 with five
+    // blocks of coefficients, 12 with fewer); a part repeats the coefficients,
+    // worth about ten pairs
+    const dim3 grid(static_cast<unsigned>(nblk), group_parts(static_cast<int>((p->Nr + 1) / 2), nblk, 256,
+                                                             nb == 5 ? 8 : 12, 24, p->resident_blocks / 2));
+    ProfScope ps(st, "czt_fold_col", 8.0 * (p->M + 1) * (Nt + p->Nr));  // F read, Yc written, once each
+    if (!fold_dispatch(nb, nc, [&](auto B, auto C) { czt_fold_col<B(), C()><<<grid, 256, 0, st>>>(c); }))
+      return fail(ZDT_ENOTSUP, "fused output: Nt=%d", Nt);
+    ZDT_CHECK_LAUNCH("czt_fold_col");
   }
   K2cArgs a;
   a.Yc = p->Yc;
