@@ -962,42 +962,50 @@ void fast_set_smax(FastPlan* p, float* smax) {
 
 int fast_plan_n2(const FastPlan* p) { return p != nullptr ? p->N2 : 0; }
 
+int fast_output_part(FastPlan* p, float* dest, int64_t j0, int64_t n, hipStream_t st, bool stats) {
+  const int64_t tiles = p->N1 / 16;  // per rate
+  K3Args a;
+  a.B = p->B;
+  a.yhalf = p->yhalf + j0;
+  a.dest = dest + j0 * p->Nf;
+  a.ld = p->Nf;
+  a.tw2 = p->tw2;
+  a.logN1 = p->logN1;
+  a.Nr = static_cast<int>(n);
+  a.ntiles = static_cast<int>(n * tiles);
+  a.part = stats ? p->part + j0 * tiles * k3_waves(p) * 3 : nullptr;
+  a.paired = p->paired ? 1 : 0;
+  a.smax = p->smax != nullptr ? p->smax + j0 * tiles * p->N2 : nullptr;
+  ProfScope ps(st, "k3_output", 8.0 * p->M * n + 4.0 * p->Nf * n);
+  if (p->precision != ZDT_PRECISION_FP32) {
+    ZDT_TRY(launch_k3_mfma(p, a, st));
+  } else if (p->N2 == 1024) {
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(a.ntiles, p->resident_blocks / 2));
+    if (a.smax) k3_output<32, true><<<grid, CF<32>::THREADS, 0, st>>>(a);
+    else k3_output<32, false><<<grid, CF<32>::THREADS, 0, st>>>(a);
+  } else {
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(a.ntiles, p->resident_blocks));
+    if (a.smax) k3_output<16, true><<<grid, CF<16>::THREADS, 0, st>>>(a);
+    else k3_output<16, false><<<grid, CF<16>::THREADS, 0, st>>>(a);
+  }
+  ZDT_CHECK_LAUNCH("k3_output");
+  return ZDT_OK;
+}
+
+int fast_stats_merge(FastPlan* p, hipStream_t st, double* colmean, double* colvar) {
+  if (p->part == nullptr) return fail(ZDT_ESTATE, "fused statistics: no partials buffer");
+  const int np = (p->N1 / 16) * k3_waves(p);
+  k3_stats_merge<<<static_cast<unsigned>(p->Nr), 256, 0, st>>>(p->part, np, p->Nf, colmean, colvar);
+  ZDT_CHECK_LAUNCH("k3_stats_merge");
+  return ZDT_OK;
+}
+
 int fast_output(FastPlan* p, float* dest, double scale, hipStream_t st, double* colmean, double* colvar) {
   (void)scale;  // folded into k2
   if (!p->have_B) return fail(ZDT_ESTATE, "output!: no post-processed spectra");
   if (colmean != nullptr && p->part == nullptr) return fail(ZDT_ESTATE, "fused statistics: no partials buffer");
-  K3Args a;
-  a.B = p->B;
-  a.yhalf = p->yhalf;
-  a.dest = dest;
-  a.ld = p->Nf;
-  a.tw2 = p->tw2;
-  a.logN1 = p->logN1;
-  a.Nr = static_cast<int>(p->Nr);
-  a.ntiles = static_cast<int>(p->Nr * (p->N1 / 16));
-  a.part = colmean != nullptr ? p->part : nullptr;
-  a.paired = p->paired ? 1 : 0;
-  a.smax = p->smax;
-  {
-    ProfScope ps(st, "k3_output", 8.0 * p->M * p->Nr + 4.0 * p->Nf * p->Nr);
-    if (p->precision != ZDT_PRECISION_FP32) {
-      ZDT_TRY(launch_k3_mfma(p, a, st));
-    } else if (p->N2 == 1024) {
-      const unsigned grid = static_cast<unsigned>(std::min<int64_t>(a.ntiles, p->resident_blocks / 2));
-      if (a.smax) k3_output<32, true><<<grid, CF<32>::THREADS, 0, st>>>(a);
-      else k3_output<32, false><<<grid, CF<32>::THREADS, 0, st>>>(a);
-    } else {
-      const unsigned grid = static_cast<unsigned>(std::min<int64_t>(a.ntiles, p->resident_blocks));
-      if (a.smax) k3_output<16, true><<<grid, CF<16>::THREADS, 0, st>>>(a);
-      else k3_output<16, false><<<grid, CF<16>::THREADS, 0, st>>>(a);
-    }
-    ZDT_CHECK_LAUNCH("k3_output");
-  }
-  if (colmean != nullptr) {
-    const int np = (p->N1 / 16) * k3_waves(p);
-    k3_stats_merge<<<static_cast<unsigned>(p->Nr), 256, 0, st>>>(p->part, np, p->Nf, colmean, colvar);
-    ZDT_CHECK_LAUNCH("k3_stats_merge");
-  }
+  ZDT_TRY(fast_output_part(p, dest, 0, p->Nr, st, colmean != nullptr));
+  if (colmean != nullptr) ZDT_TRY(fast_stats_merge(p, st, colmean, colvar));
   return ZDT_OK;
 }
 

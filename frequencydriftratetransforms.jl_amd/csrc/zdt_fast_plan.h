@@ -54,6 +54,11 @@ int upload_table(c32** dst, const std::vector<c32>& h);
 std::vector<c32> twiddles(int N);
 // allocates p->part (fast_stats_doubles) unless rc already holds an error
 void alloc_part(FastPlan* p, int& rc);
+// k3 over the n rates whose spectra fill the start of p->B, into columns j0 ..
+// of dest (statistics partials and run maxima at the same columns)
+int fast_output_part(FastPlan* p, float* dest, int64_t j0, int64_t n, hipStream_t st, bool stats);
+// per-column mean and variance from the partials of all rates
+int fast_stats_merge(FastPlan* p, hipStream_t st, double* colmean, double* colvar);
 // k1_input over Nt time steps of spec into G
 int launch_k1(const FastPlan* p, const float* spec, c32* G, int64_t Nt, hipStream_t st);
 

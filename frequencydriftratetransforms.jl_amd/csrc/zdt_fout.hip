@@ -99,6 +99,12 @@ struct K2cArgs {
   float oscale;   // output scale / M
 };
 
+__device__ __forceinline__ c32 load_nt(const c32* p) {
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  const f2v v = __builtin_nontemporal_load(reinterpret_cast<const f2v*>(p));
+  return {v.x, v.y};
+}
+
 // the rate loop of k2_czt with the spectra read from Yc instead of evaluated
 template <int N1, int N2, int ROWS>
 __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c2r(K2cArgs a) {
@@ -146,8 +152,8 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
     for (int jj = 0; jj < JG; ++jj) {
       if (jj < njn) {
         const int64_t off = static_cast<int64_t>(j0n + jj) * a.M;
-        ya[jj] = srcA[off];
-        yb[jj] = nyq ? a.yM[j0n + jj] : srcB[off];
+        ya[jj] = load_nt(srcA + off);
+        yb[jj] = nyq ? a.yM[j0n + jj] : load_nt(srcB + off);
       }
     }
   };
@@ -309,21 +315,25 @@ __device__ __forceinline__ void wave_ifft_2048(c32* x, const c32* tw, int lane, 
   }
 }
 
-// k2_c2r for N1 = 1024, 2048 (Nf = 2^21, 2^22): 512 threads, PP = N1/512
-// pairs each, groups of 4 rates (8 rows, one per wavefront) in one LDS
-// buffer; each wavefront runs the inverse DFT_N1 of its row in place
-// (wave_fft_row) and stores it, so a group costs two barriers.  The next
-// group's spectra are loaded into registers before the DFTs, so their
-// latency overlaps them (their addresses are formed inside the rate loop:
-// hoisted out of it, they spilled).
-template <int N1, int N2>
-__global__ __launch_bounds__(512) void k2_c2r_wave(K2cArgs a) {
-  constexpr int T = 512;
+// k2_c2r for N1 = 1024, 2048 (Nf = 2^21, 2^22): ROWS wavefronts, PP = N1/(64
+// ROWS) pairs per thread, groups of ROWS/2 rates (one row per wavefront) in
+// one LDS buffer; each wavefront runs the inverse DFT_N1 of its row in place
+// (wave_fft_row) and stores it, so a group costs two barriers.  Blocks walk the
+// units (rate group, column pair), all pairs of a group before the next group:
+// at N1 = 1024 as many blocks as the CUs hold, so that the few groups of a
+// last-level-cache chunk (see fast_out_run) keep every CU busy; at N1 = 2048
+// (no chunks) a block per pair.  The next unit's spectra are loaded into registers before the DFTs,
+// so their latency overlaps them.  At 2^22 x 257 it moves its 8.6 GB in 1.78 ms
+// (4.8 TB/s, a copy's rate); ROWS = 4 with two blocks a CU took 2.28 ms there,
+// but at N1 = 1024 four blocks of ROWS = 4 beat two of 8 (2^21 x 257 in
+// chunks: 890 against 928 us).
+template <int N1, int N2, int ROWS>
+__global__ __launch_bounds__(64 * ROWS, 2) void k2_c2r_wave(K2cArgs a) {
+  constexpr int T = 64 * ROWS;
   constexpr int PP = N1 / T;
   constexpr bool BIG = N1 == 2048;  // wave_ifft_2048 layout (no row padding)
   constexpr int P = BIG ? N1 : N1 + N1 / 8;
   constexpr int HALF = N1 / 2;
-  constexpr int ROWS = 8;
   constexpr int JG = ROWS / 2;
   __shared__ c32 buf[ROWS * P];
   __shared__ c32 twl[BIG ? N1 : 1];
@@ -332,81 +342,62 @@ __global__ __launch_bounds__(512) void k2_c2r_wave(K2cArgs a) {
   }
   auto pos = [](int i) { return BIG ? s2048(i) : lsw(i); };
   const int tid = threadIdx.x;
-  const int p = blockIdx.x;
-  const bool special = (p == 0);
-  const int colA = special ? 0 : p;
-  const int colB = special ? N2 / 2 : N2 - p;
-  int rowA[PP], rowB[PP], k1A[PP], k1B[PP];
-  bool nyq[PP];
-  c32 WA[PP];
-  int offA[PP], offB[PP];  // within a rate's M spectra
-#pragma unroll
-  for (int i = 0; i < PP; ++i) {
-    const HPair h = hpair<N1, N2>(p, tid + i * T);
-    rowA[i] = h.rowA;
-    rowB[i] = h.rowB;
-    k1A[i] = h.k1A;
-    k1B[i] = h.k1B;
-    nyq[i] = h.nyq;
-    const int cA = h.cA, cB = h.cB;
-    const int64_t kA = cA + static_cast<int64_t>(N2) * k1A[i];
-    WA[i] = cis_rev(-static_cast<float>(kA) / static_cast<float>(a.Nf));
-    offA[i] = cA * N1 + k1A[i];
-    offB[i] = cB * N1 + (nyq[i] ? 0 : k1B[i]);
-  }
   const float h = 0.5f * a.oscale;
-  if (special) {
-    for (int j = tid; j < a.Nr; j += T) {
-      const c32 y = a.Yc[static_cast<int64_t>(j) * a.M + HALF];
-      a.yhalf[j] = {y.x * a.oscale, -y.y * a.oscale};
-    }
-  }
+  const float invNf = 1.0f / static_cast<float>(a.Nf);
+  const int units = (a.Nr + JG - 1) / JG * (N2 / 2);
   c32 ya[JG][PP], yb[JG][PP];
-  auto load = [&](int j0n) {
-    const int njn = min(JG, a.Nr - j0n);
+  auto load = [&](int u) {
+    const int p = u % (N2 / 2), j0 = u / (N2 / 2) * JG;
 #pragma unroll
-    for (int jj = 0; jj < JG; ++jj) {
-      if (jj < njn) {
-        const c32* y = a.Yc + static_cast<int64_t>(j0n + jj) * a.M;  // uniform
+    for (int i = 0; i < PP; ++i) {
+      const HPair q = hpair<N1, N2>(p, tid + i * T);
+      const int oa = q.cA * N1 + q.k1A, ob = q.cB * N1 + (q.nyq ? 0 : q.k1B);
 #pragma unroll
-        for (int i = 0; i < PP; ++i) {
-          // opaque offsets: the 64-bit addresses are formed here, not hoisted
-          // out of the rate loop (where they would be spilled)
-          int oa = offA[i], ob = offB[i];
-          asm volatile("" : "+v"(oa), "+v"(ob));
-          ya[jj][i] = y[oa];
-          yb[jj][i] = nyq[i] ? a.yM[j0n + jj] : y[ob];
+      for (int jj = 0; jj < JG; ++jj) {
+        if (j0 + jj < a.Nr) {  // uniform
+          const c32* y = a.Yc + static_cast<int64_t>(j0 + jj) * a.M;  // uniform
+          ya[jj][i] = load_nt(y + oa);
+          yb[jj][i] = q.nyq ? a.yM[j0 + jj] : load_nt(y + ob);
         }
       }
     }
   };
-  load(0);
+  int u = blockIdx.x;
+  if (u < units) load(u);
   const int wv = tid >> 6, lane = tid & 63;
-  for (int j0 = 0; j0 < a.Nr; j0 += JG) {
+  for (; u < units; u += gridDim.x) {
+    const int p = u % (N2 / 2), j0 = u / (N2 / 2) * JG;
     const int nj = min(JG, a.Nr - j0);
 #pragma unroll
-    for (int jj = 0; jj < JG; ++jj) {
-      if (jj < nj) {
+    for (int i = 0; i < PP; ++i) {
+      const HPair q = hpair<N1, N2>(p, tid + i * T);
+      const c32 WA = cis_rev(-static_cast<float>(q.cA + N2 * q.k1A) * invNf);
 #pragma unroll
-        for (int i = 0; i < PP; ++i) {
+      for (int jj = 0; jj < JG; ++jj) {
+        if (jj < nj) {
           const c32 YA = {ya[jj][i].x * h, ya[jj][i].y * h}, YB = {yb[jj][i].x * h, yb[jj][i].y * h};
-          if (nyq[i]) {
-            buf[(2 * jj + rowA[i]) * P] = {YA.x + YB.x, YA.x - YB.x};
-            buf[(2 * jj + rowA[i]) * P + pos(HALF)] = {0.0f, 0.0f};
+          if (q.nyq) {
+            buf[(2 * jj + q.rowA) * P] = {YA.x + YB.x, YA.x - YB.x};
+            buf[(2 * jj + q.rowA) * P + pos(HALF)] = {0.0f, 0.0f};
           } else {
             const c32 E = {YA.x + YB.x, YA.y - YB.y};
             const c32 D = {YA.x - YB.x, YA.y + YB.y};
-            const c32 O = cmulc(D, WA[i]);
-            buf[(2 * jj + rowA[i]) * P + pos(k1A[i])] = {E.x - O.y, E.y + O.x};
-            buf[(2 * jj + rowB[i]) * P + pos(k1B[i])] = {E.x + O.y, -E.y + O.x};
+            const c32 O = cmulc(D, WA);
+            buf[(2 * jj + q.rowA) * P + pos(q.k1A)] = {E.x - O.y, E.y + O.x};
+            buf[(2 * jj + q.rowB) * P + pos(q.k1B)] = {E.x + O.y, -E.y + O.x};
           }
         }
       }
     }
+    if (p == 0 && tid < nj) {  // the bin M/2: k2 = 0, k1 = N1/2
+      const c32 y = a.Yc[static_cast<int64_t>(j0 + tid) * a.M + HALF];
+      a.yhalf[j0 + tid] = {y.x * a.oscale, -y.y * a.oscale};
+    }
     __syncthreads();
-    if (j0 + JG < a.Nr) load(j0 + JG);
+    if (u + static_cast<int>(gridDim.x) < units) load(u + gridDim.x);
     if (wv < 2 * nj) {  // uniform per wavefront: wavefront wv owns row wv
-      c32* dst = a.B + static_cast<int64_t>(j0 + (wv >> 1)) * (N1 * N2) + ((wv & 1) ? colB : colA) * 16;
+      const int col = p == 0 ? (wv & 1) * (N2 / 2) : ((wv & 1) ? N2 - p : p);
+      c32* dst = a.B + static_cast<int64_t>(j0 + (wv >> 1)) * (N1 * N2) + col * 16;
       auto emit = [&](int jx, auto& v) {
         constexpr int RL = sizeof(v) / sizeof(c32);
 #pragma unroll
@@ -423,7 +414,7 @@ __global__ __launch_bounds__(512) void k2_c2r_wave(K2cArgs a) {
         wave_fft_row<N1, true>(buf + wv * P, a.tw1, ln, emit);
       }
     }
-    __syncthreads();  // the rows are rewritten by the next group
+    __syncthreads();  // the rows are rewritten by the next unit
   }
 }
 
@@ -548,6 +539,9 @@ namespace zdt {
 
 // ---------------------------------------------------------------- fused output (host)
 
+// bytes of spectra per chunk of rates (see fast_out_run)
+constexpr int64_t FOUT_CHUNK = int64_t(224) << 20;
+
 bool fast_out_supported(int64_t Nf, int64_t Nt, int64_t Nr) {
   if (Nf < (1 << 16) || Nf > (1 << 22) || (Nf & (Nf - 1)) != 0) return false;
   return Nt >= 1 && Nt <= FOUT_MAX_NT && Nr >= 1 && Nr <= 65535;
@@ -613,7 +607,10 @@ static int launch_k2c(const K2cArgs& a, int64_t ncu, hipStream_t st) {
     const dim3 grid(N2 / 2, group_parts((a.Nr + JG - 1) / JG, N2 / 2, N1, 24, 2, ncu));
     k2_c2r<N1, N2, k2_rows(N1)><<<grid, N1, 0, st>>>(a);
   } else {
-    k2_c2r_wave<N1, N2><<<N2 / 2, 512, 0, st>>>(a);
+    constexpr int ROWS = N1 == 2048 ? 8 : 4;
+    const int64_t units = static_cast<int64_t>((a.Nr + ROWS / 2 - 1) / (ROWS / 2)) * (N2 / 2);
+    const unsigned grid = static_cast<unsigned>(std::min<int64_t>(units, N1 == 2048 ? N2 / 2 : 4 * ncu));
+    k2_c2r_wave<N1, N2, ROWS><<<grid, 64 * ROWS, 0, st>>>(a);
   }
   ZDT_CHECK_LAUNCH("k2_c2r");
   return ZDT_OK;
@@ -680,6 +677,36 @@ int fast_out_unpack_F(FastPlan* p, const c32* Ft, int64_t Nt, c32* F, hipStream_
   return ZDT_OK;
 }
 
+static int run_k2c(const FastPlan* p, const K2cArgs& a, hipStream_t st) {
+  ProfScope ps(st, "k2_c2r", 16.0 * p->M * a.Nr);
+  switch (p->N1 * 2048 + p->N2) {
+    case 64 * 2048 + 512:
+      ZDT_TRY((launch_k2c<64, 512>(a, p->resident_blocks / 2, st)));
+      break;
+    case 64 * 2048 + 1024:
+      ZDT_TRY((launch_k2c<64, 1024>(a, p->resident_blocks / 2, st)));
+      break;
+    case 128 * 2048 + 1024:
+      ZDT_TRY((launch_k2c<128, 1024>(a, p->resident_blocks / 2, st)));
+      break;
+    case 256 * 2048 + 1024:
+      ZDT_TRY((launch_k2c<256, 1024>(a, p->resident_blocks / 2, st)));
+      break;
+    case 512 * 2048 + 1024:
+      ZDT_TRY((launch_k2c<512, 1024>(a, p->resident_blocks / 2, st)));
+      break;
+    case 1024 * 2048 + 1024:
+      ZDT_TRY((launch_k2c<1024, 1024>(a, p->resident_blocks / 2, st)));
+      break;
+    case 2048 * 2048 + 1024:
+      ZDT_TRY((launch_k2c<2048, 1024>(a, p->resident_blocks / 2, st)));
+      break;
+    default:
+      return fail(ZDT_ENOTSUP, "fused output: N1=%d N2=%d", p->N1, p->N2);
+  }
+  return ZDT_OK;
+}
+
 int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkind, const float* window, float* dest,
                  double scale, hipStream_t st, double* colmean, double* colvar) {
   if (Nt < 1 || Nt > FOUT_MAX_NT) return fail(ZDT_ENOTSUP, "fused output: Nt=%d", Nt);
@@ -716,45 +743,37 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
     ZDT_CHECK_LAUNCH("czt_fold_col");
   }
   K2cArgs a;
-  a.Yc = p->Yc;
-  a.yM = p->yM;
   a.B = p->B;
-  a.yhalf = p->yhalf;
   a.tw1 = p->tw1;
-  a.Nr = static_cast<int>(p->Nr);
   a.M = p->M;
   a.Nf = p->Nf;
   a.oscale = static_cast<float>(scale / static_cast<double>(p->M));
-  {
-    ProfScope ps(st, "k2_c2r", 16.0 * p->M * p->Nr);
-    switch (p->N1 * 2048 + p->N2) {
-      case 64 * 2048 + 512:
-        ZDT_TRY((launch_k2c<64, 512>(a, p->resident_blocks / 2, st)));
-        break;
-      case 64 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<64, 1024>(a, p->resident_blocks / 2, st)));
-        break;
-      case 128 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<128, 1024>(a, p->resident_blocks / 2, st)));
-        break;
-      case 256 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<256, 1024>(a, p->resident_blocks / 2, st)));
-        break;
-      case 512 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<512, 1024>(a, p->resident_blocks / 2, st)));
-        break;
-      case 1024 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<1024, 1024>(a, p->resident_blocks / 2, st)));
-        break;
-      case 2048 * 2048 + 1024:
-        ZDT_TRY((launch_k2c<2048, 1024>(a, p->resident_blocks / 2, st)));
-        break;
-      default:
-        return fail(ZDT_ENOTSUP, "fused output: N1=%d N2=%d", p->N1, p->N2);
-    }
+  // Rates in chunks whose spectra B (written by k2_c2r, read once by k3) stay
+  // in the 256 MB last-level cache: every chunk reuses the start of p->B, Yc is
+  // read and the FDR written past the cache (nontemporal).  A copy from there
+  // runs at 7-8 TB/s against 5.5 from HBM.  224 MB a chunk: smaller ones pay
+  // more launches and tails, larger ones spill (2^20 x 60 x 481, whole call:
+  // 2555 us in one piece, 2457, 2412, 2395, 2358 in chunks of 128, 160, 192, 224
+  // MB).  Not at 2^22, whose k2_c2r_wave has one block a CU and loses what k3
+  // gains (6090 and 6155 us).  Without dest, p->B holds every rate for output!.
+  const int64_t rate_bytes = 8 * p->M;
+  int64_t per = p->Nr;
+  if (dest != nullptr && p->N1 <= 1024 && rate_bytes * p->Nr > FOUT_CHUNK + FOUT_CHUNK / 8) {
+    const int64_t nch = (rate_bytes * p->Nr + FOUT_CHUNK - 1) / FOUT_CHUNK;
+    const int64_t r = p->N1 <= 512 ? 8 : 4;  // whole rate groups and, at 2^20, whole rounds of k3's tiles
+    per = ((p->Nr + nch - 1) / nch + r - 1) / r * r;
   }
-  p->have_B = true;
-  if (dest != nullptr) ZDT_TRY(fast_output(p, dest, scale, st, colmean, colvar));
+  for (int64_t j0 = 0; j0 < p->Nr; j0 += per) {
+    const int64_t n = std::min(per, p->Nr - j0);
+    a.Yc = p->Yc + j0 * p->M;
+    a.yM = p->yM + j0;
+    a.yhalf = p->yhalf + j0;
+    a.Nr = static_cast<int>(n);
+    ZDT_TRY(run_k2c(p, a, st));
+    if (dest != nullptr) ZDT_TRY(fast_output_part(p, dest, j0, n, st, colmean != nullptr));
+  }
+  p->have_B = per >= p->Nr;
+  if (colmean != nullptr && dest != nullptr) ZDT_TRY(fast_stats_merge(p, st, colmean, colvar));
   return ZDT_OK;
 }
 
