@@ -450,9 +450,8 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
 #pragma unroll
     for (int i = 0; i < PP; ++i)  // e^{2 pi i k r_g0/Nf}
       zp[i] = cis64f(static_cast<double>(kA[i]) * (a.hz0 + static_cast<double>(g0) * a.hd2));
-    c32* cur = buf;
-    c32* nxt = buf2;
-    for (int p0 = g0; p0 >= glo; p0 -= NPG) {
+    // the c2r rows of pair group p0 (in dst), and z of the group after it
+    auto rows_of = [&](int p0, c32* dst) {
       const int np = min(NPG, npairs - p0);
 #pragma unroll
       for (int i = 0; i < PP; ++i) zq[i] = zp[i];
@@ -476,23 +475,33 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
             if (m == 1 && !twin) break;
             const int slot = 2 * pp + m;
             if (nyq[i]) {
-              cur[(2 * slot + rowA[i]) * P] = {YA[m].x + YB[m].x, YA[m].x - YB[m].x};
-              cur[(2 * slot + rowA[i]) * P + ix(HALF)] = {0.0f, 0.0f};
+              dst[(2 * slot + rowA[i]) * P] = {YA[m].x + YB[m].x, YA[m].x - YB[m].x};
+              dst[(2 * slot + rowA[i]) * P + ix(HALF)] = {0.0f, 0.0f};
             } else {
               const c32 E = {YA[m].x + YB[m].x, YA[m].y - YB[m].y};
               const c32 D = {YA[m].x - YB[m].x, YA[m].y + YB[m].y};
               const c32 O = cmulc(D, WA[i]);
-              cur[(2 * slot + rowA[i]) * P + ix(k1A[i])] = {E.x - O.y, E.y + O.x};
-              cur[(2 * slot + rowB[i]) * P + ix(k1B[i])] = {E.x + O.y, -E.y + O.x};
+              dst[(2 * slot + rowA[i]) * P + ix(k1A[i])] = {E.x - O.y, E.y + O.x};
+              dst[(2 * slot + rowB[i]) * P + ix(k1B[i])] = {E.x + O.y, -E.y + O.x};
             }
           }
         }
       }
-      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < PP; ++i) {  // back one group: conj(gamma)^NPG, formed here to spare registers
+        c64 g = {gam[i].x, -gam[i].y};
+#pragma unroll
+        for (int s = 1; s < NPG; ++s) g = cmul(g, c64{gam[i].x, -gam[i].y});
+        zp[i] = cmul(zp[i], g);
+      }
+    };
+    // inverse DFT_N1 of the wavefront's rows of group p0 (in src) and their store
+    auto fft_of = [&](int p0, c32* src) {
+      const int np = min(NPG, npairs - p0);
       // slots 2pp, 2pp+1 hold rates p0+pp, Pm-p0-pp (the middle rate once, last)
       const int nslots = 2 * np - ((Pm & 1) == 0 && p0 + np == npairs ? 1 : 0);
       const int nrw = min(RPW, max(0, 2 * nslots - wv * RPW));  // uniform per wavefront
-      wave_fft<N1, true, 1, true, LAY>(cur + wv * RPW * P, P, nrw, twl, lane, [&](int f, int jx, auto& v) {
+      wave_fft<N1, true, 1, true, LAY>(src + wv * RPW * P, P, nrw, twl, lane, [&](int f, int jx, auto& v) {
         constexpr int RL = sizeof(v) / sizeof(c32);
         const int row = wv * RPW + f;
         const int slot = row >> 1;
@@ -504,16 +513,24 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
           dst[(n1 >> 4) * (N2 * 16) + (n1 & 15)] = v[r];
         }
       });
+    };
+    c32* cur = buf;
+    c32* nxt = buf2;
+    // Between two barriers a wavefront transforms its rows of one group and
+    // makes its part of the next group's: the first half of the wavefronts in
+    // this order, the second half in the other, so that on every SIMD one is
+    // at its LDS passes while the other keeps the VALU busy.
+    const bool early = __builtin_amdgcn_readfirstlane(wv) < NW / 2;
+    rows_of(g0, cur);
+    __syncthreads();
+    for (int p0 = g0; p0 >= glo; p0 -= NPG) {
+      if (early) fft_of(p0, cur);
+      if (p0 > glo) rows_of(p0 - NPG, nxt);
+      if (!early) fft_of(p0, cur);
+      __syncthreads();
       c32* t = cur;
       cur = nxt;
       nxt = t;
-#pragma unroll
-      for (int i = 0; i < PP; ++i) {  // back one group: conj(gamma)^NPG, formed here to spare registers
-        c64 g = {gam[i].x, -gam[i].y};
-#pragma unroll
-        for (int s = 1; s < NPG; ++s) g = cmul(g, c64{gam[i].x, -gam[i].y});
-        zp[i] = cmul(zp[i], g);
-      }
     }
   } else {
     // ---- chirp-Z for every rate, c2r pre-pass, inverse DFT_N1, store
