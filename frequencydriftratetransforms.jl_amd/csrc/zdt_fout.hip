@@ -433,7 +433,11 @@ struct K2iArgs {
 // (regular block p: columns p and N2-p; block 0: columns 0 and N2/2); for each
 // group of TG = ROWS/2 time steps the 2 TG rows get the twiddle W_M^{n1 k2}
 // and a forward DFT_N1, then each thread untangles its pairs (k, M-k) into
-// the r2c spectrum and writes both bins back over the rows it read.
+// the r2c spectrum and writes both bins back over the rows it read.  Bound by
+// HBM now (4.4 TB/s for its read and write of G at 2^22 x 64): loading the next
+// group's rows before the DFT and the twiddle table from LDS instead of
+// global memory took 2^22 x 64 from 772 to 491 us, 2^21 x 32 from 210 to 127 and
+// 2^20 x 60 from 165 to 110.
 template <int N1, int N2, int ROWS>
 __global__ __launch_bounds__(N1 < 1024 ? N1 : 1024) void k2_input(K2iArgs a) {
   constexpr int T = N1 < 1024 ? N1 : 1024;
@@ -443,6 +447,8 @@ __global__ __launch_bounds__(N1 < 1024 ? N1 : 1024) void k2_input(K2iArgs a) {
   constexpr int TG = ROWS / 2;
   __shared__ c32 buf[ROWS * P];
   __shared__ c32 buf2[ROWS * P];
+  __shared__ c32 twl[N1 + N1 / 8];  // W_N1^m at lsw(m)
+  for (int i = threadIdx.x; i < N1; i += T) twl[lsw(i)] = a.tw1[i];
   const int tid = threadIdx.x;
   const int p = blockIdx.x;
   const bool special = (p == 0);
@@ -473,19 +479,33 @@ __global__ __launch_bounds__(N1 < 1024 ? N1 : 1024) void k2_input(K2iArgs a) {
   const int ng = (a.Nt + TG - 1) / TG;
   const int tlo = group_first(ng, blockIdx.y, gridDim.y) * TG;
   const int thi = min(a.Nt, group_first(ng, blockIdx.y + 1, gridDim.y) * TG);
-  for (int t0 = tlo; t0 < thi; t0 += TG) {
+  // the next group's rows are loaded before this group's DFT
+  c32 v[ROWS][PP];
+  auto load = [&](int t0) {
     const int nt = min(TG, a.Nt - t0);
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
       if (r < 2 * nt) {
         const c32* src = a.G + (static_cast<int64_t>(t0 + (r >> 1)) * N2 + ((r & 1) ? colB : colA)) * N1;
 #pragma unroll
-        for (int i = 0; i < PP; ++i)
-          buf[r * P + lsw(tid + i * T)] = cmulc(src[tid + i * T], (r & 1) ? twS1[i] : twS0[i]);
+        for (int i = 0; i < PP; ++i) v[r][i] = src[tid + i * T];
       }
     }
+  };
+  load(tlo);
+  for (int t0 = tlo; t0 < thi; t0 += TG) {
+    const int nt = min(TG, a.Nt - t0);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      if (r < 2 * nt) {
+#pragma unroll
+        for (int i = 0; i < PP; ++i)
+          buf[r * P + lsw(tid + i * T)] = cmulc(v[r][i], (r & 1) ? twS1[i] : twS0[i]);
+      }
+    }
+    if (t0 + TG < thi) load(t0 + TG);
     __syncthreads();
-    const c32* fz = lds_fft_pp<N1, T, false>(buf, buf2, P, 2 * nt, a.tw1);
+    const c32* fz = lds_fft_pp<N1, T, false, 1, true>(buf, buf2, P, 2 * nt, twl);
 #pragma unroll
     for (int uu = 0; uu < TG; ++uu) {
       if (uu < nt) {
