@@ -134,6 +134,11 @@ __device__ __forceinline__ void fold_sums(const FoldCoef<NB>& c, const FoldPow& 
   }
 }
 
+__device__ __forceinline__ void store_past(c32* p, c32 v) {
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(f2v{v.x, v.y}, reinterpret_cast<f2v*>(p));
+}
+
 // A bin's chirp-Z over a range of rate pairs.  F, dst and their steps are
 // uniform over the block, so that only the bin's offset takes a vector register.
 struct FoldBin {
@@ -164,10 +169,13 @@ __device__ __forceinline__ float quad_xor(float v) {
 // time steps t0 .. t0 + 16 NB - 1, t0 = tbase + 16 NB q, and the NC partial
 // sums are added with each lane keeping a share (with four lanes and more: one
 // of the two rates by its bit 0, the real or imaginary part by its bit 1), so
-// a pair takes log2(NC) + 1 exchanges.  acc: add to what dst holds.
+// a pair takes log2(NC) + 1 exchanges.  acc: add to what dst holds.  past
+// (one lane per bin): store past the last-level cache (nontemporal), for
+// destinations larger than it whose rows are whole cache lines; on rows that are
+// not, such stores cost half as much again (10^6 channels x 129: 136 -> 192 us).
 template <int NB, int NC>
 __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r, int q, int tbase, int jlo, int jhi,
-                                           bool acc) {
+                                           bool acc, bool past) {
   const int t0 = tbase + FOLD * NB * q;
   FoldCoef<NB> c;
   // the time step's input; past the last step the last one again, dropped below
@@ -188,11 +196,16 @@ __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r,
         return t < r.Nt ? c32{v.x * b.w, v.y * b.w} : c32{0.0f, 0.0f};
       });
   const double hs = r.hz + static_cast<double>(jlo) * r.hd2;  // (r_jlo - rc)/Nf
-  // h = z^{1/2} and its step between rates wait in LDS: their eight registers
-  // would spill beside 128 of coefficients at three wavefronts per SIMD
-  __shared__ c64 state[2][256];
-  state[0][threadIdx.x] = cis64f(0.5 * b.kd * hs);
-  state[1][threadIdx.x] = cis64f(0.5 * b.kd * r.hd2);
+  // h = z^{1/2} and its step between rates.  With four and five blocks they wait
+  // in LDS: their eight registers would spill beside 128 of coefficients at
+  // three wavefronts per SIMD
+  constexpr bool PARK = NB >= 4;
+  __shared__ c64 state[2][PARK ? 256 : 1];
+  c64 h = cis64f(0.5 * b.kd * hs), g = cis64f(0.5 * b.kd * r.hd2);
+  if constexpr (PARK) {
+    state[0][threadIdx.x] = h;
+    state[1][threadIdx.x] = g;
+  }
   // the lane's place in the sum: z^{t0}, by a recurrence of its own
   const bool placed = NC > 1 || tbase > 0;
   const double td = static_cast<double>(t0);
@@ -204,10 +217,15 @@ __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r,
   for (int j = jlo; j < jhi; ++j) {
     const int jp = r.Nr - 1 - j;
     int me = static_cast<int>(threadIdx.x);
-    asm volatile("" : "+v"(me));  // read and written here, not carried in registers
-    const c64 h = state[0][me];
-    state[0][me] = cmul(h, state[1][me]);
+    if constexpr (PARK) {
+      asm volatile("" : "+v"(me));  // read and written here, not carried in registers
+      h = state[0][me];
+    }
     const FoldPow w = fold_powers<NB>(h);
+    if constexpr (PARK)
+      state[0][me] = cmul(h, state[1][me]);
+    else
+      h = cmul(h, g);
     c32 U, V, z75 = w.z75;
     if (placed) {
       z75 = cmul(z75, to_c32(zq));
@@ -220,12 +238,15 @@ __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r,
     if constexpr (NC == 1) {
       if (acc) {
         y = cadd(y, dj[b.o]);
-        yc = cadd(yc, dp[b.o]);
+        if (jp != j) yc = cadd(yc, dp[b.o]);
       }
-      // the middle rate is stored twice: a branch here would keep the next
-      // pair's powers from being scheduled among the sums
-      dj[b.o] = y;
-      dp[b.o] = jp != j ? yc : y;
+      if (past) {  // uniform
+        store_past(dj + b.o, y);
+        if (jp != j) store_past(dp + b.o, yc);
+      } else {
+        dj[b.o] = y;
+        if (jp != j) dp[b.o] = yc;
+      }
     } else {
       // bit 0 keeps y (0) or yc (1)
       const bool b0 = q & 1;
@@ -250,12 +271,25 @@ __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r,
   }
 }
 
+// First of the n rate (or time) groups that part y of np takes (0 <= y <= np,
+// n < 2^16): the column-pair kernels split their groups over blockIdx.y where
+// the column pairs alone leave the chip idle (group_parts, zdt_fast_plan.h).
+__device__ __forceinline__ int group_first(int n, unsigned y, unsigned np) {
+  return static_cast<int>(static_cast<unsigned>(n) * y / np);
+}
+
 // Lanes per bin and blocks per lane for Nt time steps: up to five blocks (160
 // coefficient registers, two wavefronts per SIMD) stay in one lane, because
 // the powers (about 70 operations a pair) are made by every lane of a bin.
 // At most FOLD_MAX_NC lanes: FOLD_MAX_NT steps in one go.
 constexpr int FOLD_MAX_NB = 5, FOLD_MAX_NC = 16;
 constexpr int FOLD_MAX_NT = FOLD * FOLD_MAX_NB * FOLD_MAX_NC;
+
+// Whether the chirp-Z of `bytes` of spectra with nb blocks per bin stores past
+// the last-level cache: spectra that fit half of it are read from it next, and
+// from four blocks on the VALU sets the pace (2^22 x 64 x 257: 1556 us through
+// the cache, 1610 past it; 2^22 x 16 x 65 270 and 229).
+inline bool fold_past(int64_t bytes, int nb) { return bytes > (int64_t(128) << 20) && nb < 4; }
 
 inline void fold_split(int64_t Nt, int* nb, int* nc) {
   const int n = static_cast<int>((Nt + FOLD - 1) / FOLD);

@@ -240,6 +240,10 @@ double out_scale(const zdt_ws* ws) {
   return (ws->flags & ZDT_FLAG_UNNORMALIZED) ? static_cast<double>(ws->Nf) * static_cast<double>(ws->Nl) : 1.0;
 }
 
+// column stride of the generic path's spectra Ys: whole 128-byte lines, which
+// the chirp-Z can then write past the cache
+int64_t ys_stride(int64_t Nk) { return (Nk + 15) / 16 * 16; }
+
 bool use_fast(const zdt_ws* ws) { return ws->fast != nullptr; }
 
 int ensure_stepwise(zdt_ws* ws) {
@@ -308,7 +312,7 @@ int run_impl(zdt_ws* ws, float r0, int wkind, const float* window, float* dest) 
   a.F = ws->F;
   a.ldF = ws->Nk;
   a.Ys = ws->Ys;
-  a.ldY = ws->Nk;
+  a.ldY = ys_stride(ws->Nk);
   a.Nk = ws->Nk;
   a.Nf = ws->Nf;
   a.Nt = static_cast<int>(ws->Nt);
@@ -326,7 +330,7 @@ int run_impl(zdt_ws* ws, float r0, int wkind, const float* window, float* dest) 
   a.scale = 1.0f;
   ZDT_TRY(launch_czt(a, ws->stream));
   ws->ys_src = ws->Ys;
-  ws->ys_ld = ws->Nk;
+  ws->ys_ld = ys_stride(ws->Nk);
   ws->ys_fast = false;
   ws->ys_fout = false;
   if (dest != nullptr) ZDT_TRY(output_impl(ws, dest));
@@ -369,7 +373,7 @@ int64_t zdt_workspace_bytes(int64_t Nf, int64_t Nt, int64_t Nr, const int* facto
   if (!(flags & ZDT_FLAG_GENERIC) && fast_out_supported(Nf, Nt, Nr)) return Nk * Nt * 8 + fast_out_bytes(Nf, Nr);
   const int64_t b = std::max(Nt, Nr);
   const int64_t sc = static_cast<int64_t>(fft_real_scratch_elems(Nf, b) * sizeof(c32));
-  return Nk * Nt * 8 + Nk * Nr * 8 + 3 * sc;
+  return Nk * Nt * 8 + ys_stride(Nk) * Nr * 8 + 3 * sc;
 }
 
 }  // extern "C"
@@ -430,7 +434,7 @@ int create_ws_tuned(const float* spec, int64_t Nf, int64_t Nt, float r0, float d
     } else {
       rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->F), static_cast<size_t>(ws->Nk * Nt) * sizeof(c32));
       if (rc == ZDT_OK)
-        rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->Ys), static_cast<size_t>(ws->Nk * Nr) * sizeof(c32));
+        rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->Ys), static_cast<size_t>(ys_stride(ws->Nk) * Nr) * sizeof(c32));
       if (rc == ZDT_OK) rc = ensure_scratch(ws, real_scratch_bytes(ws));
     }
     if (rc == ZDT_OK) {

@@ -433,13 +433,6 @@ constexpr int k2_waves_per_eu(int n1) { return n1 >= 512 ? 4 : 2; }
 // wavefront-level passes (8 rows for 512 = 8*8*8 over 8 wavefronts, ...)
 constexpr int k2_rows(int n1) { return n1 == 256 ? 16 : 8; }
 
-// First of the n rate (or time) groups that part y of np takes (0 <= y <= np,
-// n < 2^16): the column-pair kernels split their groups over blockIdx.y where
-// the column pairs alone leave the chip idle (group_parts, zdt_fast_plan.h).
-__device__ __forceinline__ int group_first(int n, unsigned y, unsigned np) {
-  return static_cast<int>(static_cast<unsigned>(n) * y / np);
-}
-
 // The Hermitian pair q of column-pair block p (see k2_czt): bin
 // kA = cA + N2 k1A in row rowA of the block's two rows and its partner
 // M - kA = cB + N2 k1B in row rowB.  Block p > 0 holds columns p and N2-p;

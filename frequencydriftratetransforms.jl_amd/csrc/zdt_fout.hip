@@ -35,6 +35,7 @@ struct CztColArgs {
   int64_t M, Nf;
   int logN1, logN2;
   FoldRates r;
+  int past;      // store Yc past the last-level cache
   double r0, dr;
   int wkind;
   const float* wcustom;
@@ -51,9 +52,9 @@ struct CztColArgs {
 // on: 235 operations per bin and pair of rates at 64 steps (28 of them FP64),
 // where the Reinsch recurrence it replaced took 395 and serialized its input
 // loads.  Three wavefronts per SIMD up to 64 steps.  Measured, before -> after:
-// 2^20 x 60 x 481 985 -> 705 us, 2^22 x 64 x 257 2229 -> 1556, 2^20 x 80 x 257
+// 2^20 x 60 x 481 985 -> 689 us, 2^22 x 64 x 257 2229 -> 1556, 2^20 x 80 x 257
 // 1043 -> 480 (two lanes a bin -> one), 2^16 x 279 x 257 342 -> 171; below 40
-// steps the writes of Yc bound it (2^20 x 32 x 257 329 -> 258 us, 4.7 TB/s).
+// steps the writes of Yc bound it (2^20 x 32 x 257 329 -> 244 us, 5.0 TB/s).
 template <int NB, int NC>
 __global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold_col(CztColArgs a) {
   constexpr int BPB = 256 / NC;  // bins per block
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold_col(CztColArgs 
   b.w = fast_window(a.wkind, a.wcustom, k, a.Nf) * a.scale;
   const int npair = (a.r.Nr + 1) / 2;
   fold_rates<NB, NC>(b, a.r, q, 0, group_first(npair, blockIdx.y, gridDim.y),
-                     group_first(npair, blockIdx.y + 1, gridDim.y), false);
+                     group_first(npair, blockIdx.y + 1, gridDim.y), false, a.past != 0);
   // the Nyquist bin, a wavefront per rate over all blocks (a block of its own
   // would cost a whole round where the others fill the chip exactly)
   const int lane = threadIdx.x & 63, nw = 4 * gridDim.x * gridDim.y;
@@ -730,6 +731,22 @@ static int run_k2c(const FastPlan* p, const K2cArgs& a, hipStream_t st) {
 int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkind, const float* window, float* dest,
                  double scale, hipStream_t st, double* colmean, double* colvar) {
   if (Nt < 1 || Nt > FOUT_MAX_NT) return fail(ZDT_ENOTSUP, "fused output: Nt=%d", Nt);
+  // Rates in chunks whose spectra B (written by k2_c2r, read once by k3) stay
+  // in the 256 MB last-level cache: every chunk reuses the start of p->B, Yc is
+  // read and the FDR written past the cache (nontemporal).  A copy from there
+  // runs at 7-8 TB/s against 5.5 from HBM.  224 MB a chunk: smaller ones pay
+  // more launches and tails, larger ones spill (2^20 x 60 x 481, whole call:
+  // 2555 us in one piece, 2457, 2412, 2395, 2358 in chunks of 128, 160, 192, 224
+  // MB).  Not at 2^22, whose k2_c2r_wave has one block a CU and loses what k3
+  // gains (6090 and 6155 us).  Without dest, p->B holds every rate for output!.
+  const int64_t rate_bytes = 8 * p->M;
+  int64_t per = p->Nr;
+  if (dest != nullptr && p->N1 <= 1024 && rate_bytes * p->Nr > FOUT_CHUNK + FOUT_CHUNK / 8) {
+    const int64_t nch = (rate_bytes * p->Nr + FOUT_CHUNK - 1) / FOUT_CHUNK;
+    const int64_t r = p->N1 <= 512 ? 8 : 4;  // whole rate groups and, at 2^20, whole rounds of k3's tiles
+    per = ((p->Nr + nch - 1) / nch + r - 1) / r * r;
+  }
+  const bool chunked = per < p->Nr;
   CztColArgs c;
   c.F = F;
   c.Yc = p->Yc;
@@ -750,8 +767,10 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
   {
     int nb = 0, nc = 0;
     fold_split(Nt, &nb, &nc);
-    const int per = 256 / nc;  // bins per block
-    const int nblk = static_cast<int>(p->M / per);
+    // (Yc in rate chunks is read past the cache too: see below)
+    c.past = fold_past(8 * p->M * p->Nr, nb) || chunked ? 1 : 0;
+    const int bpb = 256 / nc;  // bins per block
+    const int nblk = static_cast<int>(p->M / bpb);
     // rate pairs over blockIdx.y up to the wavefronts a CU holds (8 with five
     // blocks of coefficients, 12 with fewer); a part repeats the coefficients,
     // worth about ten pairs
@@ -768,21 +787,6 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
   a.M = p->M;
   a.Nf = p->Nf;
   a.oscale = static_cast<float>(scale / static_cast<double>(p->M));
-  // Rates in chunks whose spectra B (written by k2_c2r, read once by k3) stay
-  // in the 256 MB last-level cache: every chunk reuses the start of p->B, Yc is
-  // read and the FDR written past the cache (nontemporal).  A copy from there
-  // runs at 7-8 TB/s against 5.5 from HBM.  224 MB a chunk: smaller ones pay
-  // more launches and tails, larger ones spill (2^20 x 60 x 481, whole call:
-  // 2555 us in one piece, 2457, 2412, 2395, 2358 in chunks of 128, 160, 192, 224
-  // MB).  Not at 2^22, whose k2_c2r_wave has one block a CU and loses what k3
-  // gains (6090 and 6155 us).  Without dest, p->B holds every rate for output!.
-  const int64_t rate_bytes = 8 * p->M;
-  int64_t per = p->Nr;
-  if (dest != nullptr && p->N1 <= 1024 && rate_bytes * p->Nr > FOUT_CHUNK + FOUT_CHUNK / 8) {
-    const int64_t nch = (rate_bytes * p->Nr + FOUT_CHUNK - 1) / FOUT_CHUNK;
-    const int64_t r = p->N1 <= 512 ? 8 : 4;  // whole rate groups and, at 2^20, whole rounds of k3's tiles
-    per = ((p->Nr + nch - 1) / nch + r - 1) / r * r;
-  }
   for (int64_t j0 = 0; j0 < p->Nr; j0 += per) {
     const int64_t n = std::min(per, p->Nr - j0);
     a.Yc = p->Yc + j0 * p->M;

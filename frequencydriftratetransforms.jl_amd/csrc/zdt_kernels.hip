@@ -8,14 +8,16 @@
 // The reference evaluates the convolution over t as a length-Nl circular
 // convolution through FFTs (:249-253); the identity chirp(k,l) = chirp(k,-l)
 // makes the high lags of V (:182-184) the negative lags, so the result equals
-// the linear convolution above for any Nl >= Nt+Nr-1.  czt_reinsch (Nt <= 64)
-// and czt_reinsch_chunks (Nt > 64) evaluate it directly (about Nt operations
-// per output), which costs less than the two length-Nl FFTs, needs no V, and
-// is exact up to float rounding.  The step functions (preprocess!,
+// the linear convolution above for any Nl >= Nt+Nr-1.  czt_fold evaluates it
+// directly (two to three operations per time step and output), which costs
+// less than the two length-Nl FFTs, needs no V, and is exact up to float
+// rounding.  The step functions (preprocess!,
 // convolve!, postprocess!) keep the reference's FFT data flow on the
 // materialized Nk x Nl matrix Y for API parity.
 #include <hip/hip_runtime.h>
 
+#include "czt_fold.h"
+#include "zdt_fast_plan.h"
 #include "zdt_kernels.h"
 
 namespace zdt {
@@ -52,181 +54,55 @@ __device__ __forceinline__ float window_value(int wkind, const float* wcustom, i
 }
 
 // ---------------------------------------------------------------------------
-// Vandermonde form for Nt <= 64: by Bluestein's identity the sum above is
-//   Ys[k,j] = w(k) sum_t a_t z_j^t,  a_t = F[k,t] e^{2 pi i k t r0/Nf},
-//   z_j = gamma^j, gamma = e^{2 pi i k dr/Nf},
-// a polynomial in z_j.  A thread keeps its bin's coefficients in registers
-// and writes every Ys[k,j] once.  The rates are taken in mirrored pairs: with the
-// centre rate rc = r0 + (Nr-1) dr/2 folded into the coefficients
-// (c_t = F[k,t] e^{2 pi i k t rc/Nf}), rates j and Nr-1-j are the sums at
-// z = e^{i theta} and conj(z), theta = 2 pi k (r0 + j dr - rc)/Nf, and one
-// Reinsch-modified Goertzel recurrence over the real and the imaginary parts
-// gives both (C. Reinsch, 1967; J. Oliver, "An error analysis of the modified
-// Clenshaw method", 1977).  With s = sign(cos theta), lambda = 2 (cos theta - s),
-//   D_t = c_t + lambda U_{t+1} + s D_{t+1},  U_t = D_t + s U_{t+1}  (t = Nt-1 .. 1),
-//   sum c_t cos(t theta) = c_0 + (lambda/2) U_1 + s D_1,  sum c_t sin(t theta) = U_1 sin theta,
-// (evaluated with s folded into the state, so that every update is an
-// in-place add or FMA), six operations per term for the two rates against
-// eight for two complex Horner
-// evaluations.  z comes from an FP64 recurrence started at an exactly
-// evaluated value, and lambda from the FP64 cos theta, so no accuracy is lost
-// near theta = 0 or pi.  The middle rate of an odd Nr is its own partner.
-template <int NT>
-__global__ __launch_bounds__(256) void czt_reinsch(CztArgs a) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k >= a.Nk) return;
-  const double kd = static_cast<double>(k);
-  const float w = window_value(a.wkind, a.wcustom, k, a.Nf) * a.scale;
-  float cr[NT], ci[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    if (t < a.Nt) {
-      c32 f = a.F[k + static_cast<int64_t>(t) * a.ldF];
-      if (a.hc != 0.0) f = cmul(f, cis_nh(kd * static_cast<double>(t), a.hc));  // uniform
-      cr[t] = f.x * w;
-      ci[t] = f.y * w;
-    } else {
-      cr[t] = 0.0f;
-      ci[t] = 0.0f;
-    }
-  }
-  const c64 g = cis64(2.0 * kd * a.hd);  // gamma = e^{2 pi i k dr/Nf}
-  c64 z = cis64(kd * a.hz);              // e^{2 pi i k (r0 - rc)/Nf}
-  c32* dst = a.Ys + k;
-  const int npair = (a.Nr + 1) / 2;  // j < npair; partner Nr-1-j
-  for (int j = 0; j < npair; ++j) {
-    const int jp = a.Nr - 1 - j;
-    // the recurrence with s folded into the state (D~_t = s^t D_t,
-    // U~_t = s^t U_t): every update accumulates in place
-    const float s = z.x >= 0.0 ? 1.0f : -1.0f;
-    const float lamp = static_cast<float>(2.0 * (z.x - static_cast<double>(s))) * s;
-    const float ssn = static_cast<float>(z.y) * s;
-    constexpr bool odd = (NT - 1) & 1;
-    float Dr = odd ? s * cr[NT - 1] : cr[NT - 1], Di = odd ? s * ci[NT - 1] : ci[NT - 1];
-    float Ur = Dr, Ui = Di;
-#pragma unroll
-    for (int t = NT - 2; t >= 1; --t) {
-      if (t & 1) {
-        Dr = fmaf(s, cr[t], Dr);
-        Di = fmaf(s, ci[t], Di);
-      } else {
-        Dr += cr[t];
-        Di += ci[t];
-      }
-      Dr = fmaf(lamp, Ur, Dr);
-      Di = fmaf(lamp, Ui, Di);
-      Ur += Dr;
-      Ui += Di;
-    }
-    const float hl = 0.5f * lamp;
-    const float Cr = fmaf(hl, Ur, cr[0]) + Dr;
-    const float Ci = fmaf(hl, Ui, ci[0]) + Di;
-    const float Sr = ssn * Ur, Si = ssn * Ui;
-    dst[static_cast<int64_t>(j) * a.ldY] = {Cr - Si, Sr + Ci};
-    if (jp != j) dst[static_cast<int64_t>(jp) * a.ldY] = {Cr + Si, Ci - Sr};
-    z = cmul(z, g);
-  }
-}
-
-// Nt > 64: the sum in chunks of 64 time steps, sum_t c_t z^t =
-// sum_q z^{64q} P_q(z) with P_q the polynomial of chunk q, evaluated for both
-// rates of a pair by the recurrence of czt_reinsch; z^{64q} (conj for the
-// partner) comes from an FP64 recurrence over the rates.  Chunk 0 writes Ys,
-// later chunks add to it (one read-modify-write of Ys per further chunk).
-__global__ __launch_bounds__(256) void czt_reinsch_chunks(CztArgs a) {
-  constexpr int NT = 64;
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k >= a.Nk) return;
-  const double kd = static_cast<double>(k);
-  const float w = window_value(a.wkind, a.wcustom, k, a.Nf) * a.scale;
-  const c64 g = cis64(2.0 * kd * a.hd);  // gamma = e^{2 pi i k dr/Nf}
-  c32* dst = a.Ys + k;
-  const int npair = (a.Nr + 1) / 2;  // j < npair; partner Nr-1-j
-  for (int t0 = 0; t0 < a.Nt; t0 += NT) {
-    float cr[NT], ci[NT];
-#pragma unroll
-    for (int u = 0; u < NT; ++u) {
-      const int t = t0 + u;
-      if (t < a.Nt) {
-        c32 f = a.F[k + static_cast<int64_t>(t) * a.ldF];
-        if (a.hc != 0.0) f = cmul(f, cis_nh(kd * static_cast<double>(t), a.hc));  // uniform
-        cr[u] = f.x * w;
-        ci[u] = f.y * w;
-      } else {
-        cr[u] = 0.0f;
-        ci[u] = 0.0f;
-      }
-    }
-    const double td = static_cast<double>(t0);
-    c64 z = cis64(kd * a.hz);               // e^{2 pi i k (r0 - rc)/Nf}
-    c64 zq = cis64(kd * a.hz * td);         // z^{t0} of rate 0
-    const c64 gq = cis64(2.0 * kd * a.hd * td);  // gamma^{t0}
-    for (int j = 0; j < npair; ++j) {
-      const int jp = a.Nr - 1 - j;
-      const float s = z.x >= 0.0 ? 1.0f : -1.0f;
-      const float lamp = static_cast<float>(2.0 * (z.x - static_cast<double>(s))) * s;
-      const float ssn = static_cast<float>(z.y) * s;
-      float Dr = s * cr[NT - 1], Di = s * ci[NT - 1];  // NT - 1 is odd
-      float Ur = Dr, Ui = Di;
-#pragma unroll
-      for (int t = NT - 2; t >= 1; --t) {
-        if (t & 1) {
-          Dr = fmaf(s, cr[t], Dr);
-          Di = fmaf(s, ci[t], Di);
-        } else {
-          Dr += cr[t];
-          Di += ci[t];
-        }
-        Dr = fmaf(lamp, Ur, Dr);
-        Di = fmaf(lamp, Ui, Di);
-        Ur += Dr;
-        Ui += Di;
-      }
-      const float hl = 0.5f * lamp;
-      const float Cr = fmaf(hl, Ur, cr[0]) + Dr;
-      const float Ci = fmaf(hl, Ui, ci[0]) + Di;
-      const float Sr = ssn * Ur, Si = ssn * Ui;
-      const c32 q = {static_cast<float>(zq.x), static_cast<float>(zq.y)};
-      c32 yz = cmul(c32{Cr - Si, Sr + Ci}, q);
-      c32 yc = cmulc(c32{Cr + Si, Ci - Sr}, q);
-      c32* dj = dst + static_cast<int64_t>(j) * a.ldY;
-      c32* dp = dst + static_cast<int64_t>(jp) * a.ldY;
-      if (t0 > 0) {
-        yz = cadd(yz, *dj);
-        if (jp != j) yc = cadd(yc, *dp);
-      }
-      *dj = yz;
-      if (jp != j) *dp = yc;
-      z = cmul(z, g);
-      zq = cmul(zq, gq);
-    }
-  }
+// The chirp-Z of every bin (natural layout): by Bluestein's identity the sum
+// above is Ys[k,j] = w(k) sum_t a_t z_j^t, a_t = F[k,t] e^{2 pi i k t r0/Nf},
+// z_j = e^{2 pi i k j dr/Nf}, taken for mirrored pairs of rates about the
+// centre rate by the fold of czt_fold.h, NC lanes per bin.  The rate pairs are
+// split over blockIdx.y; sums longer than FOLD_MAX_NT take one launch per
+// FOLD_MAX_NT steps, the later ones (tbase > 0) adding to Ys.  Bound by the
+// writes of Ys from about 10^5 bins on (10^6 channels x 16 x 129: 128 -> 111 us,
+// 5.2 TB/s, with Ys in columns of whole cache lines), below by latency: all input loads are in flight together, where the Reinsch
+// kernels this replaced waited for each and reread Ys for every 64 steps past
+// the first (4096 x 16 x 33 11.2 -> 7.5 us, 4096 x 60 x 257 130 -> 23, 2^15 x 177 x
+// 394 611 -> 118, 21609 x 234 x 205 465 -> 66).
+template <int NB, int NC>
+__global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold(CztArgs a, int tbase, int past) {
+  constexpr int BPB = 256 / NC;  // bins per block
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * BPB + threadIdx.x / NC;
+  if (k >= a.Nk) return;  // whole groups of NC lanes leave together
+  FoldBin b;
+  b.F = a.F;
+  b.fs = a.ldF;
+  b.dst = a.Ys;
+  b.stride = a.ldY;
+  b.o = static_cast<unsigned>(k);
+  b.kd = static_cast<double>(k);
+  b.w = window_value(a.wkind, a.wcustom, k, a.Nf) * a.scale;
+  const FoldRates r = {a.Nt, a.Nr, 2.0 * a.hd, a.hc, a.hz};
+  const int npair = (a.Nr + 1) / 2;
+  fold_rates<NB, NC>(b, r, threadIdx.x % NC, tbase, group_first(npair, blockIdx.y, gridDim.y),
+                     group_first(npair, blockIdx.y + 1, gridDim.y), tbase > 0, past != 0);
 }
 
 int launch_czt(const CztArgs& a, hipStream_t st) {
-  const unsigned grid = static_cast<unsigned>((a.Nk + 255) / 256);
-  if (a.Nt > 64) {
-    ProfScope ps(st, "czt_reinsch_chunks",
-                 8.0 * static_cast<double>(a.Nk) * (a.Nt + a.Nr * (2.0 * ((a.Nt + 63) / 64) - 1.0)));
-    czt_reinsch_chunks<<<grid, 256, 0, st>>>(a);
-    ZDT_CHECK_LAUNCH("czt_reinsch_chunks");
-    return ZDT_OK;
+  int dev = 0, ncu = 256;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  ProfScope ps(st, "czt_fold", 8.0 * static_cast<double>(a.Nk) * (a.Nt + a.Nr));
+  for (int tbase = 0; tbase < a.Nt; tbase += FOLD_MAX_NT) {
+    int nb = 0, nc = 0;
+    fold_split(a.Nt - tbase, &nb, &nc);
+    const int per = 256 / nc;
+    const int nblk = static_cast<int>((a.Nk + per - 1) / per);
+    // (whole cache lines: a 128-byte aligned destination and column stride)
+    const int past = fold_past(8 * a.Nk * a.Nr, nb) && a.ldY % 16 == 0 ? 1 : 0;
+    // rate pairs over blockIdx.y up to the wavefronts a CU holds; a part repeats
+    // the coefficients
+    const dim3 grid(static_cast<unsigned>(nblk),
+                    group_parts((a.Nr + 1) / 2, nblk, 256, nb == 5 ? 8 : 12, 4 * (nb + 1), ncu));
+    if (!fold_dispatch(nb, nc, [&](auto B, auto C) { czt_fold<B(), C()><<<grid, 256, 0, st>>>(a, tbase, past); }))
+      return fail(ZDT_ENOTSUP, "chirp-Z: Nt=%d", a.Nt);
+    ZDT_CHECK_LAUNCH("czt_fold");
   }
-  ProfScope ps(st, "czt_reinsch", 8.0 * static_cast<double>(a.Nk) * (a.Nt + a.Nr));
-  if (a.Nt <= 2) {
-    czt_reinsch<2><<<grid, 256, 0, st>>>(a);
-  } else if (a.Nt <= 4) {
-    czt_reinsch<4><<<grid, 256, 0, st>>>(a);
-  } else if (a.Nt <= 8) {
-    czt_reinsch<8><<<grid, 256, 0, st>>>(a);
-  } else if (a.Nt <= 16) {
-    czt_reinsch<16><<<grid, 256, 0, st>>>(a);
-  } else if (a.Nt <= 32) {
-    czt_reinsch<32><<<grid, 256, 0, st>>>(a);
-  } else {
-    czt_reinsch<64><<<grid, 256, 0, st>>>(a);
-  }
-  ZDT_CHECK_LAUNCH("czt_reinsch");
   return ZDT_OK;
 }
 
@@ -318,7 +194,6 @@ int launch_shift_phase(const c32* F, int64_t ldF, c32* Y, int64_t ldY, int64_t N
   ZDT_CHECK_LAUNCH("shift_phase");
   return ZDT_OK;
 }
-
 
 // ---------------------------------------------------------------------------
 // step functions (materialized Y, src/zdtfdr.jl:221-321)
