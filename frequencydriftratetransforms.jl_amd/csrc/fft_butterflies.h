@@ -169,9 +169,68 @@ __device__ __forceinline__ void dft_odd(cplx<T>* v) {
   for (int i = 0; i < R; ++i) v[i] = out[i];
 }
 
+// cos and sin of 2 pi m/R at compile time (Taylor series on [-pi, pi])
+template <int R>
+struct RootTab {
+  double c[R], s[R];
+  constexpr RootTab() : c(), s() {
+    for (int m = 0; m < R; ++m) {
+      const double x = 2.0 * 3.14159265358979323846 * (2 * m > R ? m - R : m) / R;
+      double tc = 1.0, ts = x;
+      c[m] = tc;
+      s[m] = ts;
+      for (int n = 1; n < 20; ++n) {
+        tc *= -x * x / ((2 * n - 1) * (2 * n));
+        ts *= -x * x / ((2 * n) * (2 * n + 1));
+        c[m] += tc;
+        s[m] += ts;
+      }
+    }
+  }
+};
+
+template <typename T, int R>
+__device__ __forceinline__ void dft(cplx<T>* v);
+
+// length-PQ DFT from Q length-P and P length-Q ones (decimation in time)
+template <typename T, int P, int Q>
+__device__ __forceinline__ void dft_pq(cplx<T>* v) {
+  constexpr RootTab<P * Q> W;
+  cplx<T> y[P * Q];
+#pragma unroll
+  for (int n2 = 0; n2 < Q; ++n2) {
+    cplx<T> t[P];
+#pragma unroll
+    for (int n1 = 0; n1 < P; ++n1) t[n1] = v[Q * n1 + n2];
+    dft<T, P>(t);
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1)
+      y[k1 * Q + n2] = k1 * n2 == 0 ? t[k1]
+                                    : cmul(t[k1], cplx<T>{static_cast<T>(W.c[k1 * n2]), static_cast<T>(-W.s[k1 * n2])});
+  }
+#pragma unroll
+  for (int k1 = 0; k1 < P; ++k1) {
+    dft<T, Q>(y + k1 * Q);
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) v[k1 + P * k2] = y[k1 * Q + k2];
+  }
+}
+
 template <typename T, int R>
 __device__ __forceinline__ void dft(cplx<T>* v) {
-  if constexpr (R == 2) {
+  if constexpr (R == 6) {
+    dft_pq<T, 2, 3>(v);
+  } else if constexpr (R == 9) {
+    dft_pq<T, 3, 3>(v);
+  } else if constexpr (R == 10) {
+    dft_pq<T, 2, 5>(v);
+  } else if constexpr (R == 12) {
+    dft_pq<T, 4, 3>(v);
+  } else if constexpr (R == 14) {
+    dft_pq<T, 2, 7>(v);
+  } else if constexpr (R == 15) {
+    dft_pq<T, 3, 5>(v);
+  } else if constexpr (R == 2) {
     dft2(v[0], v[1]);
   } else if constexpr (R == 4) {
     dft4(v);

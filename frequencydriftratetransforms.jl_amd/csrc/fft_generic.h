@@ -12,13 +12,13 @@ struct FftPlan {
   bool dbl = false;
   std::vector<int> radices;  // passes, in order
   void* tw = nullptr;        // device table W_N^m, m < N (c32 or c64)
-  // four-step split N = N1 * N2 of the FP32 contiguous transforms (N1 = 0: none):
-  // N1-point column DFTs and N2-point row DFTs, each in LDS, TC columns / TR rows
-  // per block; twiddles W_N^m = thi[m >> 10] * tlo[m & 1023]
+  // FP32 contiguous transforms in LDS.  rad0: all passes of one kernel (N <=
+  // FS_ONE, else empty).  N1, N2 (N1 = 0: none): the four-step split N = N1 * N2,
+  // N1-point column DFTs (passes rad1) TC columns a block and N2-point row DFTs
+  // (rad2) TR rows a block.  tw0, tw1, tw2: the passes' twiddles, in order
   int N1 = 0, N2 = 0, TC = 0, TR = 0;
-  std::vector<int> rad1, rad2;
-  c32* tlo = nullptr;
-  c32* thi = nullptr;
+  std::vector<int> rad0, rad1, rad2;
+  c32 *tw0 = nullptr, *tw1 = nullptr, *tw2 = nullptr;
 };
 
 // Factor N into the supported radices, largest power-of-two radix first and
@@ -47,8 +47,10 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
             void* s1, void* s2, hipStream_t st, int maxr = 16);
 
 // Complex-to-real inverse: the normalized inverse (1/N) times `scale`; the imaginary
-// parts of the DC and (even N) Nyquist bins are ignored.
+// parts of the DC and (even N) Nyquist bins are ignored.  pairs: odd N may
+// transform two columns as the real and imaginary part of one (a value that is
+// not finite then reaches both).
 int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int64_t batch, double scale,
-            void* s0, void* s1, void* s2, hipStream_t st, int maxr = 16);
+            void* s0, void* s1, void* s2, hipStream_t st, int maxr = 16, bool pairs = false);
 
 }  // namespace zdt

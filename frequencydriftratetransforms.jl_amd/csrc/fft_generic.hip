@@ -130,50 +130,73 @@ __global__ __launch_bounds__(256) void scale_copy(const cplx<T>* __restrict__ in
   }
 }
 
-// ---------------------------------------------------------------- four-step transforms
+static int pow2_floor(int64_t x) {
+  int r = 1;
+  while (static_cast<int64_t>(r) * 2 <= x) r *= 2;
+  return r;
+}
+
+// ---------------------------------------------------------------- transforms in LDS
 //
-// For FP32 transforms along a contiguous axis with N = N1 * N2 (N1 <= 1024,
-// N2 <= 2048, N <= 2^20) the passes are grouped into two kernels that each
-// move the data through HBM once (the "four-step" FFT, D. H. Bailey, "FFTs in
-// external or hierarchical memory", 1990):
+// FP32 transforms along a contiguous axis run as Stockham passes on one LDS
+// buffer: each pass reads its butterflies' inputs into registers, synchronizes,
+// and writes the outputs in place.  N <= FS_ONE takes one kernel (fs_one, T
+// transforms a block).  Longer ones with N = N1 * N2 (N1 <= 1024, N2 <= 2048, N <=
+// 2^20) take two kernels that each move the data through HBM once (the
+// "four-step" FFT, D. H. Bailey, "FFTs in external or hierarchical memory", 1990):
 //   fs_cols  X1[n2 + N2 k1] = W_N^{n2 k1} sum_{n1} x[n2 + N2 n1] W_N1^{n1 k1}
 //            (TC adjacent columns n2 per block, so loads and stores are
 //            TC-element runs)
 //   fs_rows  X[k1 + N1 k2] = sum_{n2} X1[n2 + N2 k1] W_N2^{n2 k2}
 //            (TR adjacent rows k1 per block; the stores are TR-element runs)
-// Inside a block the sub-transforms run as Stockham passes on one LDS buffer
-// of up to FS_E elements: each pass reads its butterflies' inputs into
-// registers, synchronizes, and writes the outputs in place.  Twiddles are
-// W_N^m = thi[m >> 10] * tlo[m & 1023] from two 1024-entry tables held in LDS
-// (the sub-transform twiddle W_L^e is W_N^{e N/L}).  The inverse is
-// conj(forward(conj(x))): fs_cols conjugates on load, fs_rows on store.
+// A pass reads its twiddles W_{Ns R}^{r k} from a table of its own in LDS
+// (contiguous or broadcast reads, no products); the radices (up to 16, the
+// composite ones 6, 9, 10, 12, 14, 15 among them) are chosen for the fewest
+// passes.  The four-step and c2r twiddles of a thread's 16 elements are
+// products of four starts and four steps evaluated from exact phases.  The
+// inverse is conj(forward(conj(x))), conjugated on the first load and the last
+// store, where the real transforms' packing happens too (fs_mode).
+//
+// Bound: HBM traffic overlapped badly with the passes' LDS latency (two blocks a
+// CU; loads, passes and stores of one block are serial).  Against prime radices
+// up to 13 and 16 with one twiddle table of the whole length in global memory
+// (us): Nf = 10^6, 129 rates (1.03 GB through fs_cols, as much through fs_rows)
+// c2r columns 412 -> 318, rows 370 -> 295; r2c columns 59 -> 44.  Odd Nf = 99225, 77
+// rates, two columns a transform instead of a zero imaginary part: 84 + 68 + 40
+// for filling in the Hermitian half and taking the real part -> 56 + 44.  Nf =
+// 4096, 33 rates: six launches of 5 to 6 -> two of 5 (fs_one).  Persistent blocks
+// that load the next rows before the passes spill (128 VGPRs): 295 -> 569.
 
 constexpr int FS_T = 512;    // threads per block
-constexpr int FS_E = 8192;   // elements per block (TC * N1 or TR * N2)
-constexpr int FS_LGB = 10;   // table split
-constexpr int FS_TAB = 1 << FS_LGB;
+constexpr int FS_E = 8192;   // elements per block of fs_cols / fs_rows (TC * N1 or TR * N2)
+constexpr int FS_ONE = 4096; // elements per block of fs_one
 constexpr int FS_MAXP = 12;  // passes per sub-transform
+
+enum fs_mode {
+  FS_C2C,
+  FS_C2R,      // in: half spectra X[0..N] of real sequences of length 2N; out: their N packed pairs
+  FS_R2C,      // fs_one: the reverse
+  FS_ODD_R2C,  // in: real sequences of odd length N; out: X[0 .. N/2]
+  FS_ODD_C2R,  // in: half spectra X[0 .. N/2] of two columns (or one); out: the real columns
+};
 
 struct FsArgs {
   const c32* in;
-  int64_t ibs;
+  int64_t ibs;  // between transforms (complex elements; floats for FS_ODD_R2C)
   c32* out;
-  int64_t obs;
-  const c32* tlo;
-  const c32* thi;
-  int N, N1, N2, T;  // T = TC (fs_cols) or TR (fs_rows)
-  int nhi;           // entries of thi
+  int64_t obs;  // (floats for FS_ODD_C2R)
+  const c32* tw;
+  int ntw;
+  int N, N1, N2, T;  // T = TC (fs_cols), TR (fs_rows) or transforms per block (fs_one)
   int np;            // passes of the sub-transform
   int rad[FS_MAXP];
-  int inverse;
+  int inverse, mode;
+  int64_t batch;     // transforms
+  int64_t ncol;      // FS_ODD_C2R: real columns
+  int pair;          // FS_ODD_C2R: two columns a transform
   float scale;
-  float pscale;  // fs_cols<true>: scale of the c2r pre-pass
-  c32 w2;        // fs_cols<true>: W_{2N}^1
+  double h;          // 1/N
 };
-
-__device__ __forceinline__ c32 fs_tw(const c32* tl, const c32* th, int m) {
-  return cmul(th[m >> FS_LGB], tl[m & (FS_TAB - 1)]);
-}
 
 // u / d for u * d < 2^32 by one high multiply with m = ceil(2^32 / d)
 // (m = 0 marks d = 1)
@@ -189,12 +212,13 @@ __device__ __forceinline__ int fs_quo(int u, FsDiv q) {
 }
 
 // One Stockham pass of radix R over T interleaved transforms of length L
-// held in buf (element n of transform c at n * T + c, T a power of two).
-// Butterfly u covers transform c = u mod T and index j = u / T < L/R.  Every
-// index is below 2^13, so j mod Ns is an exact high multiply.
-template <int R>
-__device__ __forceinline__ void fs_pass(c32* buf, const c32* tl, const c32* th, int L, int T, int Ns, int mstep) {
-  constexpr int NB = (FS_E / R + FS_T - 1) / FS_T;
+// held in buf (element n of transform c at n * T + c, T a power of two, L * T <=
+// E).  Butterfly u covers transform c = u mod T and index j = u / T < L/R.  Every
+// index is below 2^13, so j mod Ns is an exact high multiply.  tw: the pass's
+// twiddles W_{Ns R}^{r k} at (r - 1) Ns + k (none for Ns = 1).
+template <int R, int E>
+__device__ __forceinline__ void fs_pass(c32* buf, const c32* tw, int L, int T, int Ns) {
+  constexpr int NB = (E / R + FS_T - 1) / FS_T;
   const int Lr = L / R;
   const int nbf = Lr * T;
   const int lgT = __ffs(T) - 1;
@@ -211,11 +235,12 @@ __device__ __forceinline__ void fs_pass(c32* buf, const c32* tl, const c32* th, 
       const int c = u & (T - 1), j = u >> lgT;
 #pragma unroll
       for (int r = 0; r < R; ++r) v[i][r] = buf[(j + r * Lr) * T + c];
-      const int k = j - fs_quo(j, dNs) * Ns;
-      if (k != 0) {
+      if (Ns > 1) {  // uniform
+        const int k = j - fs_quo(j, dNs) * Ns;
 #pragma unroll
-        for (int r = 1; r < R; ++r) v[i][r] = cmul(v[i][r], fs_tw(tl, th, r * k * mstep));
+        for (int r = 1; r < R; ++r) v[i][r] = cmul(v[i][r], tw[(r - 1) * Ns + k]);
       }
+      dft<float, R>(v[i]);
     }
   }
   __syncthreads();
@@ -225,7 +250,6 @@ __device__ __forceinline__ void fs_pass(c32* buf, const c32* tl, const c32* th, 
     if (u < nbf) {
       const int c = u & (T - 1), j = u >> lgT;
       const int k = j - fs_quo(j, dNs) * Ns;
-      dft<float, R>(v[i]);
       const int ob = ((j - k) * R + k) * T + c;
 #pragma unroll
       for (int r = 0; r < R; ++r) buf[ob + r * Ns * T] = v[i][r];
@@ -236,128 +260,183 @@ __device__ __forceinline__ void fs_pass(c32* buf, const c32* tl, const c32* th, 
 
 // all passes of the T interleaved sub-transforms of length L (natural order in
 // and out)
-__device__ __forceinline__ void fs_dft(c32* buf, const c32* tl, const c32* th, const FsArgs& a, int L) {
+template <int E>
+__device__ __forceinline__ void fs_dft(c32* buf, const c32* tw, const FsArgs& a, int L) {
   int Ns = 1;
   for (int p = 0; p < a.np; ++p) {
     const int R = a.rad[p];
-    const int mstep = a.N / (Ns * R);  // W_{Ns R}^{r k} = W_N^{r k mstep}
     switch (R) {
-      case 2: fs_pass<2>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 3: fs_pass<3>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 4: fs_pass<4>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 5: fs_pass<5>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 7: fs_pass<7>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 8: fs_pass<8>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 11: fs_pass<11>(buf, tl, th, L, a.T, Ns, mstep); break;
-      case 13: fs_pass<13>(buf, tl, th, L, a.T, Ns, mstep); break;
-      default: fs_pass<16>(buf, tl, th, L, a.T, Ns, mstep); break;
+#define ZDT_FS_CASE(RR)                           \
+  case RR:                                        \
+    fs_pass<RR, E>(buf, tw, L, a.T, Ns);          \
+    break;
+      ZDT_FS_CASE(2)
+      ZDT_FS_CASE(3)
+      ZDT_FS_CASE(4)
+      ZDT_FS_CASE(5)
+      ZDT_FS_CASE(6)
+      ZDT_FS_CASE(7)
+      ZDT_FS_CASE(8)
+      ZDT_FS_CASE(9)
+      ZDT_FS_CASE(10)
+      ZDT_FS_CASE(11)
+      ZDT_FS_CASE(12)
+      ZDT_FS_CASE(13)
+      ZDT_FS_CASE(14)
+      ZDT_FS_CASE(15)
+      ZDT_FS_CASE(16)
+#undef ZDT_FS_CASE
     }
+    if (Ns > 1) tw += (R - 1) * Ns;
     Ns *= R;
   }
 }
 
-__device__ __forceinline__ void fs_tables(c32* tl, c32* th, const FsArgs& a) {
-  for (int i = threadIdx.x; i < FS_TAB; i += FS_T) tl[i] = a.tlo[i];
-  for (int i = threadIdx.x; i < a.nhi; i += FS_T) th[i] = a.thi[i];
+// W^{n0 + i dn}, i < 16, W = e^{-2 pi i h}: four starts times four steps
+struct FsProg {
+  c32 a[4], b[4];
+  __device__ __forceinline__ FsProg(int n0, int dn, double h) {
+    const c32 s1 = cis_nh(-static_cast<double>(dn), h);
+    a[0] = cis_nh(-static_cast<double>(n0), h);
+    a[1] = cmul(a[0], s1);
+    a[2] = cmul(a[0], cmul(s1, s1));
+    a[3] = cmul(a[2], s1);
+    b[1] = cis_nh(-4.0 * static_cast<double>(dn), h);
+    b[2] = cmul(b[1], b[1]);
+    b[3] = cmul(b[2], b[1]);
+  }
+  __device__ __forceinline__ c32 operator()(int i) const { return i < 4 ? a[i] : cmul(a[i & 3], b[i >> 2]); }
+};
+
+// the packed sequence of the c2r transform: Z[k] = E + i O with
+// E = (p + conj q)/2, O = W_{2N}^{-k} (p - conj q)/2, p = X[k], q = X[N-k], w = W_{2N}^k;
+// Im X[0] and Im X[N] are ignored
+__device__ __forceinline__ c32 c2r_pack(int k, c32 p, c32 q, c32 w) {
+  if (k == 0) return {0.5f * (p.x + q.x), 0.5f * (p.x - q.x)};
+  const c32 Ev = {0.5f * (p.x + q.x), 0.5f * (p.y - q.y)};
+  const c32 D = {0.5f * (p.x - q.x), 0.5f * (p.y + q.y)};
+  const c32 O = cmulc(D, w);
+  return {Ev.x - O.y, Ev.y + O.x};
 }
 
-// columns: block = (batch b, columns n2 in [c0, c0 + TC)); TC is a power of two.
-// C2R: the input is the half spectrum X[0..N] of a real sequence of length 2N
-// (column stride ibs) and the kernel forms the packed sequence of the c2r
-// transform on load (as c2r_pre): Z[k] = (E + i O) pscale with
-// E = (X[k] + conj X[N-k])/2, O = W_{2N}^{-k} (X[k] - conj X[N-k])/2,
-// W_{2N}^k = W_N^{k/2} (W_{2N}^1 for odd k); Im X[0] and Im X[N] are ignored.
-template <bool C2R>
+// element n of transform b for the modes that need no twiddle, before the
+// conjugation of the inverse
+__device__ __forceinline__ c32 fs_input(const FsArgs& a, int64_t b, int n) {
+  if (a.mode == FS_ODD_R2C) return {reinterpret_cast<const float*>(a.in)[b * a.ibs + n], 0.0f};
+  if (a.mode == FS_ODD_C2R) {
+    // the full Hermitian spectra of columns c0 and c0 + 1 as A + i B
+    const bool up = 2 * n > a.N;
+    const int k = up ? a.N - n : n;
+    const int64_t c0 = a.pair ? 2 * b : b;
+    c32 A = a.in[c0 * a.ibs + k], B = {0.0f, 0.0f};
+    if (a.pair && c0 + 1 < a.ncol) B = a.in[(c0 + 1) * a.ibs + k];
+    if (n == 0) A.y = B.y = 0.0f;
+    if (up) {
+      A.y = -A.y;
+      B.y = -B.y;
+    }
+    return {A.x - B.y, A.y + B.x};
+  }
+  return a.in[b * a.ibs + n];
+}
+
+// element k of transform b, scaled and (inverse) conjugated
+__device__ __forceinline__ void fs_output(const FsArgs& a, int64_t b, int k, c32 v) {
+  v = {v.x * a.scale, (a.inverse ? -v.y : v.y) * a.scale};
+  if (a.mode == FS_ODD_C2R) {
+    float* out = reinterpret_cast<float*>(a.out);
+    const int64_t c0 = a.pair ? 2 * b : b;
+    out[c0 * a.obs + k] = v.x;
+    if (a.pair && c0 + 1 < a.ncol) out[(c0 + 1) * a.obs + k] = v.y;
+  } else if (a.mode != FS_ODD_R2C || 2 * k < a.N) {
+    a.out[b * a.obs + k] = v;
+  }
+}
+
+// The unit of this block, of n units in all, such that each of the eight XCDs
+// (blocks are dealt to them round-robin) takes one contiguous range of them;
+// -1 for a block without one.  Neighbouring tiles share the cache lines at their
+// edges (TC-element runs on rows that start anywhere) and so one XCD's L2: Nf =
+// 10^6, 129 rates: fs_rows 370 -> 313 us, fs_cols 341 -> 329; 21609 x 234 rows
+// 50 -> 48, columns unchanged.
+__device__ __forceinline__ int64_t xcd_block(int64_t n) {
+  const int64_t per = (n + 7) / 8;
+  const int64_t u = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  return (blockIdx.x >> 3) < per && u < n ? u : -1;
+}
+
+// columns: block = (batch b, columns n2 in [c0, c0 + TC)); TC is a power of two
 __global__ __launch_bounds__(FS_T, 4) void fs_cols(FsArgs a) {
   __shared__ c32 buf[FS_E];
-  __shared__ c32 tl[FS_TAB], th[FS_TAB];
-  fs_tables(tl, th, a);
+  __shared__ c32 tw[1024];
+  for (int i = threadIdx.x; i < a.ntw; i += FS_T) tw[i] = a.tw[i];
   const int TC = a.T;
   const int lgT = __ffs(TC) - 1;
   const int tiles = (a.N2 + TC - 1) / TC;
-  const int64_t b = blockIdx.x / tiles;
-  int q = static_cast<int>(blockIdx.x % tiles);
-  if (C2R && (tiles & 15) == 0) {
-    // tile i and its mirror tiles-1-i (which reads the same columns of X)
-    // eight blocks apart: same XCD (blocks go round-robin over the eight),
-    // in flight together, so the second read of a column hits in L2
-    const int g = q >> 4, x = q & 15;
-    q = x < 8 ? g * 8 + x : tiles - 1 - (g * 8 + x - 8);
-  }
-  const int c0 = q * TC;
+  const int64_t blk = xcd_block(tiles * a.batch);
+  if (blk < 0) return;
+  const int64_t b = blk / tiles;
+  const int c0 = static_cast<int>(blk % tiles) * TC;
   const int E = a.N1 * TC;
-  if constexpr (!C2R) {
-    const c32* src = a.in + b * a.ibs + c0;
-    // all loads issued before the first LDS store
-    c32 v[FS_E / FS_T];
-#pragma unroll
-    for (int i = 0; i < FS_E / FS_T; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-      const int c = e & (TC - 1), n = e >> lgT;
-      v[i] = {0.0f, 0.0f};
-      if (e < E && c0 + c < a.N2) v[i] = src[c + static_cast<int64_t>(n) * a.N2];
-    }
-#pragma unroll
-    for (int i = 0; i < FS_E / FS_T; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-      if (e < E) buf[e] = {v[i].x, a.inverse ? -v[i].y : v[i].y};  // element n of column c at n * TC + c
-    }
-  } else {
+  // element i of a thread: column c of the block, row n0 + i dn
+  const int c = static_cast<int>(threadIdx.x) & (TC - 1), r0 = static_cast<int>(threadIdx.x) >> lgT;
+  const int dr = FS_T >> lgT;
+  const bool in = c0 + c < a.N2;
+  constexpr int PER = FS_E / FS_T;
+  // all loads issued before the first LDS store
+  c32 v[PER];
+  if (a.mode == FS_C2R) {
     const c32* X = a.in + b * a.ibs;
-    c32 p[FS_E / FS_T], q[FS_E / FS_T];
+    c32 w[PER];
 #pragma unroll
-    for (int i = 0; i < FS_E / FS_T; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-      const int c = e & (TC - 1), n = e >> lgT;
-      p[i] = q[i] = {0.0f, 0.0f};
-      if (e < E && c0 + c < a.N2) {
-        const int k = c0 + c + n * a.N2;
-        p[i] = X[k];
-        q[i] = X[a.N - k];  // X[N] for k = 0
+    for (int i = 0; i < PER; ++i) {
+      v[i] = w[i] = {0.0f, 0.0f};
+      if (in && r0 + i * dr < a.N1) {
+        const int k = c0 + c + (r0 + i * dr) * a.N2;
+        v[i] = X[k];
+        w[i] = X[a.N - k];  // X[N] for k = 0
       }
     }
-    __syncthreads();  // tables
+    const FsProg tp(c0 + c + r0 * a.N2, dr * a.N2, 0.5 * a.h);
 #pragma unroll
-    for (int i = 0; i < FS_E / FS_T; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-      const int c = e & (TC - 1), n = e >> lgT;
-      const int k = c0 + c + n * a.N2;
-      c32 z;
-      if (k == 0) {
-        z = {0.5f * (p[i].x + q[i].x), 0.5f * (p[i].x - q[i].x)};
-      } else {
-        const c32 Ev = {0.5f * (p[i].x + q[i].x), 0.5f * (p[i].y - q[i].y)};
-        const c32 D = {0.5f * (p[i].x - q[i].x), 0.5f * (p[i].y + q[i].y)};
-        c32 w = fs_tw(tl, th, k >> 1);
-        if (k & 1) w = cmul(w, a.w2);
-        const c32 O = cmulc(D, w);
-        z = {Ev.x - O.y, Ev.y + O.x};
-      }
-      if (e < E) buf[e] = {z.x * a.pscale, -z.y * a.pscale};  // the inverse: conjugated
+    for (int i = 0; i < PER; ++i) v[i] = c2r_pack(c0 + c + (r0 + i * dr) * a.N2, v[i], w[i], tp(i));
+  } else {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      v[i] = {0.0f, 0.0f};
+      if (in && r0 + i * dr < a.N1) v[i] = fs_input(a, b, c0 + c + (r0 + i * dr) * a.N2);
     }
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = static_cast<int>(threadIdx.x) + i * FS_T;
+    if (e < E) buf[e] = {v[i].x, a.inverse ? -v[i].y : v[i].y};  // element n of column c at n * TC + c
   }
   __syncthreads();
-  fs_dft(buf, tl, th, a, a.N1);
-  c32* dst = a.out + b * static_cast<int64_t>(a.N) + c0;
-  int tid = static_cast<int>(threadIdx.x);
-  asm volatile("" : "+v"(tid));  // keeps the store indices from being computed before the passes
+  fs_dft<FS_E>(buf, tw, a, a.N1);
+  if (!in) return;
+  c32* dst = a.out + b * static_cast<int64_t>(a.N) + c0 + c;
+  int k0 = r0;
+  asm volatile("" : "+v"(k0));  // keeps the store indices from being computed before the passes
+  const FsProg tp((c0 + c) * k0, (c0 + c) * dr, a.h);
 #pragma unroll
-  for (int i = 0; i < FS_E / FS_T; ++i) {
-    const int e = tid + i * FS_T;
-    const int c = e & (TC - 1), k1 = e >> lgT;
-    if (e < E && c0 + c < a.N2) dst[c + static_cast<int64_t>(k1) * a.N2] = cmul(buf[e], fs_tw(tl, th, (c0 + c) * k1));
+  for (int i = 0; i < PER; ++i) {
+    const int k1 = k0 + i * dr;
+    if (k1 < a.N1) dst[static_cast<int64_t>(k1) * a.N2] = cmul(buf[k1 * TC + c], tp(i));
   }
 }
 
 // rows: block = (batch b, rows k1 in [r0, r0 + TR)); TR is a power of two
 __global__ __launch_bounds__(FS_T, 4) void fs_rows(FsArgs a) {
   __shared__ c32 buf[FS_E];
-  __shared__ c32 tl[FS_TAB], th[FS_TAB];
-  fs_tables(tl, th, a);
+  __shared__ c32 tw[2048];
+  for (int i = threadIdx.x; i < a.ntw; i += FS_T) tw[i] = a.tw[i];
   const int TR = a.T;
   const int tiles = (a.N1 + TR - 1) / TR;
-  const int64_t b = blockIdx.x / tiles;
-  const int r0 = static_cast<int>(blockIdx.x % tiles) * TR;
+  const int64_t blk = xcd_block(tiles * a.batch);
+  if (blk < 0) return;
+  const int64_t b = blk / tiles;
+  const int r0 = static_cast<int>(blk % tiles) * TR;
   const int nrow = min(TR, a.N1 - r0);
   const c32* src = a.in + b * static_cast<int64_t>(a.N) + static_cast<int64_t>(r0) * a.N2;
   const int E = a.N2 * TR;
@@ -380,68 +459,160 @@ __global__ __launch_bounds__(FS_T, 4) void fs_rows(FsArgs a) {
     }
   }
   __syncthreads();
-  fs_dft(buf, tl, th, a, a.N2);
-  c32* dst = a.out + b * a.obs + r0;
+  fs_dft<FS_E>(buf, tw, a, a.N2);
   int tid = static_cast<int>(threadIdx.x);
   asm volatile("" : "+v"(tid));  // keeps the store indices from being computed before the passes
 #pragma unroll
   for (int i = 0; i < FS_E / FS_T; ++i) {
     const int e = tid + i * FS_T;
     const int c = e & (TR - 1), k2 = e >> lgT;
-    if (e < E && c < nrow) {
-      c32 v = buf[e];
-      v = {v.x * a.scale, (a.inverse ? -v.y : v.y) * a.scale};
-      dst[c + static_cast<int64_t>(k2) * a.N1] = v;
-    }
+    if (e < E && c < nrow) fs_output(a, b, r0 + c + k2 * a.N1, buf[e]);
   }
 }
 
-// c2r (c2r = true): in is the half spectrum X[0..N] (column stride ibs) of real
-// sequences of length 2N, out their values as N complex pairs, scaled by
-// `scale` / N (the normalized inverse times scale).
-static int fs_c2c(const FftPlan* p, const c32* in, int64_t ibs, c32* out, int64_t obs, int64_t batch, bool inverse,
-                  double scale, c32* s0, hipStream_t st, bool c2r = false) {
+// whole transforms: block = transforms [T blockIdx, T blockIdx + T), element n of
+// transform c at n * T + c; LDS: N * T elements, then the twiddles
+__global__ __launch_bounds__(FS_T, 4) void fs_one(FsArgs a) {
+  extern __shared__ c32 lds[];
+  c32* buf = lds;
+  c32* tw = lds + a.N * a.T;
+  for (int i = threadIdx.x; i < a.ntw; i += FS_T) tw[i] = a.tw[i];
+  const int64_t b0 = static_cast<int64_t>(blockIdx.x) * a.T;
+  const int nt = static_cast<int>(min(static_cast<int64_t>(a.T), a.batch - b0));
+  const int E = a.N * nt;
+  const FsDiv dN = fs_div(a.N);
+  constexpr int PER = FS_ONE / FS_T;
+  {
+    c32 v[PER], w[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
+      const int c = fs_quo(e, dN), n = e - c * a.N;
+      v[i] = w[i] = {0.0f, 0.0f};
+      if (e < E) {
+        if (a.mode == FS_C2R) {
+          const c32* X = a.in + (b0 + c) * a.ibs;
+          v[i] = X[n];
+          w[i] = X[a.N - n];
+        } else {
+          v[i] = fs_input(a, b0 + c, n);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
+      const int c = fs_quo(e, dN), n = e - c * a.N;
+      if (e < E) {
+        if (a.mode == FS_C2R) v[i] = c2r_pack(n, v[i], w[i], cis_nh(-static_cast<double>(n), 0.5 * a.h));
+        buf[n * a.T + c] = {v[i].x, a.inverse ? -v[i].y : v[i].y};
+      }
+    }
+  }
+  __syncthreads();
+  fs_dft<FS_ONE>(buf, tw, a, a.N);
+  int tid = static_cast<int>(threadIdx.x);
+  asm volatile("" : "+v"(tid));
+  if (a.mode == FS_R2C) {
+    // X[k] = E + W_{2N}^k O, X[N-k] = conj(E - W_{2N}^k O), E = (Z[k] + conj Z[N-k])/2,
+    // O = (Z[k] - conj Z[N-k])/(2i)
+    const int half = a.N / 2 + 1;
+    const FsDiv dH = fs_div(half);
+    for (int e = tid; e < half * nt; e += FS_T) {
+      const int c = fs_quo(e, dH), k = e - c * half;
+      c32* x = a.out + (b0 + c) * a.obs;
+      const c32 z = buf[k * a.T + c];
+      if (k == 0) {
+        x[0] = {z.x + z.y, 0.0f};
+        x[a.N] = {z.x - z.y, 0.0f};
+      } else {
+        const c32 y = buf[(a.N - k) * a.T + c];
+        const c32 Ev = {0.5f * (z.x + y.x), 0.5f * (z.y - y.y)};
+        const c32 O = {0.5f * (z.y + y.y), -0.5f * (z.x - y.x)};
+        const c32 WO = cmul(cis_nh(-static_cast<double>(k), 0.5 * a.h), O);
+        x[k] = cadd(Ev, WO);
+        if (2 * k != a.N) x[a.N - k] = {Ev.x - WO.x, -(Ev.y - WO.y)};
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = tid + i * FS_T;
+    const int c = fs_quo(e, dN), k = e - c * a.N;
+    if (e < E) fs_output(a, b0 + c, k, buf[k * a.T + c]);
+  }
+}
+
+static bool fs_has(const FftPlan* p) { return !p->rad0.empty() || p->N1 > 0; }
+
+static void fs_passes(FsArgs* a, const std::vector<int>& rad, const c32* tw) {
+  a->np = static_cast<int>(rad.size());
+  int Ns = 1;
+  a->ntw = 0;
+  for (int i = 0; i < a->np; ++i) {
+    a->rad[i] = rad[i];
+    if (Ns > 1) a->ntw += (rad[i] - 1) * Ns;
+    Ns *= rad[i];
+  }
+  a->tw = tw;
+}
+
+// `batch` transforms of plan p in mode `mode`; the result is multiplied by
+// scale.  s0: scratch of N * batch elements (four-step only).
+static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void* out, int64_t obs, int64_t batch,
+                  bool inverse, double scale, c32* s0, hipStream_t st, int64_t ncol = 0, bool pair = false) {
   FsArgs a;
-  a.tlo = p->tlo;
-  a.thi = p->thi;
   a.N = static_cast<int>(p->N);
   a.N1 = p->N1;
   a.N2 = p->N2;
-  a.nhi = static_cast<int>((p->N + FS_TAB - 1) / FS_TAB);
   a.inverse = inverse ? 1 : 0;
+  a.batch = batch;
+  a.ncol = ncol;
+  a.pair = pair ? 1 : 0;
+  a.h = 1.0 / static_cast<double>(p->N);
   const double bytes = 16.0 * static_cast<double>(p->N) * static_cast<double>(batch);
+  if (!p->rad0.empty()) {
+    a.in = static_cast<const c32*>(in);
+    a.ibs = ibs;
+    a.out = static_cast<c32*>(out);
+    a.obs = obs;
+    a.mode = mode;
+    a.scale = static_cast<float>(scale);
+    // as many transforms a block as fit, but blocks for every CU first
+    int T = std::min<int>(16, pow2_floor(FS_ONE / p->N));
+    while (T > 1 && batch / T < 512) T /= 2;
+    a.T = T;
+    fs_passes(&a, p->rad0, p->tw0);
+    const size_t lds = (static_cast<size_t>(p->N) * T + a.ntw) * sizeof(c32);
+    ProfScope ps(st, "fft_fs_one", bytes);
+    fs_one<<<static_cast<unsigned>((batch + T - 1) / T), FS_T, lds, st>>>(a);
+    ZDT_CHECK_LAUNCH("fs_one");
+    return ZDT_OK;
+  }
   {
-    a.in = in;
+    a.in = static_cast<const c32*>(in);
     a.ibs = ibs;
     a.out = s0;
     a.obs = p->N;
+    a.mode = mode;
     a.T = p->TC;
-    a.np = static_cast<int>(p->rad1.size());
-    for (int i = 0; i < a.np; ++i) a.rad[i] = p->rad1[i];
     a.scale = 1.0f;
-    a.pscale = static_cast<float>(scale / static_cast<double>(p->N));
-    const double ph = -3.14159265358979323846 / static_cast<double>(p->N);
-    a.w2 = {static_cast<float>(std::cos(ph)), static_cast<float>(std::sin(ph))};
-    const int64_t grid = (p->N2 + p->TC - 1) / p->TC * batch;
-    if (c2r) {
-      ProfScope ps(st, "fft_fs_cols_c2r", bytes + 8.0 * static_cast<double>(p->N) * static_cast<double>(batch));
-      fs_cols<true><<<static_cast<unsigned>(grid), FS_T, 0, st>>>(a);
-    } else {
-      ProfScope ps(st, "fft_fs_cols", bytes);
-      fs_cols<false><<<static_cast<unsigned>(grid), FS_T, 0, st>>>(a);
-    }
+    fs_passes(&a, p->rad1, p->tw1);
+    const int64_t grid = ((p->N2 + p->TC - 1) / p->TC * batch + 7) / 8 * 8;
+    ProfScope ps(st, mode == FS_C2R ? "fft_fs_cols_c2r" : "fft_fs_cols", bytes);
+    fs_cols<<<static_cast<unsigned>(grid), FS_T, 0, st>>>(a);
     ZDT_CHECK_LAUNCH("fs_cols");
   }
   {
     a.in = s0;
     a.ibs = p->N;
-    a.out = out;
+    a.out = static_cast<c32*>(out);
     a.obs = obs;
     a.T = p->TR;
-    a.np = static_cast<int>(p->rad2.size());
-    for (int i = 0; i < a.np; ++i) a.rad[i] = p->rad2[i];
-    a.scale = c2r ? 1.0f : static_cast<float>(scale);
-    const int64_t grid = (p->N1 + p->TR - 1) / p->TR * batch;
+    a.scale = static_cast<float>(scale);
+    fs_passes(&a, p->rad2, p->tw2);
+    const int64_t grid = ((p->N1 + p->TR - 1) / p->TR * batch + 7) / 8 * 8;
     ProfScope ps(st, "fft_fs_rows", bytes);
     fs_rows<<<static_cast<unsigned>(grid), FS_T, 0, st>>>(a);
     ZDT_CHECK_LAUNCH("fs_rows");
@@ -449,29 +620,51 @@ static int fs_c2c(const FftPlan* p, const c32* in, int64_t ibs, c32* out, int64_
   return ZDT_OK;
 }
 
-static int pow2_floor(int64_t x) {
-  int r = 1;
-  while (static_cast<int64_t>(r) * 2 <= x) r *= 2;
-  return r;
+// Radices of an LDS transform of length n with the fewest passes (fewest large
+// ones among those): composite and power-of-two radices up to maxr, primes up to 13.
+// False if n has another prime factor.
+static bool fs_radices(int64_t n, int maxr, std::vector<int>* best) {
+  best->clear();
+  if (n == 1) return true;
+  bool found = false;
+  for (int r : {16, 15, 14, 13, 12, 11, 10, 9, 8, 7, 6, 5, 4, 3, 2}) {
+    const bool prime = r == 2 || r == 3 || r == 5 || r == 7 || r == 11 || r == 13;
+    if (n % r != 0 || (!prime && r > maxr)) continue;
+    std::vector<int> sub;
+    if (!fs_radices(n / r, std::min(maxr, r), &sub)) continue;  // non-increasing
+    if (!sub.empty() && sub[0] > r) continue;
+    if (!found || sub.size() + 1 <= best->size()) {  // later candidates start smaller
+      best->assign(1, r);
+      best->insert(best->end(), sub.begin(), sub.end());
+      found = true;
+    }
+  }
+  return found;
 }
 
-// Chooses the four-step split of an FP32 plan (sets p->N1 = 0 if none applies):
-// the one whose column and row blocks both move the longest contiguous runs.
+// Chooses the LDS form of an FP32 plan (neither if none applies): one kernel, or
+// the four-step split whose column and row blocks both move the longest
+// contiguous runs and, among those, takes the fewest passes.
 static void fs_choose(FftPlan* p, int maxr) {
   p->N1 = 0;
   const int64_t N = p->N;
-  if (p->dbl || N < 4096 || N > (int64_t{1} << 20)) return;
+  if (p->dbl || N < 2) return;
+  if (N <= FS_ONE) {
+    if (!fs_radices(N, maxr, &p->rad0) || static_cast<int>(p->rad0.size()) > FS_MAXP) p->rad0.clear();
+    return;
+  }
+  if (N > (int64_t{1} << 20)) return;
   int best = -1;
   for (int64_t n1 = 2; n1 <= 1024; ++n1) {
     if (N % n1 != 0) continue;
     const int64_t n2 = N / n1;
     if (n2 < 2 || n2 > 2048) continue;
     std::vector<int> r1, r2;
-    if (!fft_factorize(n1, &r1, maxr) || !fft_factorize(n2, &r2, maxr)) continue;
+    if (!fs_radices(n1, maxr, &r1) || !fs_radices(n2, maxr, &r2)) continue;
     if (static_cast<int>(r1.size()) > FS_MAXP || static_cast<int>(r2.size()) > FS_MAXP) continue;
     const int tc = std::min(16, pow2_floor(FS_E / n1));
     const int tr = std::min(16, pow2_floor(FS_E / n2));
-    const int score = std::min(tc, tr) * 100 + tc;
+    const int score = (std::min(tc, tr) * 100 + tc) * 32 + 31 - static_cast<int>(r1.size() + r2.size());
     if (score > best) {
       best = score;
       p->N1 = static_cast<int>(n1);
@@ -482,6 +675,28 @@ static void fs_choose(FftPlan* p, int maxr) {
       p->rad2 = r2;
     }
   }
+}
+
+// the passes' twiddles W_{Ns R}^{r k} (r = 1 .. R-1, k < Ns) of every pass but the
+// first, in order
+static std::vector<c32> fs_twiddles(const std::vector<int>& rad) {
+  std::vector<c32> t;
+  int64_t Ns = 1;
+  for (int R : rad) {
+    if (Ns > 1)
+      for (int r = 1; r < R; ++r)
+        for (int64_t k = 0; k < Ns; ++k) {
+          const int64_t n = Ns * R, m = r * k;  // m < n
+          const long double x = 2.0L * 3.14159265358979323846264338327950288L * static_cast<long double>(m) /
+                                static_cast<long double>(n);
+          double c = static_cast<double>(cosl(x)), sn = -static_cast<double>(sinl(x));
+          if (4 * m == n || 4 * m == 3 * n) c = 0.0;
+          if (2 * m == n) sn = 0.0;
+          t.push_back({static_cast<float>(c), static_cast<float>(sn)});
+        }
+    Ns *= R;
+  }
+  return t;
 }
 
 // ---------------------------------------------------------------- plans
@@ -563,35 +778,30 @@ int fft_plan_get(int64_t N, bool dbl, const FftPlan** out, int maxr) {
     return hip_fail(e, "hipMemcpy(twiddles)");
   }
   fs_choose(p, maxr);
-  if (p->N1 > 0) {
-    // W_N^m for m < 1024 and W_N^{1024 m} for m < ceil(N/1024)
-    const int64_t nhi = (N + FS_TAB - 1) / FS_TAB;
-    std::vector<c32> lo(FS_TAB), hi(static_cast<size_t>(nhi));
-    const auto wn = [N](int64_t m) -> c32 {
-      m %= N;
-      const long double a = 2.0L * 3.14159265358979323846264338327950288L * static_cast<long double>(m) /
-                            static_cast<long double>(N);
-      double c = static_cast<double>(cosl(a)), sn = -static_cast<double>(sinl(a));
-      if (4 * m == N || 4 * m == 3 * N) c = 0.0;
-      if (2 * m == N) sn = 0.0;
-      return {static_cast<float>(c), static_cast<float>(sn)};
-    };
-    for (int64_t m = 0; m < FS_TAB; ++m) lo[static_cast<size_t>(m)] = wn(m);
-    for (int64_t m = 0; m < nhi; ++m) hi[static_cast<size_t>(m)] = wn(m * FS_TAB);
-    e = hipMalloc(&p->tlo, (FS_TAB + nhi) * sizeof(c32));
-    if (e != hipSuccess) {
-      (void)hipFree(p->tw);
-      delete p;
-      return fail(ZDT_ENOMEM, "hipMalloc of FFT twiddles failed");
-    }
-    p->thi = p->tlo + FS_TAB;
-    e = hipMemcpy(p->tlo, lo.data(), FS_TAB * sizeof(c32), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(p->thi, hi.data(), nhi * sizeof(c32), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      (void)hipFree(p->tlo);
-      (void)hipFree(p->tw);
-      delete p;
-      return hip_fail(e, "hipMemcpy(twiddles)");
+  {
+    // one allocation for the passes' twiddles of whichever forms the plan has
+    const std::vector<c32> t0 = fs_twiddles(p->rad0), t1 = fs_twiddles(p->rad1), t2 = fs_twiddles(p->rad2);
+    std::vector<c32> all(t0);
+    all.insert(all.end(), t1.begin(), t1.end());
+    all.insert(all.end(), t2.begin(), t2.end());
+    if (!all.empty()) {
+      c32* d = nullptr;
+      e = hipMalloc(&d, all.size() * sizeof(c32));
+      if (e != hipSuccess) {
+        (void)hipFree(p->tw);
+        delete p;
+        return fail(ZDT_ENOMEM, "hipMalloc of FFT twiddles failed");
+      }
+      e = hipMemcpy(d, all.data(), all.size() * sizeof(c32), hipMemcpyHostToDevice);
+      if (e != hipSuccess) {
+        (void)hipFree(d);
+        (void)hipFree(p->tw);
+        delete p;
+        return hip_fail(e, "hipMemcpy(twiddles)");
+      }
+      p->tw0 = d;
+      p->tw1 = d + t0.size();
+      p->tw2 = d + t0.size() + t1.size();
     }
   }
   g_plans[key] = p;
@@ -607,9 +817,8 @@ static int c2c_impl(const FftPlan* p, const void* in, int64_t ies, int64_t ibs, 
   const int64_t N = p->N;
   const cplx<T>* tw = static_cast<const cplx<T>*>(p->tw);
   if constexpr (std::is_same<T, float>::value) {
-    if (p->N1 > 0 && ies == 1 && oes == 1)
-      return fs_c2c(p, static_cast<const c32*>(in), ibs, static_cast<c32*>(out), obs, batch, inverse, scale,
-                    static_cast<c32*>(s0), st);
+    if (fs_has(p) && ies == 1 && oes == 1)
+      return fs_run(p, FS_C2C, in, ibs, out, obs, batch, inverse, scale, static_cast<c32*>(s0), st);
   }
   if (N == 1) {
     // the length-1 DFT is the identity (times scale)
@@ -801,6 +1010,8 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
                                    hipMemcpyDeviceToDevice, st));
     } else {
       ZDT_TRY(fft_plan_get(M, false, &pM, maxr));
+      if (!pM->rad0.empty())  // the untangling in the same kernel
+        return fs_run(pM, FS_R2C, in, ldi / 2, out, ldo, batch, false, 1.0, nullptr, st);
       ZDT_TRY(fft_c2c(pM, in, 1, ldi / 2, Z, 1, M, batch, false, 1.0, s0, s1, st));
     }
     ProfScope ps(st, "r2c_post", 16.0 * static_cast<double>(M * batch));
@@ -811,6 +1022,7 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
   }
   const FftPlan* p = nullptr;
   ZDT_TRY(fft_plan_get(N, false, &p, maxr));
+  if (fs_has(p)) return fs_run(p, FS_ODD_R2C, in, ldi, out, ldo, batch, false, 1.0, static_cast<c32*>(s0), st);
   c32* full = static_cast<c32*>(s2);
   real_to_complex<<<grid_for(N * batch, 256), 256, 0, st>>>(in, ldi, full, N, batch);
   ZDT_CHECK_LAUNCH("real_to_complex");
@@ -823,16 +1035,16 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
 }
 
 int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int64_t batch, double scale,
-            void* s0, void* s1, void* s2, hipStream_t st, int maxr) {
+            void* s0, void* s1, void* s2, hipStream_t st, int maxr, bool pairs) {
   if (N % 2 == 0) {
     const int64_t M = N / 2;
     if (ldo % 2 != 0) return fail(ZDT_EINVAL, "c2r: column stride must be even for even N");
     const FftPlan *pM = nullptr, *pN = nullptr;
     if (M > 1) {
       ZDT_TRY(fft_plan_get(M, false, &pM, maxr));
-      if (pM->N1 > 0)  // the pre-pass fused into the four-step columns kernel
-        return fs_c2c(pM, in, ldi, reinterpret_cast<c32*>(out), ldo / 2, batch, true, scale, static_cast<c32*>(s0),
-                      st, true);
+      if (fs_has(pM))  // the pre-pass on the first load
+        return fs_run(pM, FS_C2R, in, ldi, out, ldo / 2, batch, true, scale / static_cast<double>(M),
+                      static_cast<c32*>(s0), st);
     }
     ZDT_TRY(fft_plan_get(N, false, &pN, maxr));
     c32* Z = static_cast<c32*>(s2);
@@ -853,6 +1065,9 @@ int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int6
   }
   const FftPlan* p = nullptr;
   ZDT_TRY(fft_plan_get(N, false, &p, maxr));
+  if (fs_has(p))
+    return fs_run(p, FS_ODD_C2R, in, ldi, out, ldo, pairs ? (batch + 1) / 2 : batch, true,
+                  scale / static_cast<double>(N), static_cast<c32*>(s0), st, batch, pairs);
   c32* full = static_cast<c32*>(s2);
   hermitian_extend<<<grid_for(N * batch, 256), 256, 0, st>>>(in, ldi, full, N, batch);
   ZDT_CHECK_LAUNCH("hermitian_extend");

@@ -288,7 +288,7 @@ int output_impl(zdt_ws* ws, float* dest) {
   if (ws->ys_src == nullptr) return fail(ZDT_ESTATE, "output!: no post-processed spectra (run zdtfdr! or the steps first)");
   ZDT_TRY(ensure_scratch(ws, real_scratch_bytes(ws)));
   return fft_c2r(ws->Nf, ws->ys_src, ws->ys_ld, dest, ws->Nf, ws->Nr, out_scale(ws), ws->s[0], ws->s[1], ws->s[2],
-                 ws->stream, ws->maxr);
+                 ws->stream, ws->maxr, true);
 }
 
 int run_impl(zdt_ws* ws, float r0, int wkind, const float* window, float* dest) {
