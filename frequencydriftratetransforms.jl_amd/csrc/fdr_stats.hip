@@ -33,13 +33,21 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // one block per (chunk of STAT_ROWS rows, column); grid.y is capped at the
 // launch limit, so a block walks the columns j = blockIdx.y + q*gridDim.y;
-// vec: the columns are 16-byte aligned (float4 loads)
+// vec: the columns are 16-byte aligned (float4 loads).  MAX: rmax[j][q] also takes
+// the largest value of rows [q, q + 1) * FDR_TILE of column j (NaN left out, -inf if
+// there is nothing else), from which hits_count_max knows the tiles without a
+// proto-hit.  Bound by the read of the matrix: 2^20 x 129 in 91 us (5.9 TB/s)
+// without and 93 us with the maxima.
+template <bool MAX>
 __global__ __launch_bounds__(STAT_THREADS) void colstats_partial(const float* __restrict__ fdr, int64_t Nf,
                                                                  int64_t Nr, int64_t ld, double* __restrict__ part,
-                                                                 int nchunk, int vec) {
+                                                                 int nchunk, int vec, float* __restrict__ rmax,
+                                                                 int64_t nreg) {
   const int chunk = blockIdx.x;
   constexpr int NW = STAT_THREADS / 64;
+  constexpr int NREG = static_cast<int>(STAT_ROWS / FDR_TILE);
   __shared__ double sh1[NW], sh2[NW];
+  __shared__ float shm[NW][NREG];
   const int wv = threadIdx.x >> 6;
   for (int64_t j = blockIdx.y; j < Nr; j += gridDim.y) {  // uniform per block
     const float* col = fdr + j * ld;
@@ -48,29 +56,51 @@ __global__ __launch_bounds__(STAT_THREADS) void colstats_partial(const float* __
     int64_t r1 = r0 + STAT_ROWS;
     if (r1 > Nf) r1 = Nf;
     double s1 = 0.0, s2 = 0.0;
+    float mx[NREG];
+#pragma unroll
+    for (int q = 0; q < NREG; ++q) mx[q] = -INFINITY;
     if (vec && r1 - r0 == STAT_ROWS) {
       const float4* p = reinterpret_cast<const float4*>(col + r0);
       constexpr int NV = STAT_ROWS / 4 / STAT_THREADS;
-#pragma unroll 8
+#pragma unroll
       for (int k = 0; k < NV; ++k) {
         const float4 v = p[threadIdx.x + k * STAT_THREADS];
         const double d0 = static_cast<double>(v.x) - c, d1 = static_cast<double>(v.y) - c;
         const double d2 = static_cast<double>(v.z) - c, d3 = static_cast<double>(v.w) - c;
         s1 += (d0 + d1) + (d2 + d3);
         s2 += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
+        if (MAX) {
+          constexpr int PER = NV / NREG;  // loads of a region
+          mx[k / PER] = fmaxf(mx[k / PER], fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+        }
       }
     } else {
-      for (int64_t i = r0 + threadIdx.x; i < r1; i += STAT_THREADS) {
-        const double d = static_cast<double>(col[i]) - c;
-        s1 += d;
-        s2 += d * d;
+#pragma unroll
+      for (int q = 0; q < NREG; ++q) {
+        const int64_t e = r0 + (q + 1) * FDR_TILE < r1 ? r0 + (q + 1) * FDR_TILE : r1;
+        for (int64_t i = r0 + q * FDR_TILE + threadIdx.x; i < e; i += STAT_THREADS) {
+          const float v = col[i];
+          const double d = static_cast<double>(v) - c;
+          s1 += d;
+          s2 += d * d;
+          if (MAX) mx[q] = fmaxf(mx[q], v);
+        }
       }
     }
     s1 = wave_sum(s1);
     s2 = wave_sum(s2);
+    if (MAX) {
+#pragma unroll
+      for (int q = 0; q < NREG; ++q)
+        for (int off = 32; off > 0; off >>= 1) mx[q] = fmaxf(mx[q], __shfl_xor(mx[q], off, 64));
+    }
     if ((threadIdx.x & 63) == 0) {
       sh1[wv] = s1;
       sh2[wv] = s2;
+      if (MAX) {
+#pragma unroll
+        for (int q = 0; q < NREG; ++q) shm[wv][q] = mx[q];
+      }
     }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -82,39 +112,62 @@ __global__ __launch_bounds__(STAT_THREADS) void colstats_partial(const float* __
       part[(j * nchunk + chunk) * 2 + 0] = t1;
       part[(j * nchunk + chunk) * 2 + 1] = t2;
     }
-    __syncthreads();  // sh1/sh2 are rewritten for the next column
+    if (MAX && threadIdx.x < NREG && static_cast<int64_t>(chunk) * NREG + threadIdx.x < nreg) {
+      float m = shm[0][threadIdx.x];
+      for (int w = 1; w < NW; ++w) m = fmaxf(m, shm[w][threadIdx.x]);
+      rmax[j * nreg + static_cast<int64_t>(chunk) * NREG + threadIdx.x] = m;
+    }
+    __syncthreads();  // the shared sums are rewritten for the next column
   }
 }
 
-// per column: mean and corrected variance from the partial sums (fixed order)
-__global__ __launch_bounds__(256) void colstats_final(const float* __restrict__ fdr, int64_t Nf, int64_t Nr,
-                                                      int64_t ld, const double* __restrict__ part, int nchunk,
-                                                      double* __restrict__ colmean,
-                                                      double* __restrict__ colvar) {
-  const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (j >= Nr) return;
-  double s1 = 0.0, s2 = 0.0;
-  for (int c = 0; c < nchunk; ++c) {
-    s1 += part[(j * nchunk + c) * 2 + 0];
-    s2 += part[(j * nchunk + c) * 2 + 1];
+// per column: mean and corrected variance from the partial sums, added in the
+// order of the chunks.  One wavefront a column, whose 64 lanes load 64 chunks at once:
+// with one thread a column the loads are a serial chain (64 chunks: 10 us).
+__global__ __launch_bounds__(64) void colstats_final(const float* __restrict__ fdr, int64_t Nf, int64_t Nr,
+                                                     int64_t ld, const double* __restrict__ part, int nchunk,
+                                                     double* __restrict__ colmean, double* __restrict__ colvar) {
+  __shared__ double sh[128];
+  for (int64_t j = blockIdx.x; j < Nr; j += gridDim.x) {
+    double s1 = 0.0, s2 = 0.0;
+    for (int c0 = 0; c0 < nchunk; c0 += 64) {
+      const int nc = min(64, nchunk - c0);
+      const double* p = part + (j * nchunk + c0) * 2;
+      if (static_cast<int>(threadIdx.x) < 2 * nc) sh[threadIdx.x] = p[threadIdx.x];
+      if (static_cast<int>(threadIdx.x) + 64 < 2 * nc) sh[threadIdx.x + 64] = p[threadIdx.x + 64];
+      __syncthreads();
+#pragma unroll 8
+      for (int c = 0; c < nc; ++c) {
+        s1 += sh[2 * c + 0];
+        s2 += sh[2 * c + 1];
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      const double n = static_cast<double>(Nf);
+      const double shift = static_cast<double>(fdr[j * ld]);
+      colmean[j] = shift + s1 / n;
+      colvar[j] = Nf > 1 ? (s2 - s1 * s1 / n) / (n - 1.0) : 0.0 / 0.0;
+    }
   }
-  const double n = static_cast<double>(Nf);
-  const double shift = static_cast<double>(fdr[j * ld]);
-  colmean[j] = shift + s1 / n;
-  colvar[j] = Nf > 1 ? (s2 - s1 * s1 / n) / (n - 1.0) : 0.0 / 0.0;
 }
 
 int colstats_nchunk(int64_t Nf) { return static_cast<int>((Nf + STAT_ROWS - 1) / STAT_ROWS); }
+int64_t colstats_nreg(int64_t Nf) { return (Nf + FDR_TILE - 1) / FDR_TILE; }
 
 int launch_colstats2(const float* fdr, int64_t Nf, int64_t Nr, int64_t ld, double* part, double* colmean,
-                     double* colvar, hipStream_t st) {
+                     double* colvar, hipStream_t st, float* rmax) {
   const int nchunk = colstats_nchunk(Nf);
   dim3 grid(nchunk, static_cast<unsigned>(std::min<int64_t>(Nr, 65535)));
   const int vec = (ld % 4 == 0 && (reinterpret_cast<uintptr_t>(fdr) & 15) == 0) ? 1 : 0;
-  colstats_partial<<<grid, STAT_THREADS, 0, st>>>(fdr, Nf, Nr, ld, part, nchunk, vec);
+  if (rmax != nullptr)
+    colstats_partial<true><<<grid, STAT_THREADS, 0, st>>>(fdr, Nf, Nr, ld, part, nchunk, vec, rmax,
+                                                          colstats_nreg(Nf));
+  else
+    colstats_partial<false><<<grid, STAT_THREADS, 0, st>>>(fdr, Nf, Nr, ld, part, nchunk, vec, nullptr, 0);
   ZDT_CHECK_LAUNCH("colstats_partial");
-  colstats_final<<<static_cast<unsigned>((Nr + 255) / 256), 256, 0, st>>>(fdr, Nf, Nr, ld, part, nchunk,
-                                                                          colmean, colvar);
+  colstats_final<<<static_cast<unsigned>(std::min<int64_t>(Nr, 65535)), 64, 0, st>>>(fdr, Nf, Nr, ld, part, nchunk,
+                                                                                     colmean, colvar);
   ZDT_CHECK_LAUNCH("colstats_final");
   return ZDT_OK;
 }
@@ -255,6 +308,40 @@ __global__ __launch_bounds__(HIT_THREADS) void hits_count_sparse(const float* __
       if (static_cast<double>(fdr_unordered(tm[threadIdx.x])) < thr) counts[tile] = 0;
       else atomicOr(&need, 1u << threadIdx.x);
     }
+  }
+  __syncthreads();
+  for (unsigned mk = need; mk != 0u; mk &= mk - 1u) {  // uniform
+    const int64_t tl = t0 + (__ffs(mk) - 1);
+    const int c = count_tile(fdr, Nf, n, ld, thr, tl, vec, sh);
+    if (threadIdx.x == 0) counts[tl] = c;
+  }
+}
+
+// hits_count with colstats_partial's region maxima (rmax[j][q]: rows [q, q + 1) *
+// HIT_TILE of column j), Nf >= HIT_TILE: a tile lies in at most four consecutive
+// regions, and is read only if one of them reaches the threshold.  2^20 x 129: 90 us
+// for reading the matrix again -> 5 us.
+__global__ __launch_bounds__(HIT_THREADS) void hits_count_max(const float* __restrict__ fdr, int64_t Nf, int64_t n,
+                                                              int64_t ld, double thr_h, const double* thr_d,
+                                                              const float* __restrict__ rmax, int64_t nreg,
+                                                              int64_t ntiles, int64_t* __restrict__ counts, int vec) {
+  const double thr = thr_d ? *thr_d : thr_h;
+  __shared__ int sh[HIT_THREADS / 64];
+  __shared__ unsigned need;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * HIT_GROUP;
+  if (threadIdx.x < 64) {
+    const int64_t tile = t0 + threadIdx.x;
+    bool read = false;
+    if (threadIdx.x < HIT_GROUP && tile < ntiles) {
+      const int64_t g0 = tile * HIT_TILE, g1 = g0 + HIT_TILE <= n ? g0 + HIT_TILE - 1 : n - 1;
+      const int64_t j0 = g0 / Nf, j1 = g1 / Nf;
+      const int64_t q1 = j1 * nreg + (g1 - j1 * Nf) / HIT_TILE;
+      for (int64_t q = j0 * nreg + (g0 - j0 * Nf) / HIT_TILE; q <= q1; ++q)
+        read = read || static_cast<double>(rmax[q]) >= thr;
+      if (!read) counts[tile] = 0;
+    }
+    const unsigned long long b = __ballot(read);
+    if (threadIdx.x == 0) need = static_cast<unsigned>(b);
   }
   __syncthreads();
   for (unsigned mk = need; mk != 0u; mk &= mk - 1u) {  // uniform
@@ -430,7 +517,7 @@ __global__ __launch_bounds__(HIT_THREADS) void hits_write(const float* __restric
 }
 
 int launch_hits_count(const float* fdr, int64_t Nf, int64_t Nr, int64_t ld, double thr, const double* thr_dev,
-                      int64_t* counts, hipStream_t st, const float* smax, int smax_n2) {
+                      int64_t* counts, hipStream_t st, const float* smax, int smax_n2, const float* rmax) {
   const int64_t nt = hits_tiles(Nf, Nr);
   if (nt == 0) return ZDT_OK;
   const int vec = (ld == Nf && (reinterpret_cast<uintptr_t>(fdr) & 15) == 0) ? 1 : 0;
@@ -447,6 +534,14 @@ int launch_hits_count(const float* fdr, int64_t Nf, int64_t Nr, int64_t ld, doub
     hits_count_sparse<<<static_cast<unsigned>((nt + HIT_GROUP - 1) / HIT_GROUP), HIT_THREADS, 0, st>>>(
         fdr, Nf, Nf * Nr, ld, thr, thr_dev, smax, nt, counts, vec, smax_n2, static_cast<int>(2048 / N1));
     ZDT_CHECK_LAUNCH("hits_count_sparse");
+    return ZDT_OK;
+  }
+  if (rmax != nullptr && Nf >= HIT_TILE) {
+    const int64_t nreg = colstats_nreg(Nf);
+    ProfScope ps(st, "hits_count_max", 4.0 * nreg * Nr + 8.0 * nt);
+    hits_count_max<<<static_cast<unsigned>((nt + HIT_GROUP - 1) / HIT_GROUP), HIT_THREADS, 0, st>>>(
+        fdr, Nf, Nf * Nr, ld, thr, thr_dev, rmax, nreg, nt, counts, vec);
+    ZDT_CHECK_LAUNCH("hits_count_max");
     return ZDT_OK;
   }
   ProfScope ps(st, "hits_count", 4.0 * Nf * Nr + 8.0 * nt);
@@ -500,14 +595,19 @@ int launch_accumulate_i64(int64_t* acc, const int64_t* v, bool init, hipStream_t
 
 // fdrdenormalize on the device (src/fdrutils.jl:104-119 with :39-50):
 // thr = snr * s + m, s = sqrt(min_j colvar[j]) (NaN if any is NaN),
-// m = colmean[0]; one wavefront, the minimum taken lane-wise then across the
-// lanes (min is exact, so the order does not matter)
-__global__ __launch_bounds__(64) void hits_threshold(const double* __restrict__ colmean,
-                                                     const double* __restrict__ colvar, int64_t Nr, double snr,
-                                                     double* __restrict__ thr) {
+// m = colmean[0]; one block, the minimum taken thread-wise then across the
+// threads (min is exact, so the order does not matter).  Product and sum round
+// separately, as they do on the host.
+__global__ __launch_bounds__(256) void hits_threshold(const double* __restrict__ colmean,
+                                                      const double* __restrict__ colvar, int64_t Nr, double snr,
+                                                      double* __restrict__ thr) {
+#pragma clang fp contract(off)
+  __shared__ double shv[4];
+  __shared__ int shn[4];
   double vmin = INFINITY;
   int nan = 0;
-  for (int64_t j = threadIdx.x; j < Nr; j += 64) {
+#pragma unroll 4
+  for (int64_t j = threadIdx.x; j < Nr; j += 256) {
     const double v = colvar[j];
     if (v != v) nan = 1;
     vmin = fmin(vmin, v);
@@ -516,8 +616,14 @@ __global__ __launch_bounds__(64) void hits_threshold(const double* __restrict__ 
     vmin = fmin(vmin, __shfl_xor(vmin, off, 64));
     nan |= __shfl_xor(nan, off, 64);
   }
+  if ((threadIdx.x & 63) == 0) {
+    shv[threadIdx.x >> 6] = vmin;
+    shn[threadIdx.x >> 6] = nan;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const double sd = nan ? NAN : sqrt(fmax(vmin, 0.0));
+    vmin = fmin(fmin(shv[0], shv[1]), fmin(shv[2], shv[3]));
+    const double sd = (shn[0] | shn[1] | shn[2] | shn[3]) ? NAN : sqrt(fmax(vmin, 0.0));
     *thr = snr * sd + colmean[0];
   }
 }
@@ -535,7 +641,7 @@ int launch_set_double(double* p, double v, hipStream_t st) {
 int launch_hits_threshold(const double* colmean, const double* colvar, int64_t Nr, double snr, double* thr,
                           hipStream_t st) {
   ProfScope ps(st, "hits_threshold", 16.0 * Nr);
-  hits_threshold<<<1, 64, 0, st>>>(colmean, colvar, Nr, snr, thr);
+  hits_threshold<<<1, 256, 0, st>>>(colmean, colvar, Nr, snr, thr);
   ZDT_CHECK_LAUNCH("hits_threshold");
   return ZDT_OK;
 }

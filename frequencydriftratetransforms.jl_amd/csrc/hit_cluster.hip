@@ -436,9 +436,22 @@ struct SmallArgs {
   int64_t ld;
   Mats mats;
   int want;  // cap > 0 or labels asked for
+  // not null: results packed for one copy to the host (the Found layout); n is
+  // then *pack, read on the device, and more than nmax proto-hits are left alone
+  int64_t* pack;
+  int64_t nmax;
 };
 
 __global__ __launch_bounds__(CL_SMALL_THREADS) void cl_small(SmallArgs a) {
+  if (a.pack != nullptr) {
+    const int64_t np = a.pack[0];
+    if (np > a.nmax) {  // uniform
+      if (threadIdx.x == 0) a.pack[2] = 0;
+      return;
+    }
+    a.n = static_cast<int>(np);
+    a.label = a.pack + FOUND_HEAD + np;
+  }
   __shared__ int hv[CL_SMALL_MAX];   // the proto-hits, as int32 linear indices
   // the forest; after numbering, -(ordinal + 1) at the roots; at the end,
   // the hits' accumulators
@@ -476,6 +489,10 @@ __global__ __launch_bounds__(CL_SMALL_THREADS) void cl_small(SmallArgs a) {
       if (hv[k - 1] >= hv[k]) lds_st(&bad, 1);
   __syncthreads();
   if (bad) {  // uniform
+    if (a.pack != nullptr) {
+      if (tid == 0) a.pack[2] = 0;
+      return;
+    }
     for (int k = tid; k < n; k += CL_SMALL_THREADS) a.cid[k] = INT_MAX;
     if (tid == 0) {
       a.flags[0] = 0;
@@ -541,6 +558,18 @@ __global__ __launch_bounds__(CL_SMALL_THREADS) void cl_small(SmallArgs a) {
   // (24 bytes a hit) fit where the parents were; otherwise cl_accumulate and
   // cl_finish run them
   const bool fold = a.want && C <= CL_SMALL_ACC;
+  if (a.pack != nullptr) {
+    if (tid == 0) {
+      a.pack[1] = C;
+      a.pack[2] = fold ? 1 : 0;
+    }
+    if (!fold) return;  // uniform
+    for (int k = tid; k < n; k += CL_SMALL_THREADS) a.pack[FOUND_HEAD + k] = hv[k];
+    a.peak = a.label + n;
+    a.size = a.peak + C;
+    a.box = a.size + C;
+    a.value = reinterpret_cast<float*>(a.box + 4 * static_cast<int64_t>(C));
+  }
   int c = wsum[wv] + incl - s;
   for (int k = k0; k < k1; ++k) {
     if (par[k] != k) continue;
@@ -557,7 +586,7 @@ __global__ __launch_bounds__(CL_SMALL_THREADS) void cl_small(SmallArgs a) {
     par[k] = -(c + 1);  // read only after the barrier below
     ++c;
   }
-  if (tid == 0) {
+  if (tid == 0 && a.pack == nullptr) {
     a.flags[0] = C;
     a.flags[1] = 0;
     a.flags[2] = fold ? 1 : 0;
@@ -699,7 +728,7 @@ int cluster_protohits_impl(const int64_t* hits, int64_t n, const float* const* f
     if (small) {
       ProfScope ps(st, "cluster_small", 16.0 * n);
       SmallArgs sa{hits, static_cast<int>(n), Nf, ncol, di, dj, cid, flags_dev, cap, peak, value, size, box, label,
-                   static_cast<int>(Nr), ld, mats, cap > 0 || label != nullptr ? 1 : 0};
+                   static_cast<int>(Nr), ld, mats, cap > 0 || label != nullptr ? 1 : 0, nullptr, 0};
       cl_small<<<1, CL_SMALL_THREADS, 0, st>>>(sa);
       ZDT_CHECK_LAUNCH("cl_small");
     } else {
@@ -749,6 +778,34 @@ int cluster_protohits_impl(const int64_t* hits, int64_t n, const float* const* f
   *nclusters = flags[0];
   if (flags[0] > cap)
     return fail(ZDT_ETRUNC, "clusterprotohits: %lld hits exceed capacity %lld", (long long)flags[0], (long long)cap);
+  return ZDT_OK;
+}
+
+int64_t found_words() { return FOUND_HEAD + 2 * CL_SMALL_MAX + CL_SMALL_ACC * 6 + (CL_SMALL_ACC + 1) / 2; }
+
+bool found_fits(int nb, int64_t Nf, int64_t Nr) {
+  constexpr int64_t lim = int64_t(1) << 31;
+  return Nf < lim && Nr < lim && Nf * Nr < lim && Nf * Nr * nb < lim;
+}
+
+int launch_cluster_found(int64_t* pack, const int64_t* hits, int64_t cap, const float* const* tab, const float* one,
+                         int nb, int64_t Nf, int64_t Nr, int64_t ld, int di, int dj, hipStream_t st) {
+  SmallArgs sa{};
+  sa.hits = hits;
+  sa.Nf = Nf;
+  sa.ncol = nb * Nr;
+  sa.di = di;
+  sa.dj = dj;
+  sa.cap = CL_SMALL_MAX;
+  sa.Nr = static_cast<int>(Nr);
+  sa.ld = ld;
+  sa.mats = Mats{one, tab};
+  sa.want = 1;
+  sa.pack = pack;
+  sa.nmax = cap < CL_SMALL_MAX ? cap : CL_SMALL_MAX;
+  ProfScope ps(st, "cluster_small", 0.0);
+  cl_small<<<1, CL_SMALL_THREADS, 0, st>>>(sa);
+  ZDT_CHECK_LAUNCH("cl_small");
   return ZDT_OK;
 }
 

@@ -937,4 +937,107 @@ int zdt_clusterprotohits(const int64_t* hits, int64_t n, const float* const* fdr
                                 label, static_cast<hipStream_t>(stream));
 }
 
+namespace {
+// the scratch of zdt_findhits, in bytes from its start
+struct FindLayout {
+  int64_t pack, counts, tab, part, mean, var, rmax, bytes;
+  FindLayout(int nb, int64_t Nf, int64_t Nr, bool snr) {
+    auto up = [](int64_t b) { return (b + 255) & ~int64_t(255); };
+    const int64_t ntall = hits_tiles(Nf, Nr) * nb;
+    pack = 0;
+    counts = pack + up(8 * found_words());
+    tab = counts + up(8 * (ntall + hits_scan_scratch(ntall)));
+    part = tab + up(8 * static_cast<int64_t>(nb));
+    mean = part + (snr ? up(16 * static_cast<int64_t>(colstats_nchunk(Nf)) * Nr) : 0);
+    var = mean + (snr ? up(8 * nb * Nr) : 0);
+    rmax = var + (snr ? up(8 * nb * Nr) : 0);
+    bytes = rmax + (snr ? up(4 * nb * Nr * colstats_nreg(Nf)) : 0);
+  }
+};
+}  // namespace
+
+int zdt_findhits_scratch(int nb, int64_t Nf, int64_t Nr, int snr, int64_t* bytes, int64_t* words) {
+  if (nb < 1 || Nf < 1 || Nr < 1 || bytes == nullptr || words == nullptr)
+    return fail(ZDT_EINVAL, "findhits: bad shape or NULL");
+  if (!found_fits(nb, Nf, Nr))
+    return fail(ZDT_ENOTSUP, "findhits: 2^31 cells or more take findprotohits and clusterprotohits");
+  *bytes = FindLayout(nb, Nf, Nr, snr != 0).bytes;
+  *words = found_words();
+  return ZDT_OK;
+}
+
+// Whole call at 2^20 x 129 with 44 proto-hits: 509 us as fdrstats, findprotohits and
+// clusterprotohits (three synchronizations, each with memory allocated and given
+// back, six copies of results, two reads of the matrix) -> 193, of which 93 the read and 43
+// eight launches.
+int zdt_findhits(const float* const* fdrs, int nb, int64_t Nf, int64_t Nr, int64_t ld, double threshold, int snr,
+                 int di, int dj, void* scratch, int64_t scratch_bytes, int64_t* hits, int64_t cap, int64_t* found,
+                 int64_t* nproto, int64_t* nhits, double* thr, void* stream) {
+  ZDT_TRY(check_fdrs(reinterpret_cast<const void* const*>(fdrs), nb, Nf, Nr, ld));
+  if (cap < 0 || (cap > 0 && hits == nullptr)) return fail(ZDT_EINVAL, "findprotohits: bad output buffer");
+  if (!found_fits(nb, Nf, Nr))
+    return fail(ZDT_ENOTSUP, "findhits: 2^31 cells or more take findprotohits and clusterprotohits");
+  if (found != nullptr && (di < 0 || dj < 0))
+    return fail(ZDT_EINVAL, "clusterprotohits: negative neighbourhood (%d, %d)", di, dj);
+  const FindLayout lay(nb, Nf, Nr, snr != 0);
+  if (scratch == nullptr || (reinterpret_cast<uintptr_t>(scratch) & 15) != 0 || scratch_bytes < lay.bytes ||
+      nproto == nullptr || nhits == nullptr || thr == nullptr)
+    return fail(ZDT_EINVAL, "findhits: bad scratch or NULL result");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  char* base = static_cast<char*>(scratch);
+  int64_t* pack = reinterpret_cast<int64_t*>(base + lay.pack);
+  int64_t* counts = reinterpret_cast<int64_t*>(base + lay.counts);
+  // the threshold's word of the head, which hits_threshold writes and the copy brings back
+  double* thr_dev = snr ? reinterpret_cast<double*>(pack + 3) : nullptr;
+  float* rmax = snr && Nf >= FDR_TILE ? reinterpret_cast<float*>(base + lay.rmax) : nullptr;
+  const int64_t nreg = colstats_nreg(Nf);
+  if (snr) {
+    double* part = reinterpret_cast<double*>(base + lay.part);
+    double* mean = reinterpret_cast<double*>(base + lay.mean);
+    double* var = reinterpret_cast<double*>(base + lay.var);
+    for (int b = 0; b < nb; ++b)
+      ZDT_TRY(launch_colstats2(fdrs[b], Nf, Nr, ld, part, mean + b * Nr, var + b * Nr, st,
+                               rmax ? rmax + b * Nr * nreg : nullptr));
+    ZDT_TRY(launch_hits_threshold(mean, var, nb * Nr, threshold, thr_dev, st));
+  }
+  const int64_t nt = hits_tiles(Nf, Nr), ntall = nt * nb;
+  for (int b = 0; b < nb; ++b)
+    ZDT_TRY(launch_hits_count(fdrs[b], Nf, Nr, ld, threshold, thr_dev, counts + b * nt, st, nullptr, 0,
+                              rmax ? rmax + b * Nr * nreg : nullptr));
+  ZDT_TRY(launch_hits_scan(counts, ntall, pack, counts + ntall, st));
+  if (cap > 0)
+    for (int b = 0; b < nb; ++b)
+      ZDT_TRY(launch_hits_write_impl(fdrs[b], Nf, Nr, ld, threshold, thr_dev, counts, ntall, b * nt, pack,
+                                     static_cast<int64_t>(b) * Nf * Nr, hits, cap, st));
+  // the head, and with it what a few hits take
+  int64_t first = FOUND_HEAD;
+  int64_t head[FOUND_HEAD];
+  int64_t* host = head;
+  if (found != nullptr) {
+    const float* const* tab = nullptr;
+    if (nb > 1) {
+      tab = reinterpret_cast<const float* const*>(base + lay.tab);
+      ZDT_TRY_HIP(hipMemcpyAsync(base + lay.tab, fdrs, sizeof(float*) * nb, hipMemcpyHostToDevice, st));
+    }
+    ZDT_TRY(launch_cluster_found(pack, hits, cap, tab, fdrs[0], nb, Nf, Nr, ld, di, dj, st));
+    first = std::min<int64_t>(1024, found_words());
+    host = found;
+  }
+  ZDT_TRY_HIP(hipMemcpyAsync(host, pack, first * 8, hipMemcpyDeviceToHost, st));
+  ZDT_TRY_HIP(hipStreamSynchronize(st));
+  *nproto = host[0];
+  *nhits = found != nullptr && host[2] == 1 ? host[1] : -1;
+  *thr = threshold;
+  if (snr) std::memcpy(thr, &host[3], sizeof(double));
+  if (*nhits >= 0) {
+    const int64_t words = FOUND_HEAD + 2 * *nproto + 6 * *nhits + (*nhits + 1) / 2;
+    if (words > first)
+      ZDT_TRY_HIP(hipMemcpyAsync(found + first, pack + first, (words - first) * 8, hipMemcpyDeviceToHost, st));
+    if (words > first) ZDT_TRY_HIP(hipStreamSynchronize(st));
+  }
+  if (*nproto > cap)
+    return fail(ZDT_ETRUNC, "findprotohits: %lld hits exceed capacity %lld", (long long)*nproto, (long long)cap);
+  return ZDT_OK;
+}
+
 }  // extern "C"

@@ -49,9 +49,12 @@ int launch_step_postphase(c32* Y, int64_t ldY, int64_t Nk, int64_t Nf, int Nr, d
 // FDR statistics: per-column mean and corrected variance (FP64) of an
 // Nf x Nr matrix with column stride ld.  part needs 2*Nr*colstats_nchunk(Nf)
 // doubles of scratch; colmean/colvar receive Nr doubles each.
+// rmax: NULL, or Nr*colstats_nreg(Nf) floats that receive the largest value of each
+// FDR_TILE rows of a column.
 int colstats_nchunk(int64_t Nf);
+int64_t colstats_nreg(int64_t Nf);
 int launch_colstats2(const float* fdr, int64_t Nf, int64_t Nr, int64_t ld, double* part, double* colmean,
-                     double* colvar, hipStream_t st);
+                     double* colvar, hipStream_t st, float* rmax = nullptr);
 // x = (x - m)/s in place
 int launch_normalize(float* fdr, int64_t Nf, int64_t Nr, int64_t ld, double m, double s, hipStream_t st);
 // proto-hits: count per tile, exclusive scan, ordered write (see fdr_stats.hip)
@@ -59,9 +62,11 @@ int64_t hits_tiles(int64_t Nf, int64_t Nr);
 // thr_dev, when not NULL, holds the threshold on the device (thr is ignored)
 // smax: NULL, or the matrix's run maxima as the fused output writes them
 // (K3Args::smax, [Nr][N1/16][smax_n2] with N1 = Nf/(2 smax_n2); needs ld == Nf):
-// tiles whose runs are all under the threshold are not read
+// tiles whose runs are all under the threshold are not read.
+// rmax: the same with launch_colstats2's maxima, for any shape and ld
 int launch_hits_count(const float* fdr, int64_t Nf, int64_t Nr, int64_t ld, double thr, const double* thr_dev,
-                      int64_t* counts, hipStream_t st, const float* smax = nullptr, int smax_n2 = 0);
+                      int64_t* counts, hipStream_t st, const float* smax = nullptr, int smax_n2 = 0,
+                      const float* rmax = nullptr);
 // scratch: hits_scan_scratch(n) int64 words
 int64_t hits_scan_scratch(int64_t n);
 int launch_hits_scan(int64_t* counts, int64_t n, int64_t* total, int64_t* scratch, hipStream_t st);
@@ -89,5 +94,17 @@ int launch_hits_threshold(const double* colmean, const double* colvar, int64_t N
 int cluster_protohits_impl(const int64_t* hits, int64_t n, const float* const* fdrs, int nb, int64_t Nf,
                            int64_t Nr, int64_t ld, int di, int dj, int64_t* peak, float* value, int64_t* size,
                            int64_t* box, int64_t cap, int64_t* nclusters, int64_t* label, hipStream_t st);
+
+// The same for proto-hits whose count the host does not know yet: pack[0]
+// proto-hits at hits (cap entries).  When they and their clusters fit one
+// workgroup, pack receives, in int64 words, [1] the number of clusters C, [2] 1,
+// and from FOUND_HEAD on n proto-hits, n labels, C peaks, C sizes, 4 C box limits and
+// C float values; otherwise [2] = 0.  pack: found_words() words.  Only for shapes that
+// found_fits.
+constexpr int FOUND_HEAD = 8;
+int64_t found_words();
+bool found_fits(int nb, int64_t Nf, int64_t Nr);
+int launch_cluster_found(int64_t* pack, const int64_t* hits, int64_t cap, const float* const* tab, const float* one,
+                         int nb, int64_t Nf, int64_t Nr, int64_t ld, int di, int dj, hipStream_t st);
 
 }  // namespace zdt

@@ -94,6 +94,9 @@ SIGNATURES = {
     "zdt_bshuf_decompress": (C.c_int, [_vp, C.c_size_t, _vp, C.c_size_t, C.c_size_t, C.c_size_t, C.c_int]),
     "zdt_clusterprotohits": (C.c_int, [_vp, _i64, C.POINTER(_vp), C.c_int, _i64, _i64, _i64, C.c_int, C.c_int,
                                        _vp, _vp, _vp, _vp, _i64, _i64p, _vp, _vp]),
+    "zdt_findhits_scratch": (C.c_int, [C.c_int, _i64, _i64, C.c_int, _i64p, _i64p]),
+    "zdt_findhits": (C.c_int, [C.POINTER(_vp), C.c_int, _i64, _i64, _i64, C.c_double, C.c_int, C.c_int, C.c_int, _vp,
+                               _i64, _vp, _i64, _vp, _i64p, _i64p, C.POINTER(C.c_double), _vp]),
     "zdt_findprotohits_noalloc": (C.c_int, [C.POINTER(_vp), C.c_int, _i64, _i64, _i64, C.c_double, _vp, _i64,
                                             _i64p, _vp]),
     "zdt_plan_ragged": (C.c_int, [C.c_int, _i64p, _i64p, C.POINTER(C.c_float), C.POINTER(C.c_float), _i64p,

@@ -110,18 +110,60 @@ def _protohits_device(lst: List[torch.Tensor], threshold: float, capacity: int):
         return buf, int(n.value), Nf, Nr, ld, arr
 
 
+def _find_device(lst: List[torch.Tensor], threshold, snr: bool, capacity: int, di: int = 1, dj: int = 1,
+                 cluster: bool = False):
+    """The proto-hits in a device buffer and, when they are few and cluster is
+    set, (proto-hits, Hits) on the host: (buffer, count, Nf, Nr, ld, ptrs, found or None)."""
+    arr, Nf, Nr, ld = _ptrs(lst)
+    L = _lib.lib()
+    nbytes, words = C.c_int64(), C.c_int64()
+    if L.zdt_findhits_scratch(len(lst), Nf, Nr, 1 if snr else 0, C.byref(nbytes), C.byref(words)) != _lib.ZDT_OK:
+        # 2^31 cells or more (or a shape that the calls below refuse)
+        if snr:
+            threshold = fdrdenormalize(threshold, lst)
+        return (*_protohits_device(lst, threshold, capacity), None)
+    dev = lst[0].device
+    scratch = torch.empty(nbytes.value, dtype=torch.uint8, device=dev)
+    found = np.empty(words.value, dtype=np.int64) if cluster else None
+    n, nh, thr = C.c_int64(), C.c_int64(), C.c_double()
+    st = C.c_void_p(D.stream_ptr())
+    cap = int(capacity)
+    threshold = float(threshold)
+    while True:
+        buf = torch.empty(max(cap, 1), dtype=torch.int64, device=dev)
+        rc = L.zdt_findhits(arr, len(lst), Nf, Nr, ld, threshold, 1 if snr else 0, int(di), int(dj),
+                            scratch.data_ptr(), nbytes.value, buf.data_ptr(), cap,
+                            found.ctypes.data if cluster else None, C.byref(n), C.byref(nh), C.byref(thr), st)
+        if rc == _lib.ZDT_ETRUNC:
+            cap = int(n.value)
+            continue
+        _lib.check(rc)
+        break
+    p, h = int(n.value), int(nh.value)
+    out = None
+    if h >= 0:
+        lin, label, rest = found[8:8 + p], found[8 + p:8 + 2 * p], found[8 + 2 * p:]
+        out = (_cells(lin, Nf), Hits(peak=_cells(rest[:h], Nf), value=rest[6 * h:].view(np.float32)[:h].copy(),
+                                     size=rest[h:2 * h].copy(), box=rest[2 * h:6 * h].reshape(h, 4) + 1,
+                                     labels=label + 1))
+    return buf, p, Nf, Nr, ld, arr, out
+
+
+def _cells(lin: np.ndarray, Nf: int) -> np.ndarray:
+    """1-based (channel, column) pairs of 0-based linear indices."""
+    out = np.empty((len(lin), 2), dtype=np.int64)
+    np.divmod(lin, Nf, out=(out[:, 1], out[:, 0]))
+    out += 1
+    return out
+
+
 def findprotohits(fdrs: Fdrs, threshold, snr: bool = False, capacity: int = 1 << 20) -> np.ndarray:
     """Every element >= threshold as 1-based (channel, rate) pairs, column-major
     order over the hcat'd matrices (src/fdrutils.jl:148-169).  Returns an
     (H, 2) int64 array, the counterpart of Vector{CartesianIndex{2}}."""
     lst, _ = _as_list(fdrs)
-    if snr:
-        threshold = fdrdenormalize(threshold, lst)
-    buf, n, Nf, _, _, _ = _protohits_device(lst, threshold, capacity)
-    lin = buf[:n].cpu().numpy()
-    i = lin % Nf
-    j = lin // Nf
-    return np.stack([i + 1, j + 1], axis=1).astype(np.int64)
+    buf, n, Nf, *_ = _find_device(lst, threshold, snr, capacity)
+    return _cells(buf[:n].cpu().numpy(), Nf)
 
 
 class Hits(NamedTuple):
@@ -160,7 +202,7 @@ def _cluster_device(buf: torch.Tensor, n: int, arr, nb: int, Nf: int, Nr: int, l
     h = int(ncl.value)
     pk = peak[:h].cpu().numpy()
     bx = box[: 4 * h].cpu().numpy().reshape(h, 4)
-    return Hits(peak=np.stack([pk % Nf + 1, pk // Nf + 1], axis=1).astype(np.int64),
+    return Hits(peak=_cells(pk, Nf),
                 value=value[:h].cpu().numpy(), size=size[:h].cpu().numpy(), box=bx + 1,
                 labels=label[:n].cpu().numpy() + 1)
 
@@ -186,9 +228,8 @@ def findhits(fdrs: Fdrs, threshold, snr: bool = False, di: int = 1, dj: int = 1,
     """findprotohits followed by clusterprotohits, with the proto-hits kept
     on the device between the two.  Returns (proto-hits, hits)."""
     lst, _ = _as_list(fdrs)
-    if snr:
-        threshold = fdrdenormalize(threshold, lst)
-    buf, n, Nf, Nr, ld, arr = _protohits_device(lst, threshold, capacity)
+    buf, n, Nf, Nr, ld, arr, found = _find_device(lst, threshold, snr, capacity, di, dj, True)
+    if found is not None:
+        return found
     hits = _cluster_device(buf, n, arr, len(lst), Nf, Nr, ld, di, dj, 1 << 16)
-    lin = buf[:n].cpu().numpy()
-    return np.stack([lin % Nf + 1, lin // Nf + 1], axis=1).astype(np.int64), hits
+    return _cells(buf[:n].cpu().numpy(), Nf), hits

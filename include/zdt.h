@@ -280,6 +280,25 @@ int zdt_clusterprotohits(const int64_t* hits, int64_t n, const float* const* fdr
                          float* value, int64_t* size, int64_t* box, int64_t cap,
                          int64_t* nclusters, int64_t* label, void* stream);
 
+/* findprotohits(fdrs, threshold; snr) and the clustering of its proto-hits in one
+ * call with one synchronization, for the usual case of few of them.  No counterpart
+ * in the reference.  With snr != 0 the threshold is threshold*s + m (fdrstats and
+ * fdrdenormalize on the device), and the matrices are read once for the statistics
+ * and the search.  Results:
+ *   hits (device, cap entries), *nproto: as zdt_findprotohits (ZDT_ETRUNC likewise);
+ *   *thr: the threshold applied;
+ *   found (host, or NULL for no clustering): when *nhits >= 0, from word 8 on
+ *     the *nproto proto-hits, their labels, then of the *nhits hits peak, size, box
+ *     (4 words) and value (float), as zdt_clusterprotohits describes them.
+ * *nhits = -1: not clustered (more than 16384 proto-hits or 2730 hits, or found is
+ * NULL); zdt_clusterprotohits does it.  scratch (device, 16-byte aligned) and found
+ * take the bytes and words that zdt_findhits_scratch gives.  ZDT_ENOTSUP when nb*Nf*Nr
+ * reaches 2^31. */
+int zdt_findhits_scratch(int nb, int64_t Nf, int64_t Nr, int snr, int64_t* bytes, int64_t* words);
+int zdt_findhits(const float* const* fdrs, int nb, int64_t Nf, int64_t Nr, int64_t ld, double threshold, int snr,
+                 int di, int dj, void* scratch, int64_t scratch_bytes, int64_t* hits, int64_t cap, int64_t* found,
+                 int64_t* nproto, int64_t* nhits, double* thr, void* stream);
+
 /* --------------------------------------------------------- ragged plans
  * Many coarse channels of uneven Nf and Nt, every one through input!, one
  * zdtfdr! batch, fdrdenormalize and findprotohits, replayed as ONE hipGraph
