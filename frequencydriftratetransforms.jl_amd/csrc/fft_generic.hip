@@ -152,24 +152,29 @@ static int pow2_floor(int64_t x) {
 // A pass reads its twiddles W_{Ns R}^{r k} from a table of its own in LDS
 // (contiguous or broadcast reads, no products); the radices (up to 16, the
 // composite ones 6, 9, 10, 12, 14, 15 among them) are chosen for the fewest
-// passes.  The four-step and c2r twiddles of a thread's 16 elements are
-// products of four starts and four steps evaluated from exact phases.  The
+// passes.  The four-step and c2r twiddles are products of two factors evaluated
+// from exact phases, the start of a thread and the step to its i-th element.  The
 // inverse is conj(forward(conj(x))), conjugated on the first load and the last
 // store, where the real transforms' packing happens too (fs_mode).
 //
-// Bound: HBM traffic overlapped badly with the passes' LDS latency (two blocks a
-// CU; loads, passes and stores of one block are serial).  Against prime radices
-// up to 13 and 16 with one twiddle table of the whole length in global memory
+// Bound: loads, passes and stores of a block follow one another, and two blocks a
+// CU (LDS) overlap them only partly; fs_rows runs its vector units 50% of the time,
+// the c2r columns 65%.  Against prime radices up to 13 and 16, one twiddle table of
+// the whole length in global memory and 512 threads a block with 16 elements each
 // (us): Nf = 10^6, 129 rates (1.03 GB through fs_cols, as much through fs_rows)
-// c2r columns 412 -> 318, rows 370 -> 295; r2c columns 59 -> 44.  Odd Nf = 99225, 77
-// rates, two columns a transform instead of a zero imaginary part: 84 + 68 + 40
-// for filling in the Hermitian half and taking the real part -> 56 + 44.  Nf =
-// 4096, 33 rates: six launches of 5 to 6 -> two of 5 (fs_one).  Persistent blocks
-// that load the next rows before the passes spill (128 VGPRs): 295 -> 569.
+// c2r columns 403 -> 305, rows 374 -> 278; r2c columns 59 -> 40.  Odd Nf = 99225, 77
+// rates, two columns a transform instead of a zero imaginary part: 86 + 70 + 40
+// for filling in the Hermitian half and taking the real part -> 44 + 43.  Nf =
+// 4096, 33 rates: six launches of 5 to 6 -> two, 17 together (fs_one).  Of that, 8
+// elements a thread and 1024 threads: c2r columns 318 -> 305; 32-bit offsets and
+// wave-uniform strides in place of an index per access (112 -> 76 vector
+// instructions an element in fs_rows): rows 295 -> 278.  Persistent blocks that load the
+// next rows before the passes spill (128 VGPRs, 16 elements): 295 -> 569.  Chunks
+// whose intermediate stays in the last-level cache: 0.93 to 1.0 of the speed.
 
-constexpr int FS_T = 512;    // threads per block
-constexpr int FS_E = 8192;   // elements per block of fs_cols / fs_rows (TC * N1 or TR * N2)
-constexpr int FS_ONE = 4096; // elements per block of fs_one
+constexpr int FS_PER = 8;    // elements a thread
+constexpr int FS_E = 8192;   // most elements per block of fs_cols / fs_rows (TC * N1 or TR * N2)
+constexpr int FS_ONE = 4096; // most elements per block of fs_one
 constexpr int FS_MAXP = 12;  // passes per sub-transform
 
 enum fs_mode {
@@ -187,6 +192,7 @@ struct FsArgs {
   int64_t obs;  // (floats for FS_ODD_C2R)
   const c32* tw;
   int ntw;
+  c32 half[FS_PER];  // FS_C2R of fs_cols: W_{2 N1}^{i TH / TC}
   int N, N1, N2, T;  // T = TC (fs_cols), TR (fs_rows) or transforms per block (fs_one)
   int np;            // passes of the sub-transform
   int rad[FS_MAXP];
@@ -211,18 +217,32 @@ __device__ __forceinline__ int fs_quo(int u, FsDiv q) {
   return q.m == 0 ? u : static_cast<int>(__umulhi(static_cast<uint32_t>(u), q.m));
 }
 
+// element at a 32-bit byte offset: with a wave-uniform base the offset goes into
+// the instruction as it is
+template <typename T>
+__device__ __forceinline__ T& at_byte(T* base, uint32_t off) {
+  return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + off);
+}
+template <typename T>
+__device__ __forceinline__ const T& at_byte(const T* base, uint32_t off) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
+}
+
 // One Stockham pass of radix R over T interleaved transforms of length L
 // held in buf (element n of transform c at n * T + c, T a power of two, L * T <=
-// E).  Butterfly u covers transform c = u mod T and index j = u / T < L/R.  Every
+// FS_PER TH).  Butterfly u covers transform c = u mod T and index j = u / T < L/R.  Every
 // index is below 2^13, so j mod Ns is an exact high multiply.  tw: the pass's
-// twiddles W_{Ns R}^{r k} at (r - 1) Ns + k (none for Ns = 1).
-template <int R, int E>
+// twiddles W_{Ns R}^{r k} at (r - 1) Ns + k (none in the FIRST pass, Ns = 1).
+// Addresses are one start a butterfly plus wave-uniform multiples.
+template <int R, int TH, bool FIRST>
 __device__ __forceinline__ void fs_pass(c32* buf, const c32* tw, int L, int T, int Ns) {
-  constexpr int NB = (E / R + FS_T - 1) / FS_T;
+  constexpr int NB = (FS_PER + R - 1) / R;
   const int Lr = L / R;
   const int nbf = Lr * T;
   const int lgT = __ffs(T) - 1;
   const FsDiv dNs = fs_div(Ns);
+  const uint32_t is = 8u * static_cast<uint32_t>(nbf), os = 8u * static_cast<uint32_t>(Ns * T),
+                 ws = 8u * static_cast<uint32_t>(Ns);
   // opaque to the optimizer, so that no index below is hoisted out of the
   // pass loop (which would keep every pass's indices live and spill)
   int tid = static_cast<int>(threadIdx.x);
@@ -230,15 +250,17 @@ __device__ __forceinline__ void fs_pass(c32* buf, const c32* tw, int L, int T, i
   c32 v[NB][R];
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    const int u = tid + i * FS_T;
+    const int u = tid + i * TH;
     if (u < nbf) {
-      const int c = u & (T - 1), j = u >> lgT;
+      const uint32_t ib = 8u * static_cast<uint32_t>(u);
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[i][r] = buf[(j + r * Lr) * T + c];
-      if (Ns > 1) {  // uniform
-        const int k = j - fs_quo(j, dNs) * Ns;
+      for (int r = 0; r < R; ++r) v[i][r] = at_byte(buf, ib + static_cast<uint32_t>(r) * is);
+      if (!FIRST) {
+        const int j = u >> lgT;
+        const uint32_t kb = 8u * static_cast<uint32_t>(j - fs_quo(j, dNs) * Ns);
 #pragma unroll
-        for (int r = 1; r < R; ++r) v[i][r] = cmul(v[i][r], tw[(r - 1) * Ns + k]);
+        for (int r = 1; r < R; ++r)
+          v[i][r] = cmul(v[i][r], at_byte(tw, kb + static_cast<uint32_t>(r - 1) * ws));
       }
       dft<float, R>(v[i]);
     }
@@ -246,67 +268,57 @@ __device__ __forceinline__ void fs_pass(c32* buf, const c32* tw, int L, int T, i
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NB; ++i) {
-    const int u = tid + i * FS_T;
+    const int u = tid + i * TH;
     if (u < nbf) {
-      const int c = u & (T - 1), j = u >> lgT;
-      const int k = j - fs_quo(j, dNs) * Ns;
-      const int ob = ((j - k) * R + k) * T + c;
+      const int j = u >> lgT;
+      const int q = FIRST ? j : fs_quo(j, dNs) * Ns;
+      const uint32_t ob = 8u * static_cast<uint32_t>(u + ((q * (R - 1)) << lgT));
 #pragma unroll
-      for (int r = 0; r < R; ++r) buf[ob + r * Ns * T] = v[i][r];
+      for (int r = 0; r < R; ++r) at_byte(buf, ob + static_cast<uint32_t>(r) * os) = v[i][r];
     }
   }
   __syncthreads();
 }
 
-// all passes of the T interleaved sub-transforms of length L (natural order in
-// and out)
-template <int E>
-__device__ __forceinline__ void fs_dft(c32* buf, const c32* tw, const FsArgs& a, int L) {
-  int Ns = 1;
-  for (int p = 0; p < a.np; ++p) {
-    const int R = a.rad[p];
-    switch (R) {
-#define ZDT_FS_CASE(RR)                           \
-  case RR:                                        \
-    fs_pass<RR, E>(buf, tw, L, a.T, Ns);          \
+template <int TH, bool FIRST>
+__device__ __forceinline__ void fs_pass_any(c32* buf, const c32* tw, int L, int T, int Ns, int R) {
+  switch (R) {
+#define ZDT_FS_CASE(RR)                        \
+  case RR:                                     \
+    fs_pass<RR, TH, FIRST>(buf, tw, L, T, Ns);     \
     break;
-      ZDT_FS_CASE(2)
-      ZDT_FS_CASE(3)
-      ZDT_FS_CASE(4)
-      ZDT_FS_CASE(5)
-      ZDT_FS_CASE(6)
-      ZDT_FS_CASE(7)
-      ZDT_FS_CASE(8)
-      ZDT_FS_CASE(9)
-      ZDT_FS_CASE(10)
-      ZDT_FS_CASE(11)
-      ZDT_FS_CASE(12)
-      ZDT_FS_CASE(13)
-      ZDT_FS_CASE(14)
-      ZDT_FS_CASE(15)
-      ZDT_FS_CASE(16)
+    ZDT_FS_CASE(2)
+    ZDT_FS_CASE(3)
+    ZDT_FS_CASE(4)
+    ZDT_FS_CASE(5)
+    ZDT_FS_CASE(6)
+    ZDT_FS_CASE(7)
+    ZDT_FS_CASE(8)
+    ZDT_FS_CASE(9)
+    ZDT_FS_CASE(10)
+    ZDT_FS_CASE(11)
+    ZDT_FS_CASE(12)
+    ZDT_FS_CASE(13)
+    ZDT_FS_CASE(14)
+    ZDT_FS_CASE(15)
+    ZDT_FS_CASE(16)
 #undef ZDT_FS_CASE
-    }
-    if (Ns > 1) tw += (R - 1) * Ns;
-    Ns *= R;
   }
 }
 
-// W^{n0 + i dn}, i < 16, W = e^{-2 pi i h}: four starts times four steps
-struct FsProg {
-  c32 a[4], b[4];
-  __device__ __forceinline__ FsProg(int n0, int dn, double h) {
-    const c32 s1 = cis_nh(-static_cast<double>(dn), h);
-    a[0] = cis_nh(-static_cast<double>(n0), h);
-    a[1] = cmul(a[0], s1);
-    a[2] = cmul(a[0], cmul(s1, s1));
-    a[3] = cmul(a[2], s1);
-    b[1] = cis_nh(-4.0 * static_cast<double>(dn), h);
-    b[2] = cmul(b[1], b[1]);
-    b[3] = cmul(b[2], b[1]);
+// all passes of the T interleaved sub-transforms of length L (natural order in
+// and out)
+template <int TH>
+__device__ __forceinline__ void fs_dft(c32* buf, const c32* tw, const FsArgs& a, int L) {
+  int Ns = a.rad[0];
+  fs_pass_any<TH, true>(buf, tw, L, a.T, 1, Ns);
+  for (int p = 1; p < a.np; ++p) {
+    const int R = a.rad[p];
+    fs_pass_any<TH, false>(buf, tw, L, a.T, Ns, R);
+    tw += (R - 1) * Ns;
+    Ns *= R;
   }
-  __device__ __forceinline__ c32 operator()(int i) const { return i < 4 ? a[i] : cmul(a[i & 3], b[i >> 2]); }
-};
+}
 
 // the packed sequence of the c2r transform: Z[k] = E + i O with
 // E = (p + conj q)/2, O = W_{2N}^{-k} (p - conj q)/2, p = X[k], q = X[N-k], w = W_{2N}^k;
@@ -365,11 +377,17 @@ __device__ __forceinline__ int64_t xcd_block(int64_t n) {
   return (blockIdx.x >> 3) < per && u < n ? u : -1;
 }
 
-// columns: block = (batch b, columns n2 in [c0, c0 + TC)); TC is a power of two
-__global__ __launch_bounds__(FS_T, 4) void fs_cols(FsArgs a) {
-  __shared__ c32 buf[FS_E];
-  __shared__ c32 tw[1024];
-  for (int i = threadIdx.x; i < a.ntw; i += FS_T) tw[i] = a.tw[i];
+// columns: block = (batch b, columns n2 in [c0, c0 + TC)); TC is a power of two.
+// Thread: column c of the block, rows n0 + i dn; a transform's elements are within
+// 2^23 bytes, so one base and 32-bit offsets reach them.  Loads past the edges
+// take the last row or column and are not stored.
+template <int TH>
+__global__ __launch_bounds__(TH, 8) void fs_cols(FsArgs a) {
+  extern __shared__ __align__(16) c32 lds[];  // FS_PER TH elements, the steps, the passes' twiddles
+  c32* buf = lds;
+  // W_N^{n2 dr i}: with W_N^{n2 n0} of its own, a thread's four-step twiddles
+  c32* step = lds + FS_PER * TH;
+  c32* tw = step + 16 * FS_PER;
   const int TC = a.T;
   const int lgT = __ffs(TC) - 1;
   const int tiles = (a.N2 + TC - 1) / TC;
@@ -377,116 +395,130 @@ __global__ __launch_bounds__(FS_T, 4) void fs_cols(FsArgs a) {
   if (blk < 0) return;
   const int64_t b = blk / tiles;
   const int c0 = static_cast<int>(blk % tiles) * TC;
-  const int E = a.N1 * TC;
-  // element i of a thread: column c of the block, row n0 + i dn
   const int c = static_cast<int>(threadIdx.x) & (TC - 1), r0 = static_cast<int>(threadIdx.x) >> lgT;
-  const int dr = FS_T >> lgT;
-  const bool in = c0 + c < a.N2;
-  constexpr int PER = FS_E / FS_T;
+  const int dr = TH >> lgT;
+  const int col = min(c0 + c, a.N2 - 1);
   // all loads issued before the first LDS store
-  c32 v[PER];
+  c32 v[FS_PER];
   if (a.mode == FS_C2R) {
     const c32* X = a.in + b * a.ibs;
-    c32 w[PER];
+    const c32* Xe = X + a.N;
+    c32 w[FS_PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      v[i] = w[i] = {0.0f, 0.0f};
-      if (in && r0 + i * dr < a.N1) {
-        const int k = c0 + c + (r0 + i * dr) * a.N2;
-        v[i] = X[k];
-        w[i] = X[a.N - k];  // X[N] for k = 0
+    for (int i = 0; i < FS_PER; ++i) {
+      if (i * dr < a.N1) {  // uniform
+        const uint32_t k = 8u * static_cast<uint32_t>(col + min(r0 + i * dr, a.N1 - 1) * a.N2);
+        v[i] = at_byte(X, k);
+        w[i] = at_byte(X, 8u * static_cast<uint32_t>(a.N) - k);  // X[N] for k = 0
       }
     }
-    const FsProg tp(c0 + c + r0 * a.N2, dr * a.N2, 0.5 * a.h);
+    const c32 w0 = cis_nh(-static_cast<double>(c0 + c + r0 * a.N2), 0.5 * a.h);
 #pragma unroll
-    for (int i = 0; i < PER; ++i) v[i] = c2r_pack(c0 + c + (r0 + i * dr) * a.N2, v[i], w[i], tp(i));
+    for (int i = 0; i < FS_PER; ++i)
+      if (i * dr < a.N1) v[i] = c2r_pack(c0 + c + r0 + i, v[i], w[i], cmul(w0, a.half[i]));
+  } else if (a.mode == FS_C2C) {
+    const c32* x = a.in + b * a.ibs;
+#pragma unroll
+    for (int i = 0; i < FS_PER; ++i)
+      if (i * dr < a.N1)
+        v[i] = at_byte(x, 8u * static_cast<uint32_t>(col + min(r0 + i * dr, a.N1 - 1) * a.N2));
   } else {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      v[i] = {0.0f, 0.0f};
-      if (in && r0 + i * dr < a.N1) v[i] = fs_input(a, b, c0 + c + (r0 + i * dr) * a.N2);
-    }
+    for (int i = 0; i < FS_PER; ++i)
+      if (i * dr < a.N1) v[i] = fs_input(a, b, col + min(r0 + i * dr, a.N1 - 1) * a.N2);
   }
+  for (int i = threadIdx.x; i < a.ntw; i += TH) tw[i] = a.tw[i];
+  if (static_cast<int>(threadIdx.x) < TC * FS_PER)
+    step[threadIdx.x] = cis_nh(-static_cast<double>((c0 + c) * dr) * static_cast<double>(r0), a.h);
+  const float sg = a.inverse ? -1.0f : 1.0f;
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-    if (e < E) buf[e] = {v[i].x, a.inverse ? -v[i].y : v[i].y};  // element n of column c at n * TC + c
-  }
+  for (int i = 0; i < FS_PER; ++i)  // element n of column c at n * TC + c; rows past N1 land behind the last one
+    if (i * dr < a.N1) buf[static_cast<int>(threadIdx.x) + i * TH] = {v[i].x, sg * v[i].y};
   __syncthreads();
-  fs_dft<FS_E>(buf, tw, a, a.N1);
-  if (!in) return;
-  c32* dst = a.out + b * static_cast<int64_t>(a.N) + c0 + c;
+  fs_dft<TH>(buf, tw, a, a.N1);
+  if (c0 + c >= a.N2) return;
+  c32* dst = a.out + b * a.N + c0;
   int k0 = r0;
   asm volatile("" : "+v"(k0));  // keeps the store indices from being computed before the passes
-  const FsProg tp((c0 + c) * k0, (c0 + c) * dr, a.h);
+  const c32 w0 = cis_nh(-static_cast<double>((c0 + c) * k0), a.h);
+  const uint32_t o0 = 8u * static_cast<uint32_t>(c + k0 * a.N2), od = 8u * static_cast<uint32_t>(dr * a.N2);
+  const uint32_t l0 = 8u * static_cast<uint32_t>(k0 * TC + c);
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int k1 = k0 + i * dr;
-    if (k1 < a.N1) dst[static_cast<int64_t>(k1) * a.N2] = cmul(buf[k1 * TC + c], tp(i));
-  }
+  for (int i = 0; i < FS_PER; ++i)
+    if (k0 + i * dr < a.N1)
+      at_byte(dst, o0 + static_cast<uint32_t>(i) * od) = cmul(at_byte(buf, l0 + 8u * TH * i), cmul(w0, step[i * TC + c]));
 }
 
-// rows: block = (batch b, rows k1 in [r0, r0 + TR)); TR is a power of two
-__global__ __launch_bounds__(FS_T, 4) void fs_rows(FsArgs a) {
-  __shared__ c32 buf[FS_E];
-  __shared__ c32 tw[2048];
-  for (int i = threadIdx.x; i < a.ntw; i += FS_T) tw[i] = a.tw[i];
+// rows: block = (batch b, rows k1 in [r0, r0 + TR)); TR is a power of two.  Rows are
+// interleaved as in fs_cols (element n of row c at n * TR + c), which keeps the
+// passes' LDS accesses as conflict-free as fs_cols's.
+template <int TH>
+__global__ __launch_bounds__(TH, 8) void fs_rows(FsArgs a) {
+  extern __shared__ __align__(16) c32 lds[];  // FS_PER TH elements, the passes' twiddles
+  c32* buf = lds;
+  c32* tw = lds + FS_PER * TH;
+  for (int i = threadIdx.x; i < a.ntw; i += TH) tw[i] = a.tw[i];
   const int TR = a.T;
+  const int lgT = __ffs(TR) - 1;
   const int tiles = (a.N1 + TR - 1) / TR;
   const int64_t blk = xcd_block(tiles * a.batch);
   if (blk < 0) return;
   const int64_t b = blk / tiles;
   const int r0 = static_cast<int>(blk % tiles) * TR;
-  const int nrow = min(TR, a.N1 - r0);
-  const c32* src = a.in + b * static_cast<int64_t>(a.N) + static_cast<int64_t>(r0) * a.N2;
-  const int E = a.N2 * TR;
-  const int lgT = __ffs(TR) - 1;
+  const int c = static_cast<int>(threadIdx.x) & (TR - 1), n0 = static_cast<int>(threadIdx.x) >> lgT;
+  const int dn = TH >> lgT;
   {
-    // rows interleaved as in fs_cols (element n of row c at n * TR + c), which
-    // keeps the passes' LDS accesses as conflict-free as fs_cols's
-    c32 v[FS_E / FS_T];
+    const c32* src = a.in + b * a.N;
+    const int row = min(r0 + c, a.N1 - 1) * a.N2;
+    c32 v[FS_PER];
 #pragma unroll
-    for (int i = 0; i < FS_E / FS_T; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-      const int c = e & (TR - 1), n = e >> lgT;
-      v[i] = {0.0f, 0.0f};
-      if (e < E && c < nrow) v[i] = src[static_cast<int64_t>(c) * a.N2 + n];
-    }
+    for (int i = 0; i < FS_PER; ++i)
+      if (i * dn < a.N2) v[i] = at_byte(src, 8u * static_cast<uint32_t>(row + min(n0 + i * dn, a.N2 - 1)));
 #pragma unroll
-    for (int i = 0; i < FS_E / FS_T; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
-      if (e < E) buf[e] = v[i];
-    }
+    for (int i = 0; i < FS_PER; ++i)
+      if (i * dn < a.N2) buf[static_cast<int>(threadIdx.x) + i * TH] = v[i];
   }
   __syncthreads();
-  fs_dft<FS_E>(buf, tw, a, a.N2);
-  int tid = static_cast<int>(threadIdx.x);
-  asm volatile("" : "+v"(tid));  // keeps the store indices from being computed before the passes
+  fs_dft<TH>(buf, tw, a, a.N2);
+  if (r0 + c >= a.N1) return;
+  int k2 = n0;
+  asm volatile("" : "+v"(k2));  // keeps the store indices from being computed before the passes
+  const uint32_t l0 = 8u * static_cast<uint32_t>(k2 * TR + c);
+  if (a.mode == FS_C2C || a.mode == FS_C2R) {
+    const float sx = a.scale, sy = a.inverse ? -a.scale : a.scale;
+    c32* dst = a.out + b * a.obs + r0;
+    const uint32_t o0 = 8u * static_cast<uint32_t>(c + k2 * a.N1), od = 8u * static_cast<uint32_t>(dn * a.N1);
 #pragma unroll
-  for (int i = 0; i < FS_E / FS_T; ++i) {
-    const int e = tid + i * FS_T;
-    const int c = e & (TR - 1), k2 = e >> lgT;
-    if (e < E && c < nrow) fs_output(a, b, r0 + c + k2 * a.N1, buf[e]);
+    for (int i = 0; i < FS_PER; ++i)
+      if (k2 + i * dn < a.N2) {
+        const c32 z = at_byte(buf, l0 + 8u * TH * i);
+        at_byte(dst, o0 + static_cast<uint32_t>(i) * od) = {z.x * sx, z.y * sy};
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < FS_PER; ++i)
+      if (k2 + i * dn < a.N2)
+        fs_output(a, b, r0 + c + (k2 + i * dn) * a.N1, at_byte(buf, l0 + 8u * TH * i));
   }
 }
 
 // whole transforms: block = transforms [T blockIdx, T blockIdx + T), element n of
 // transform c at n * T + c; LDS: N * T elements, then the twiddles
-__global__ __launch_bounds__(FS_T, 4) void fs_one(FsArgs a) {
-  extern __shared__ c32 lds[];
+template <int TH>
+__global__ __launch_bounds__(TH, TH == 512 ? 4 : 8) void fs_one(FsArgs a) {
+  extern __shared__ __align__(16) c32 lds[];
   c32* buf = lds;
   c32* tw = lds + a.N * a.T;
-  for (int i = threadIdx.x; i < a.ntw; i += FS_T) tw[i] = a.tw[i];
+  for (int i = threadIdx.x; i < a.ntw; i += TH) tw[i] = a.tw[i];
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * a.T;
   const int nt = static_cast<int>(min(static_cast<int64_t>(a.T), a.batch - b0));
   const int E = a.N * nt;
   const FsDiv dN = fs_div(a.N);
-  constexpr int PER = FS_ONE / FS_T;
   {
-    c32 v[PER], w[PER];
+    c32 v[FS_PER], w[FS_PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
+    for (int i = 0; i < FS_PER; ++i) {
+      const int e = static_cast<int>(threadIdx.x) + i * TH;
       const int c = fs_quo(e, dN), n = e - c * a.N;
       v[i] = w[i] = {0.0f, 0.0f};
       if (e < E) {
@@ -500,8 +532,8 @@ __global__ __launch_bounds__(FS_T, 4) void fs_one(FsArgs a) {
       }
     }
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * FS_T;
+    for (int i = 0; i < FS_PER; ++i) {
+      const int e = static_cast<int>(threadIdx.x) + i * TH;
       const int c = fs_quo(e, dN), n = e - c * a.N;
       if (e < E) {
         if (a.mode == FS_C2R) v[i] = c2r_pack(n, v[i], w[i], cis_nh(-static_cast<double>(n), 0.5 * a.h));
@@ -510,7 +542,7 @@ __global__ __launch_bounds__(FS_T, 4) void fs_one(FsArgs a) {
     }
   }
   __syncthreads();
-  fs_dft<FS_ONE>(buf, tw, a, a.N);
+  fs_dft<TH>(buf, tw, a, a.N);
   int tid = static_cast<int>(threadIdx.x);
   asm volatile("" : "+v"(tid));
   if (a.mode == FS_R2C) {
@@ -518,7 +550,7 @@ __global__ __launch_bounds__(FS_T, 4) void fs_one(FsArgs a) {
     // O = (Z[k] - conj Z[N-k])/(2i)
     const int half = a.N / 2 + 1;
     const FsDiv dH = fs_div(half);
-    for (int e = tid; e < half * nt; e += FS_T) {
+    for (int e = tid; e < half * nt; e += TH) {
       const int c = fs_quo(e, dH), k = e - c * half;
       c32* x = a.out + (b0 + c) * a.obs;
       const c32 z = buf[k * a.T + c];
@@ -537,8 +569,8 @@ __global__ __launch_bounds__(FS_T, 4) void fs_one(FsArgs a) {
     return;
   }
 #pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int e = tid + i * FS_T;
+  for (int i = 0; i < FS_PER; ++i) {
+    const int e = tid + i * TH;
     const int c = fs_quo(e, dN), k = e - c * a.N;
     if (e < E) fs_output(a, b0 + c, k, buf[k * a.T + c]);
   }
@@ -586,7 +618,7 @@ static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void*
     fs_passes(&a, p->rad0, p->tw0);
     const size_t lds = (static_cast<size_t>(p->N) * T + a.ntw) * sizeof(c32);
     ProfScope ps(st, "fft_fs_one", bytes);
-    fs_one<<<static_cast<unsigned>((batch + T - 1) / T), FS_T, lds, st>>>(a);
+    fs_one<512><<<static_cast<unsigned>((batch + T - 1) / T), 512, lds, st>>>(a);
     ZDT_CHECK_LAUNCH("fs_one");
     return ZDT_OK;
   }
@@ -598,10 +630,23 @@ static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void*
     a.mode = mode;
     a.T = p->TC;
     a.scale = 1.0f;
-    fs_passes(&a, p->rad1, p->tw1);
     const int64_t grid = ((p->N2 + p->TC - 1) / p->TC * batch + 7) / 8 * 8;
+    const int E = p->N1 * p->TC;
+    // Threads for 8 elements each: the fewest that cover the block keep its passes'
+    // wavefronts full and fit more blocks a CU; a grid of one round is better off
+    // with more of them.  Columns of 147 x 16 (21609 x 234, 205 rates): 1024 threads
+    // 125 us, 512 73, 320 58; of 125 x 16 in 200 blocks: 320 20, 512 16; of 576 x 8
+    // (1179648, 100 rates), where wavefronts a CU matter more: 640 366, 1024 305.
+    const int th = E > 512 * FS_PER ? 1024 : E > 320 * FS_PER || grid < 512 ? 512 : 320;
+    for (int i = 0; i < FS_PER; ++i) {
+      const double x = 3.14159265358979323846 * i * (th / p->TC) / p->N1;
+      a.half[i] = {static_cast<float>(std::cos(x)), static_cast<float>(-std::sin(x))};
+    }
+    fs_passes(&a, p->rad1, p->tw1);
     ProfScope ps(st, mode == FS_C2R ? "fft_fs_cols_c2r" : "fft_fs_cols", bytes);
-    fs_cols<<<static_cast<unsigned>(grid), FS_T, 0, st>>>(a);
+    const size_t lds = (FS_PER * th + 16 * FS_PER + a.ntw) * sizeof(c32);
+    const auto kern = th == 320 ? fs_cols<320> : th == 512 ? fs_cols<512> : fs_cols<1024>;
+    kern<<<static_cast<unsigned>(grid), th, lds, st>>>(a);
     ZDT_CHECK_LAUNCH("fs_cols");
   }
   {
@@ -614,7 +659,10 @@ static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void*
     fs_passes(&a, p->rad2, p->tw2);
     const int64_t grid = ((p->N1 + p->TR - 1) / p->TR * batch + 7) / 8 * 8;
     ProfScope ps(st, "fft_fs_rows", bytes);
-    fs_rows<<<static_cast<unsigned>(grid), FS_T, 0, st>>>(a);
+    const int th = p->N2 * p->TR > 512 * FS_PER ? 1024 : 512;
+    const size_t lds = (FS_PER * th + a.ntw) * sizeof(c32);
+    const auto kern = th == 512 ? fs_rows<512> : fs_rows<1024>;
+    kern<<<static_cast<unsigned>(grid), th, lds, st>>>(a);
     ZDT_CHECK_LAUNCH("fs_rows");
   }
   return ZDT_OK;

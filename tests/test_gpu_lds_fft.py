@@ -55,6 +55,17 @@ def test_many_transforms(F, Nf, Nt, Nr):
     assert np.max(np.abs(out - ref)) <= 2e-6 * np.max(np.abs(ref))
 
 
+# the blocks of fs_cols: 125 x 16 and 147 x 16 elements in few and in many blocks, 243 x 16,
+# 315 x 16, 576 x 8, each with a partial last block of columns and rows
+@pytest.mark.parametrize("Nf,Nt,Nr", [(15625, 3, 7), (15625, 3, 141), (21609, 2, 151), (2 * 15625, 70, 2), (59049, 2, 9),
+                                      (99225, 2, 3), (2 * 589824, 2, 3)])
+def test_blocks_of_columns(F, Nf, Nt, Nr):
+    s = synth.spectrogram(Nf, Nt, [(Nf * 0.4, 0.1, 10.0)], seed=2)
+    out = F.zdtfdr(F.ZDTWorkspace(s, -1.0, 1.0 / 64, Nr, generic=True)).cpu().numpy()
+    ref = Z.fdr64(s, -1.0, 1.0 / 64, Nr)
+    assert np.max(np.abs(out - ref)) <= 2e-6 * np.max(np.abs(ref))
+
+
 @pytest.mark.parametrize("Nf", [4096, 30000, 99225])
 def test_radix_cap(F, Nf):
     check(F, Nf, 2, 3, radix_cap=8)
