@@ -160,6 +160,11 @@ struct zdt_ws {
   FastPlan* fout = nullptr;
   c32* Ft = nullptr;  // its input spectrum, Nk x Nt entries in the transposed layout
   bool ys_fout = false;  // last run left its spectra in fout
+  // fftfdr from Ft: its own spectra, for up to rates_cap rates at a time
+  FastPlan* rates = nullptr;
+  int64_t rates_cap = 0;
+  void* Yr = nullptr;  // fftfdr's spectra on the generic path, up to FFTFDR_KEEP with their scratch
+  size_t Yr_bytes = 0;
 
   bool have_input = false;
   const c32* ys_src = nullptr;  // post-processed spectra for zdt_output
@@ -535,6 +540,8 @@ int zdt_destroy(zdt_ws* ws) {
   for (int i = 0; i < 3; ++i) dev_free(ws->s[i]);
   if (ws->fast) fast_destroy(ws->fast);
   if (ws->fout) fast_destroy(ws->fout);
+  fast_destroy(ws->rates);
+  dev_free(ws->Yr);
   delete ws->prof;
   delete ws;
   return ZDT_OK;
@@ -698,6 +705,9 @@ struct AsyncBufs {
 };
 }  // namespace
 
+// bytes of spectra and scratch that fftfdr keeps on the generic path
+static constexpr size_t FFTFDR_KEEP = size_t(256) << 20;
+
 int zdt_fftfdr(zdt_ws* ws, const float* rates, int64_t nrates, float* dest) {
   ZDT_TRY(check_ws(ws));
   ProfInstall prof_(ws);
@@ -705,24 +715,63 @@ int zdt_fftfdr(zdt_ws* ws, const float* rates, int64_t nrates, float* dest) {
     return fail(ZDT_EINVAL, "fftfdr!: need a host rate list (1..2^24 rates) and a dest");
   ZDT_TRY(set_device(ws));
   if (!ws->have_input) return fail(ZDT_ESTATE, "fftfdr!: no input");
-  ZDT_TRY(ensure_F_natural(ws));
   // phasor(k, t, Float32(rate), Nf) = cispi(2 k t r/Nf) (src/fftfdr.jl:10-12)
   std::vector<double> rh(static_cast<size_t>(nrates));
   for (int64_t j = 0; j < nrates; ++j) {
     if (!std::isfinite(rates[j])) return fail(ZDT_EINVAL, "fftfdr!: rate %lld is not finite", (long long)j);
     rh[static_cast<size_t>(j)] = static_cast<double>(rates[j]) / static_cast<double>(ws->Nf);
   }
+  if (ws->fout != nullptr) {
+    // The spectra stay with the workspace: allocated and given back by every call
+    // they cost a caller that waits for its result 900 us a time.  2^18 x 16 x 64, whole
+    // calls back to back: 180 us on the generic kernels -> 98 (input 22, czt_rates 25,
+    // k2_c2r 26, k3 29)
+    const int64_t cap = std::min(nrates, fast_rates_chunk(ws->Nf));
+    if (ws->rates_cap < cap) {
+      fast_destroy(ws->rates);
+      ws->rates = nullptr;
+      if (ws->rates_cap > 0) ws->bytes -= fast_out_bytes(ws->Nf, ws->rates_cap);
+      ws->rates_cap = 0;
+      ZDT_TRY(fast_out_create(ws->Nf, cap, ZDT_PRECISION_FP32, &ws->rates));
+      ws->rates_cap = cap;
+      ws->bytes += fast_out_bytes(ws->Nf, cap);
+    }
+    return fast_out_rates(ws->rates, ws->Ft, static_cast<int>(ws->Nt), rh.data(), nrates, dest, ws->stream);
+  }
+  ZDT_TRY(ensure_F_natural(ws));
   AsyncBufs tmp(ws->stream);
-  void *rd = nullptr, *Y = nullptr, *s0 = nullptr, *s1 = nullptr, *s2 = nullptr;
+  void *Y = nullptr, *s0 = nullptr, *s1 = nullptr, *s2 = nullptr;
   const size_t sc = fft_real_scratch_elems(ws->Nf, nrates) * sizeof(c32);
-  ZDT_TRY(tmp.get(&rd, rh.size() * sizeof(double)));
-  ZDT_TRY(tmp.get(&Y, static_cast<size_t>(ws->Nk * nrates) * sizeof(c32)));
-  ZDT_TRY(tmp.get(&s0, sc));
-  ZDT_TRY(tmp.get(&s1, sc));
-  ZDT_TRY(tmp.get(&s2, sc));
-  ZDT_TRY_HIP(hipMemcpyAsync(rd, rh.data(), rh.size() * sizeof(double), hipMemcpyHostToDevice, ws->stream));
-  ZDT_TRY(launch_czt_rates(ws->F, ws->Nk, static_cast<c32*>(Y), ws->Nk, ws->Nk, ws->Nf, static_cast<int>(ws->Nt),
-                           static_cast<const double*>(rd), static_cast<int>(nrates), ws->stream));
+  const size_t yb = static_cast<size_t>(ws->Nk * nrates) * sizeof(c32);
+  if (yb + 3 * sc <= FFTFDR_KEEP) {
+    ZDT_TRY(ensure_scratch(ws, sc));
+    if (ws->Yr_bytes < yb) {
+      dev_free(ws->Yr);
+      ws->bytes -= static_cast<int64_t>(ws->Yr_bytes);
+      ws->Yr_bytes = 0;
+      ZDT_TRY(dev_alloc(ws, &ws->Yr, yb));
+      ws->Yr_bytes = yb;
+    }
+    Y = ws->Yr;
+    s0 = ws->s[0];
+    s1 = ws->s[1];
+    s2 = ws->s[2];
+  } else {
+    ZDT_TRY(tmp.get(&Y, yb));
+    ZDT_TRY(tmp.get(&s0, sc));
+    ZDT_TRY(tmp.get(&s1, sc));
+    ZDT_TRY(tmp.get(&s2, sc));
+  }
+  CztRatesArgs c;
+  c.F = ws->F;
+  c.fs = ws->Nk;
+  c.Ys = static_cast<c32*>(Y);
+  c.ys = ws->Nk;
+  c.n = ws->Nk;
+  c.logN1 = c.logN2 = 0;
+  c.yM = nullptr;
+  c.Nt = static_cast<int>(ws->Nt);
+  ZDT_TRY(launch_czt_rates(c, rh.data(), nrates, ws->stream));
   ZDT_TRY(fft_c2r(ws->Nf, static_cast<const c32*>(Y), ws->Nk, dest, ws->Nf, nrates, 1.0, s0, s1, s2, ws->stream,
                   ws->maxr));
   return ZDT_OK;

@@ -53,4 +53,10 @@ int fast_out_unpack_F(FastPlan* p, const c32* Ft, int64_t Nt, c32* F, hipStream_
 int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkind, const float* window, float* dest,
                  double scale, hipStream_t st, double* colmean = nullptr, double* colvar = nullptr);
 
+// fftfdr over a list of rates (rates_over_nf: host, Nr values) from the same Ft, in
+// pieces of the plan's Nr; fast_rates_chunk: the most rates a plan for it needs
+int64_t fast_rates_chunk(int64_t Nf);
+int fast_out_rates(FastPlan* p, const c32* F, int Nt, const double* rates_over_nf, int64_t Nr, float* dest,
+                   hipStream_t st);
+
 }  // namespace zdt

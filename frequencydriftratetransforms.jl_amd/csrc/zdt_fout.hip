@@ -13,6 +13,7 @@
 
 #include "zdt_fast_dev.h"
 #include "zdt_fast_plan.h"
+#include "zdt_kernels.h"
 
 namespace zdt {
 
@@ -798,6 +799,40 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
   }
   p->have_B = per >= p->Nr;
   if (colmean != nullptr && dest != nullptr) ZDT_TRY(fast_stats_merge(p, st, colmean, colvar));
+  return ZDT_OK;
+}
+
+int64_t fast_rates_chunk(int64_t Nf) { return std::max<int64_t>(1, FOUT_CHUNK / (4 * Nf)); }
+
+int fast_out_rates(FastPlan* p, const c32* F, int Nt, const double* rates_over_nf, int64_t Nr, float* dest,
+                   hipStream_t st) {
+  // chunks whose spectra B stay in the last-level cache, as in fast_out_run
+  for (int64_t j0 = 0; j0 < Nr; j0 += p->Nr) {
+    const int64_t n = std::min(p->Nr, Nr - j0);
+    CztRatesArgs c;
+    c.F = F;
+    c.fs = p->M;
+    c.Ys = p->Yc;
+    c.ys = p->M;
+    c.n = p->M;
+    c.logN1 = p->logN1;
+    c.logN2 = p->logN2;
+    c.yM = p->yM;
+    c.Nt = Nt;
+    ZDT_TRY(launch_czt_rates(c, rates_over_nf + j0, n, st));
+    K2cArgs a;
+    a.Yc = p->Yc;
+    a.yM = p->yM;
+    a.B = p->B;
+    a.yhalf = p->yhalf;
+    a.tw1 = p->tw1;
+    a.Nr = static_cast<int>(n);
+    a.M = p->M;
+    a.Nf = p->Nf;
+    a.oscale = static_cast<float>(1.0 / static_cast<double>(p->M));
+    ZDT_TRY(run_k2c(p, a, st));
+    ZDT_TRY(fast_output_part(p, dest + j0 * p->Nf, 0, n, st, false));
+  }
   return ZDT_OK;
 }
 

@@ -31,9 +31,21 @@ struct CztArgs {
 
 // F -> Ys by czt_fold
 int launch_czt(const CztArgs& a, hipStream_t st);
-// fftfdr: Ys[k,j] = sum_t F[k,t] e^{2 pi i k t rates[j]/Nf} (rates_over_nf: device, Nr doubles)
-int launch_czt_rates(const c32* F, int64_t ldF, c32* Ys, int64_t ldY, int64_t Nk, int64_t Nf, int Nt,
-                     const double* rates_over_nf, int Nr, hipStream_t st);
+// fftfdr: Ys[k,j] = sum_t F[k,t] e^{2 pi i k t rates[j]/Nf}
+constexpr int CZT_RATES_MAX = 128;  // rates a launch
+struct CztRatesArgs {
+  const c32* F;
+  int64_t fs;  // between time steps
+  c32* Ys;
+  int64_t ys;  // between rates
+  int64_t n;   // bins: Nk, or with yM the M bins before the Nyquist one
+  int logN1, logN2;
+  c32* yM;  // not null: F and Ys as the fused output has them, bin M to yM
+  int Nt, Nr;
+  double rh[CZT_RATES_MAX];
+};
+// rates_over_nf: host, Nr values; a.Nr and a.rh are set here
+int launch_czt_rates(CztRatesArgs a, const double* rates_over_nf, int64_t Nr, hipStream_t st);
 // fdshift: Y[k,t] = F[k,t] e^{2 pi i k t rate/Nf}
 int launch_shift_phase(const c32* F, int64_t ldF, c32* Y, int64_t ldY, int64_t Nk, int Nt, double rate_over_nf,
                        hipStream_t st);

@@ -112,66 +112,89 @@ int launch_czt(const CztArgs& a, hipStream_t st) {
 // Per bin and rate z = e^{2 pi i k rates[j]/Nf} and z^16 are evaluated
 // directly (k*rate/Nf reduced in FP64), and the polynomial is evaluated as
 // 16-term Horner blocks combined by Horner in z^16, so no power of a rounded
-// z above the 15th enters the sum.  For Nt > 64 every term's phase is
+// z above the 15th enters the sum.  For Nt > 64 (NT = 0) every term's phase is
 // evaluated directly.
-template <int NT>
-__global__ __launch_bounds__(256) void czt_rates(const c32* __restrict__ F, int64_t ldF, c32* __restrict__ Ys,
-                                                 int64_t ldY, int64_t Nk, int64_t Nf, int Nt,
-                                                 const double* __restrict__ rh, int Nr) {
-  constexpr int B = NT < 16 ? NT : 16;
+//
+// COL: F and Ys in the fused output's order (bin k2 + N2 k1 at k1 + N1 k2, the
+// Nyquist bins apart), else natural.  The rates are kernel arguments (no copy to
+// the device to wait for), and groups of them go over blockIdx.y up to 16 wavefronts a CU.
+// VALU-bound at 16 steps (about 115 operations a bin and rate): 2^18 x 16 x 64
+// 29 -> 25 us.
+template <int NT, bool COL>
+__global__ __launch_bounds__(256) void czt_rates(CztRatesArgs a) {
+  constexpr int B = NT < 16 ? (NT < 1 ? 1 : NT) : 16;
   constexpr int NB = NT / B;
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k >= Nk) return;
+  const int64_t g = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const bool in = COL || g < a.n;  // COL: whole blocks
+  const int64_t o = in ? g : a.n - 1;
+  const int64_t k = COL ? (g >> a.logN1) + ((g & ((int64_t(1) << a.logN1) - 1)) << a.logN2) : o;
   const double kd = static_cast<double>(k);
-  c32 c[NT];
+  const int j0 = group_first(a.Nr, blockIdx.y, gridDim.y), j1 = group_first(a.Nr, blockIdx.y + 1, gridDim.y);
+  if constexpr (NT > 0) {
+    c32 c[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) c[t] = (t < Nt) ? F[k + static_cast<int64_t>(t) * ldF] : c32{0.0f, 0.0f};
-  for (int j = 0; j < Nr; ++j) {
-    const c32 zf = cis_nh(kd, rh[j]);                          // rh[j] = rates[j]/Nf
-    const c32 zBf = cis_nh(kd * static_cast<double>(B), rh[j]);
-    c32 acc = {0.0f, 0.0f};
+    for (int t = 0; t < NT; ++t) c[t] = (t < a.Nt) ? a.F[o + t * a.fs] : c32{0.0f, 0.0f};
+#pragma unroll 2
+    for (int j = j0; j < j1; ++j) {
+      const c32 zf = cis_nh(kd, a.rh[j]);  // rh[j] = rates[j]/Nf
+      const c32 zBf = cis_nh(kd * static_cast<double>(B), a.rh[j]);
+      c32 acc = {0.0f, 0.0f};
 #pragma unroll
-    for (int b = NB - 1; b >= 0; --b) {
-      c32 p = c[b * B + B - 1];
+      for (int b = NB - 1; b >= 0; --b) {
+        c32 p = c[b * B + B - 1];
 #pragma unroll
-      for (int u = B - 2; u >= 0; --u) p = cfma(c[b * B + u], p, zf);
-      acc = (b == NB - 1) ? p : cfma(p, acc, zBf);
+        for (int u = B - 2; u >= 0; --u) p = cfma(c[b * B + u], p, zf);
+        acc = (b == NB - 1) ? p : cfma(p, acc, zBf);
+      }
+      if (in) a.Ys[o + j * a.ys] = acc;
     }
-    Ys[k + static_cast<int64_t>(j) * ldY] = acc;
-  }
-}
-
-__global__ __launch_bounds__(256) void czt_rates_any(const c32* __restrict__ F, int64_t ldF, c32* __restrict__ Ys,
-                                                     int64_t ldY, int64_t Nk, int Nt, const double* __restrict__ rh,
-                                                     int Nr) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (k >= Nk) return;
-  const double kd = static_cast<double>(k);
-  for (int j = 0; j < Nr; ++j) {
-    c32 acc = {0.0f, 0.0f};
-    for (int t = 0; t < Nt; ++t)
-      acc = cfma(acc, F[k + static_cast<int64_t>(t) * ldF], cis_nh(kd * static_cast<double>(t), rh[j]));
-    Ys[k + static_cast<int64_t>(j) * ldY] = acc;
-  }
-}
-
-int launch_czt_rates(const c32* F, int64_t ldF, c32* Ys, int64_t ldY, int64_t Nk, int64_t Nf, int Nt,
-                     const double* rates_over_nf, int Nr, hipStream_t st) {
-  const unsigned grid = static_cast<unsigned>((Nk + 255) / 256);
-  ProfScope ps(st, "czt_rates", 8.0 * static_cast<double>(Nk) * (Nt + Nr));
-  const double* rh = rates_over_nf;
-  if (Nt <= 4) {
-    czt_rates<4><<<grid, 256, 0, st>>>(F, ldF, Ys, ldY, Nk, Nf, Nt, rh, Nr);
-  } else if (Nt <= 16) {
-    czt_rates<16><<<grid, 256, 0, st>>>(F, ldF, Ys, ldY, Nk, Nf, Nt, rh, Nr);
-  } else if (Nt <= 32) {
-    czt_rates<32><<<grid, 256, 0, st>>>(F, ldF, Ys, ldY, Nk, Nf, Nt, rh, Nr);
-  } else if (Nt <= 64) {
-    czt_rates<64><<<grid, 256, 0, st>>>(F, ldF, Ys, ldY, Nk, Nf, Nt, rh, Nr);
   } else {
-    czt_rates_any<<<grid, 256, 0, st>>>(F, ldF, Ys, ldY, Nk, Nt, rh, Nr);
+    for (int j = j0; j < j1; ++j) {
+      c32 acc = {0.0f, 0.0f};
+      for (int t = 0; t < a.Nt; ++t)
+        acc = cfma(acc, a.F[o + t * a.fs], cis_nh(kd * static_cast<double>(t), a.rh[j]));
+      if (in) a.Ys[o + j * a.ys] = acc;
+    }
   }
-  ZDT_CHECK_LAUNCH("czt_rates");
+  if constexpr (COL) {
+    // the Nyquist bin, a wavefront per rate over all blocks
+    const int lane = threadIdx.x & 63, nw = 4 * gridDim.x * gridDim.y;
+    for (int j = 4 * (blockIdx.y * gridDim.x + blockIdx.x) + (threadIdx.x >> 6); j < a.Nr; j += nw) {
+      c32 s = {0.0f, 0.0f};
+      for (int t = lane; t < a.Nt; t += 64)
+        s = cfma(s, a.F[a.n * a.Nt + t], cis_nh(static_cast<double>(a.n) * static_cast<double>(t), a.rh[j]));
+#pragma unroll
+      for (int x = 32; x > 0; x >>= 1) {
+        s.x += __shfl_xor(s.x, x, 64);
+        s.y += __shfl_xor(s.y, x, 64);
+      }
+      if (lane == 0) a.yM[j] = s;
+    }
+  }
+}
+
+int launch_czt_rates(CztRatesArgs a, const double* rates_over_nf, int64_t Nr, hipStream_t st) {
+  ProfScope ps(st, "czt_rates", 8.0 * static_cast<double>(a.n) * static_cast<double>(a.Nt + Nr));
+  int ncu = 256, dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  const bool col = a.yM != nullptr;
+  const int nblk = static_cast<int>((a.n + 255) / 256);
+  for (int64_t j0 = 0; j0 < Nr; j0 += CZT_RATES_MAX) {
+    a.Nr = static_cast<int>(std::min<int64_t>(CZT_RATES_MAX, Nr - j0));
+    for (int j = 0; j < a.Nr; ++j) a.rh[j] = rates_over_nf[j0 + j];
+    const dim3 grid(static_cast<unsigned>(nblk), group_parts(a.Nr, nblk, 256, 16, 8, ncu));
+#define ZDT_RATES(NT)                              \
+  (col ? czt_rates<NT, true><<<grid, 256, 0, st>>>(a) : czt_rates<NT, false><<<grid, 256, 0, st>>>(a))
+    if (a.Nt <= 4) ZDT_RATES(4);
+    else if (a.Nt <= 16) ZDT_RATES(16);
+    else if (a.Nt <= 32) ZDT_RATES(32);
+    else if (a.Nt <= 64) ZDT_RATES(64);
+    else ZDT_RATES(0);
+#undef ZDT_RATES
+    ZDT_CHECK_LAUNCH("czt_rates");
+    a.Ys += a.Nr * a.ys;
+    if (col) a.yM += a.Nr;
+  }
   return ZDT_OK;
 }
 

@@ -30,6 +30,7 @@ ZDT_FLAG_GENERIC = 0x2
 ZDT_FLAG_PROFILE = 0x4
 ZDT_FLAG_N2_512 = 0x8
 ZDT_FLAG_RADIX8 = 0x10
+ZDT_FLAG_NO_FUSED = 0x10000  # zdt_ws.h: the fused output or the generic kernels
 
 ZDT_PLAN_AUTOTUNE = 0x100
 

@@ -22,8 +22,8 @@ class FftFdrWorkspace:
     """fftfdr_workspace(spectrogram) -- src/fftfdr.jl:39-59."""
 
     def __init__(self, spectrogram):
-        # one rate, generic kernels: the workspace only serves its input spectrum
-        self.ws = ZDTWorkspace(spectrogram, 0.0, 1.0, 1, generic=True)
+        # one rate: the workspace only serves its input spectrum
+        self.ws = ZDTWorkspace(spectrogram, 0.0, 1.0, 1, _fused_output=True)
         self.Nf, self.Nt = self.ws.Nf, self.ws.Nt
 
     @property

@@ -68,7 +68,7 @@ class ZDTWorkspace:
 
     def __init__(self, spectrogram, *args, factors=None, output_aligned: bool = False,
                  unnormalized: bool = False, generic: bool = False, n2: int = 0, radix_cap: int = 16,
-                 precision: str = "fp32"):
+                 precision: str = "fp32", _fused_output: bool = False):
         if len(args) in (1, 2) and not isinstance(args[0], (int, float, np.floating, np.integer)):
             r0, dr, Nr = rates_params(args[0])
             if len(args) == 2:
@@ -90,6 +90,7 @@ class ZDTWorkspace:
         self.device = spec.device
         self._stream = D.stream_ptr()
         flags = ((_lib.ZDT_FLAG_UNNORMALIZED if unnormalized else 0) | (_lib.ZDT_FLAG_GENERIC if generic else 0)
+                 | (_lib.ZDT_FLAG_NO_FUSED if _fused_output else 0)
                  | (_lib.ZDT_FLAG_N2_512 if n2 == 512 else 0) | (_lib.ZDT_FLAG_RADIX8 if radix_cap == 8 else 0))
         if radix_cap not in (8, 16):
             raise ValueError("radix_cap must be 8 or 16")
