@@ -21,7 +21,6 @@ struct CztArgs {
   int64_t Nk, Nf;
   int Nt, Nr;
   double hd;  // dr/(2 Nf): chirp(k,l) = exp(-2 pi i k l^2 hd)
-  double h0;  // r0/Nf:     pre(k,t) = exp(2 pi i (k t^2 hd + k t h0))
   double hc;  // rc/Nf, rc = r0 + (Nr-1) dr/2 the centre rate
   double hz;  // (r0 - rc)/Nf
   int wkind;
