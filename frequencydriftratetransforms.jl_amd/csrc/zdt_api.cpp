@@ -1016,8 +1016,8 @@ int zdt_findhits_scratch(int nb, int64_t Nf, int64_t Nr, int snr, int64_t* bytes
 
 // Whole call at 2^20 x 129 with 44 proto-hits: 509 us as fdrstats, findprotohits and
 // clusterprotohits (three synchronizations, each with memory allocated and given
-// back, six copies of results, two reads of the matrix) -> 193, of which 93 the read and 43
-// eight launches.
+// back, six copies of results, two reads of the matrix) -> 183, of which 93 the read and 33
+// six launches.
 int zdt_findhits(const float* const* fdrs, int nb, int64_t Nf, int64_t Nr, int64_t ld, double threshold, int snr,
                  int di, int dj, void* scratch, int64_t scratch_bytes, int64_t* hits, int64_t cap, int64_t* found,
                  int64_t* nproto, int64_t* nhits, double* thr, void* stream) {
@@ -1052,11 +1052,13 @@ int zdt_findhits(const float* const* fdrs, int nb, int64_t Nf, int64_t Nr, int64
   for (int b = 0; b < nb; ++b)
     ZDT_TRY(launch_hits_count(fdrs[b], Nf, Nr, ld, threshold, thr_dev, counts + b * nt, st, nullptr, 0,
                               rmax ? rmax + b * Nr * nreg : nullptr));
-  ZDT_TRY(launch_hits_scan(counts, ntall, pack, counts + ntall, st));
+  const bool local = cap > 0 && hits_scan_local_ok(ntall);
+  ZDT_TRY(launch_hits_scan(counts, ntall, pack, counts + ntall, st, local));
   if (cap > 0)
     for (int b = 0; b < nb; ++b)
       ZDT_TRY(launch_hits_write_impl(fdrs[b], Nf, Nr, ld, threshold, thr_dev, counts, ntall, b * nt, pack,
-                                     static_cast<int64_t>(b) * Nf * Nr, hits, cap, st));
+                                     static_cast<int64_t>(b) * Nf * Nr, hits, cap, st, nullptr,
+                                     local ? counts + ntall : nullptr));
   // the head, and with it what a few hits take
   int64_t first = FOUND_HEAD;
   int64_t head[FOUND_HEAD];

@@ -282,10 +282,12 @@ int enqueue_channel(Shape& s, int c, const float* spec, float* dest, double thr,
   // the run maxima exist when the statistics pass wrote them
   const float* smax = snr ? s.smax : nullptr;
   ZDT_TRY(launch_hits_count(dest, s.Nf, s.Nr, ld, thr_h, thr_dev, s.counts, s.st, smax, ws_fused_n2(s.ws)));
-  ZDT_TRY(launch_hits_scan(s.counts, nt, nhits + c, s.counts + nt, s.st));
+  const bool local = cap > 0 && hits_scan_local_ok(nt);
+  ZDT_TRY(launch_hits_scan(s.counts, nt, nhits + c, s.counts + nt, s.st, local));
   if (cap > 0)
     ZDT_TRY(launch_hits_write_impl(dest, s.Nf, s.Nr, ld, thr_h, thr_dev, s.counts, nt, 0, nhits + c, 0,
-                                   hits + static_cast<int64_t>(c) * cap, cap, s.st));
+                                   hits + static_cast<int64_t>(c) * cap, cap, s.st, nullptr,
+                                   local ? s.counts + nt : nullptr));
   return ZDT_OK;
 }
 

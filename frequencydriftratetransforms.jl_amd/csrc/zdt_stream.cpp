@@ -341,10 +341,12 @@ int stream_run(zdt_stream* s, const float* const* host_specs, int nspec, double 
       const int64_t nv = valid(b);
       const int64_t nt = hits_tiles(Nf, nv);
       ZDT_TRY(launch_hits_count(f, Nf, nv, Nf, 0.0, thr_dev, counts, s->compute, smax_of(b), ws_fused_n2(s->ws)));
-      ZDT_TRY(launch_hits_scan(counts, nt, batch_total, scan_scratch, s->compute));
+      const bool local = cap > 0 && hits_scan_local_ok(nt);
+      ZDT_TRY(launch_hits_scan(counts, nt, batch_total, scan_scratch, s->compute, local));
       if (cap > 0)
         ZDT_TRY(launch_hits_write_impl(f, Nf, nv, Nf, 0.0, thr_dev, counts, nt, 0, batch_total, b * Nrb * Nf,
-                                       s->dhits[slot], cap, s->compute, b == 0 ? nullptr : running));
+                                       s->dhits[slot], cap, s->compute, b == 0 ? nullptr : running,
+                                       local ? scan_scratch : nullptr));
       ZDT_TRY(launch_accumulate_i64(running, batch_total, b == 0, s->compute));
     }
     char* hs = static_cast<char*>(s->hsmall) + 16 * slot;

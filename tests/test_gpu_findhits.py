@@ -131,3 +131,25 @@ def test_refusals(F):
     n, nh, thr = C.c_int64(), C.c_int64(), C.c_double()
     assert L.zdt_findhits(arr, 1, 5000, 3, 5000, 5.0, 1, 1, 1, None, 0, None, 0, None, C.byref(n), C.byref(nh),
                           C.byref(thr), None) == _lib.ZDT_EINVAL
+
+
+@pytest.mark.parametrize("tiles,nb", [(1, 1), (17, 2), (2047, 1), (2048, 1), (2049, 1), (1500, 3), (4097, 2), (131072, 1),
+                                      (131073, 1)])
+def test_scan_of_tile_counts(F, tiles, nb):
+    """Proto-hits at the ends of tiles and everywhere in a few, around the chunks of
+    the scan and on both sides of the most chunks that the write pass adds up."""
+    import torch
+    rng = np.random.default_rng(tiles)
+    Nf = 4096
+    fdrs, want = [], []
+    for b in range(nb):
+        d = torch.zeros((tiles, Nf), dtype=torch.float32, device="cuda")
+        pick = np.unique(np.concatenate([rng.integers(0, tiles, 40), [0, tiles - 1], np.arange(2046, 2050) % tiles]))
+        full = pick[:3].repeat(Nf) * Nf + np.tile(np.arange(Nf), len(pick[:3]))
+        lin = np.unique(np.concatenate([pick * Nf, pick * Nf + Nf - 1, full]))
+        d.view(-1)[torch.from_numpy(lin).cuda()] = 2.0
+        fdrs.append(d.t())
+        want.append(np.stack([lin % Nf + 1, lin // Nf + 1 + b * tiles], axis=1))
+    want = np.concatenate(want)
+    assert np.array_equal(F.findprotohits(fdrs, 1.0), want)
+    assert np.array_equal(F.findprotohits(fdrs, 1.0, capacity=100), want)
