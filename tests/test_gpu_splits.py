@@ -33,7 +33,7 @@ def check(F, Nf, Nt, Nr, r0, dr, path):
     assert np.max(np.abs(out - ref)) <= 2e-6 * np.max(np.abs(ref))
 
 
-# paired rates (Nt > 8; groups of two pairs, three groups a part) and single
+# paired rates (Nt > 8; groups of two pairs, from one group a part on) and single
 # rates (groups of four), N1 = 64 and 128
 @pytest.mark.parametrize("Nf,Nt,Nr", [(1 << 16, 16, n) for n in (1, 2, 11, 12, 13, 23, 24, 25, 47, 131)]
                          + [(1 << 16, 5, n) for n in (1, 4, 11, 12, 13, 24, 25, 131)]
