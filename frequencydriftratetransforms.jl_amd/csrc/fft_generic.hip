@@ -735,9 +735,8 @@ static std::vector<c32> fs_twiddles(const std::vector<int>& rad) {
       for (int r = 1; r < R; ++r)
         for (int64_t k = 0; k < Ns; ++k) {
           const int64_t n = Ns * R, m = r * k;  // m < n
-          const long double x = 2.0L * 3.14159265358979323846264338327950288L * static_cast<long double>(m) /
-                                static_cast<long double>(n);
-          double c = static_cast<double>(cosl(x)), sn = -static_cast<double>(sinl(x));
+          const double x = 6.283185307179586 * static_cast<double>(m) / static_cast<double>(n);
+          double c = std::cos(x), sn = -std::sin(x);
           if (4 * m == n || 4 * m == 3 * n) c = 0.0;
           if (2 * m == n) sn = 0.0;
           t.push_back({static_cast<float>(c), static_cast<float>(sn)});
