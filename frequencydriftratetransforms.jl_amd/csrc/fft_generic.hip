@@ -726,7 +726,8 @@ static void fs_choose(FftPlan* p, int maxr) {
 }
 
 // the passes' twiddles W_{Ns R}^{r k} (r = 1 .. R-1, k < Ns) of every pass but the
-// first, in order
+// first, in order (double sines: 4096 entries in 0.1 to 0.4 ms on the
+// host, against 0.7 to 0.8 from 80-bit ones; rounded to 32 bits either way)
 static std::vector<c32> fs_twiddles(const std::vector<int>& rad) {
   std::vector<c32> t;
   int64_t Ns = 1;
