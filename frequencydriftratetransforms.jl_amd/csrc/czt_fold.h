@@ -21,6 +21,7 @@
 
 #include <type_traits>
 
+#include "rate_groups.h"
 #include "zdt_internal.h"
 
 namespace zdt {
@@ -269,13 +270,6 @@ __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r,
       }
     }
   }
-}
-
-// First of the n rate (or time) groups that part y of np takes (0 <= y <= np,
-// n < 2^16): the column-pair kernels split their groups over blockIdx.y where
-// the column pairs alone leave the chip idle (group_parts, zdt_fast_plan.h).
-__device__ __forceinline__ int group_first(int n, unsigned y, unsigned np) {
-  return static_cast<int>(static_cast<unsigned>(n) * y / np);
 }
 
 // Lanes per bin and blocks per lane for Nt time steps: up to five blocks (160

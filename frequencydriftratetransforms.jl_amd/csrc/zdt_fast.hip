@@ -436,7 +436,7 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
     static_assert(RPW * NW == ROWS && RPW * fft_max_nr<N1>() <= 64, "one butterfly per lane and pass");
     const int wv = tid >> 6, lane = tid & 63;
     const int Pm = a.Nr - 1;        // rate j pairs with Pm - j
-    const int npairs = Pm / 2 + 1;  // the last is the middle rate when Pm is even
+    const int npairs = rate_pairs(a.Nr);  // the last is the middle rate when Pm is even
     c64 gam[PP], zp[PP], zq[PP];
 #pragma unroll
     for (int i = 0; i < PP; ++i) {
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
     }
     // groups from the middle rates outwards, so that the rates k3 reads
     // first (Nr-1, 0, Nr-2, 1, ...) are the ones written last
-    const int ng = (npairs + NPG - 1) / NPG;
+    const int ng = k2_groups(a.Nr, ROWS, true);
     const int glo = group_first(ng, blockIdx.y, gridDim.y) * NPG;
     const int g0 = (group_first(ng, blockIdx.y + 1, gridDim.y) - 1) * NPG;
 #pragma unroll
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(N1 < 512 ? N1 : 512, k2_waves_per_eu(N1)) void k2_c
   } else {
     // ---- chirp-Z for every rate, c2r pre-pass, inverse DFT_N1, store
     constexpr int JG = ROWS / 2;
-    const int ng = (a.Nr + JG - 1) / JG;
+    const int ng = k2_groups(a.Nr, ROWS, false);
     const int jlo = group_first(ng, blockIdx.y, gridDim.y) * JG;
     const int jhi = min(a.Nr, group_first(ng, blockIdx.y + 1, gridDim.y) * JG);
     c64 gam[PP], z[PP];
@@ -831,19 +831,7 @@ template <int N1, int N2>
 static int launch_k2(const K2Args& a, int NT, bool paired, int64_t ncu, hipStream_t st) {
   constexpr unsigned TB = N1 < 512 ? N1 : 512;
   constexpr int RW = k2_rows(N1);
-  // rate groups over blockIdx.y.  Each part repeats the input phase, which costs
-  // nothing while the CUs have room (one wavefront per SIMD issues no slower
-  // beside others), so parts go down to one group: 2^16 channels 17 rates 21.3 ->
-  // 16.1 us against three groups at least, 9 17.3 -> 15.5, 33 19.9 -> 18.9, 2^18 x
-  // 65 42.2 -> 40.0; 2^17 x 33 22.9 -> 23.9.  The waves a CU holds are bounded by
-  // VGPRs (N1 <= 128) or LDS (256: 8, 512: 16).  At 129 rates, one part -> this
-  // rule: 2^16 69.8 -> 29.6 us, 2^17 72.6 -> 36.6, 2^18 93.0 -> 61.7; a second part
-  // only costs at 2^19 (110.8 -> 128.3) and 2^20 (181 -> 205), whose blocks fill the
-  // chip.
-  constexpr int WAVES = N1 >= 512 ? 16 : (N1 == 256 ? 8 : 12);
-  const int units = (paired && NT == 16) ? a.Nr / 2 + 1 : a.Nr;  // rate pairs or rates
-  const int per = (paired && NT == 16) ? RW / 4 : RW / 2;
-  const dim3 grid(N2 / 2, group_parts((units + per - 1) / per, N2 / 2, TB, WAVES, 1, ncu));
+  const dim3 grid(N2 / 2, k2_parts(N1, N2, k2_groups(a.Nr, RW, paired && NT == 16), ncu));
   if (paired && NT == 16) {
     k2_czt<N1, N2, 16, RW, true><<<grid, TB, 0, st>>>(a);
     ZDT_CHECK_LAUNCH("k2_czt");

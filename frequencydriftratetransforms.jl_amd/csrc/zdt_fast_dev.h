@@ -429,9 +429,6 @@ __device__ __forceinline__ c32 horner(const c32* a, c32 z) {
 // k2 occupancy target: two 512-thread blocks per CU (4 waves per SIMD) for
 // N1 = 512, whose LDS (2 x 8 rows x 576 + 512 entries, 78 KB) allows it.
 constexpr int k2_waves_per_eu(int n1) { return n1 >= 512 ? 4 : 2; }
-// rows per group: as many as keep one butterfly per lane in the
-// wavefront-level passes (8 rows for 512 = 8*8*8 over 8 wavefronts, ...)
-constexpr int k2_rows(int n1) { return n1 == 256 ? 16 : 8; }
 
 // The Hermitian pair q of column-pair block p (see k2_czt): bin
 // kA = cA + N2 k1A in row rowA of the block's two rows and its partner

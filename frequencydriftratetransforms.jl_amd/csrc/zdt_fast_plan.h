@@ -38,15 +38,6 @@ struct FastPlan {
   float* smax = nullptr;
 };
 
-// Parts (blockIdx.y) for ng groups of rates or time steps: as many as bring
-// nblk blocks of `threads` up to `waves` wavefronts a CU, with at least
-// `least` groups each (see group_first).
-inline unsigned group_parts(int ng, int nblk, int threads, int waves, int least, int64_t ncu) {
-  const int64_t fill = waves * ncu / (static_cast<int64_t>(nblk) * (threads / 64));
-  const int64_t s = fill < ng / least ? fill : ng / least;
-  return static_cast<unsigned>(s < 1 ? 1 : s);
-}
-
 int ilog2i(int64_t n);
 // device copy of a host table
 int upload_table(c32** dst, const std::vector<c32>& h);
