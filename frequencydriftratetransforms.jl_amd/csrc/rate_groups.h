@@ -24,7 +24,8 @@ constexpr int k2_groups(int Nr, int rows, bool paired) {
   return paired ? groups_of(rate_pairs(Nr), rows / 4) : groups_of(Nr, rows / 2);
 }
 
-// First of the n groups that part y of np takes (0 <= y <= np, n < 2^16).
+// First of the n groups that part y of np takes (0 <= y <= np; n np < 2^32, which
+// group_parts sees to).
 constexpr int group_first(int n, unsigned y, unsigned np) {
   return static_cast<int>(static_cast<unsigned>(n) * y / np);
 }
@@ -32,8 +33,9 @@ constexpr int group_first(int n, unsigned y, unsigned np) {
 // Parts (blockIdx.y) for ng groups: as many as bring nblk blocks of `threads` up
 // to `waves` wavefronts a CU, with at least `least` groups each.
 constexpr unsigned group_parts(int ng, int nblk, int threads, int waves, int least, int64_t ncu) {
-  const int64_t fill = waves * ncu / (static_cast<int64_t>(nblk) * (threads / 64));
-  const int64_t s = fill < ng / least ? fill : ng / least;
+  int64_t s = waves * ncu / (static_cast<int64_t>(nblk) * (threads / 64));
+  if (s > ng / least) s = ng / least;
+  if (s > 0xFFFFFFFFll / ng) s = 0xFFFFFFFFll / ng;  // 5.6 million groups and more
   return static_cast<unsigned>(s < 1 ? 1 : s);
 }
 

@@ -35,6 +35,19 @@ int main() {
           }
           ++n;
         }
+  // the other kernels' rules (least groups a part, wavefronts a CU) up to 2^24 rates
+  const int rules[][3] = {{256, 12, 8}, {256, 12, 20}, {256, 8, 24}, {256, 16, 8}, {64, 24, 2}, {1024, 16, 1}};
+  for (const auto& r : rules)
+    for (int nblk : {1, 2, 3, 17, 256, 1024})
+      for (int ng : {1, 2, 7, 8, 63, 65535, 65536, 5592405, 5592406, 8388607, 8388608, 16777216})
+        for (int64_t ncu : {64, 256, 304}) {
+          const unsigned np = group_parts(ng, nblk, r[0], r[1], r[2], ncu);
+          if (np > 65535 || !tiles(ng, np)) {
+            std::printf("%d groups, %d blocks of %d: %u parts\n", ng, nblk, r[0], np);
+            return 1;
+          }
+          ++n;
+        }
   std::printf("%ld grids\n", n);
   return 0;
 }
