@@ -150,7 +150,12 @@ struct FoldBin {
   unsigned o;      // the bin's offset in both
   double kd;       // the bin k
   float w;         // window weight and scale
+  int* wide;       // fold_rates<NB, NC, true>: NULL, or set where the coefficients pass FOLD_WIDE
 };
+
+// Bound on the sum of a lane's coefficients |Re| + |Im| under which spectra of up
+// to 2^20 time steps stay below 2^96, and sums over 2^20 of them far from overflow.
+constexpr float FOLD_WIDE = 1.2e24f;  // 2^80
 
 struct FoldRates {
   int Nt, Nr;
@@ -174,7 +179,9 @@ __device__ __forceinline__ float quad_xor(float v) {
 // (one lane per bin): store past the last-level cache (nontemporal), for
 // destinations larger than it whose rows are whole cache lines; on rows that are
 // not, such stores cost half as much again (10^6 channels x 129: 136 -> 192 us).
-template <int NB, int NC>
+// GUARD: set *b.wide, if there is one, where the coefficients reach FOLD_WIDE or
+// are not finite.
+template <int NB, int NC, bool GUARD = false>
 __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r, int q, int tbase, int jlo, int jhi,
                                            bool acc, bool past) {
   const int t0 = tbase + FOLD * NB * q;
@@ -269,6 +276,18 @@ __device__ __forceinline__ void fold_rates(const FoldBin& b, const FoldRates& r,
         if (mine && q < 4) *df = acc ? v + *df : v;
       }
     }
+  }
+  // last, so that nothing above waits for the coefficients any sooner
+  if (GUARD && b.wide != nullptr) {  // uniform
+    float mag = 0.0f;  // at least the sum over the coefficients
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+#pragma unroll
+      for (int i = 0; i < FOLD / 2; ++i) {
+        mag += fabsf(c.p[u][i].x) + fabsf(c.p[u][i].y);
+        mag += fabsf(c.m[u][i].x) + fabsf(c.m[u][i].y);
+      }
+    if (!(mag < FOLD_WIDE)) *b.wide = 1;
   }
 }
 

@@ -175,6 +175,7 @@ static int pow2_floor(int64_t x) {
 constexpr int FS_PER = 8;    // elements a thread
 constexpr int FS_E = 8192;   // most elements per block of fs_cols / fs_rows (TC * N1 or TR * N2)
 constexpr int FS_ONE = 4096; // most elements per block of fs_one
+constexpr int FS_ONE_TH = FS_ONE / FS_PER;
 constexpr int FS_MAXP = 12;  // passes per sub-transform
 
 enum fs_mode {
@@ -182,7 +183,7 @@ enum fs_mode {
   FS_C2R,      // in: half spectra X[0..N] of real sequences of length 2N; out: their N packed pairs
   FS_R2C,      // fs_one: the reverse
   FS_ODD_R2C,  // in: real sequences of odd length N; out: X[0 .. N/2]
-  FS_ODD_C2R,  // in: half spectra X[0 .. N/2] of two columns (or one); out: the real columns
+  FS_ODD_C2R,  // in: half spectra X[0 .. N/2]; out: the real columns
 };
 
 struct FsArgs {
@@ -198,11 +199,19 @@ struct FsArgs {
   int rad[FS_MAXP];
   int inverse, mode;
   int64_t batch;     // transforms
-  int64_t ncol;      // FS_ODD_C2R: real columns
-  int pair;          // FS_ODD_C2R: two columns a transform
   float scale;
   double h;          // 1/N
 };
+
+// and of the kernels with two real columns a transform (FS_ODD_C2R); apart, because
+// 16 bytes more of arguments cost a 6 to 9 us kernel 0.2 us
+struct FsPair {
+  int64_t ncol;
+  const int* wide;  // not 0: one column a transform after all
+};
+struct FsNoPair {};
+template <bool PAIR>
+using FsPairOf = std::conditional_t<PAIR, FsPair, FsNoPair>;
 
 // u / d for u * d < 2^32 by one high multiply with m = ceil(2^32 / d)
 // (m = 0 marks d = 1)
@@ -331,35 +340,56 @@ __device__ __forceinline__ c32 c2r_pack(int k, c32 p, c32 q, c32 w) {
   return {Ev.x - O.y, Ev.y + O.x};
 }
 
+// bin of the half spectrum X[0 .. N/2] that holds entry n of the full one (N odd),
+// and the entry made from it; Im X[0] is ignored
+__device__ __forceinline__ int odd_bin(int n, int N) { return 2 * n > N ? N - n : n; }
+__device__ __forceinline__ c32 odd_full(int n, int N, c32 x) {
+  const float y = 2 * n > N ? -x.y : x.y;
+  return {x.x, n == 0 ? 0.0f : y};
+}
+
 // element n of transform b for the modes that need no twiddle, before the
 // conjugation of the inverse
 __device__ __forceinline__ c32 fs_input(const FsArgs& a, int64_t b, int n) {
   if (a.mode == FS_ODD_R2C) return {reinterpret_cast<const float*>(a.in)[b * a.ibs + n], 0.0f};
-  if (a.mode == FS_ODD_C2R) {
-    // the full Hermitian spectra of columns c0 and c0 + 1 as A + i B
-    const bool up = 2 * n > a.N;
-    const int k = up ? a.N - n : n;
-    const int64_t c0 = a.pair ? 2 * b : b;
-    c32 A = a.in[c0 * a.ibs + k], B = {0.0f, 0.0f};
-    if (a.pair && c0 + 1 < a.ncol) B = a.in[(c0 + 1) * a.ibs + k];
-    if (n == 0) A.y = B.y = 0.0f;
-    if (up) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    return {A.x - B.y, A.y + B.x};
-  }
+  if (a.mode == FS_ODD_C2R) return odd_full(n, a.N, a.in[b * a.ibs + odd_bin(n, a.N)]);
   return a.in[b * a.ibs + n];
+}
+
+// PAIR: two real columns a transform, 2b and 2b + 1, as the real and imaginary part
+// (the last of an odd number of them alone).  With *wide one column's values could
+// overflow into the other's: the block then takes 2b alone and, in a second turn
+// (half = 1, results between the kernels at transform batch + b), 2b + 1.
+__device__ __forceinline__ bool pair_second(const FsPair& p, int64_t b, int half) {
+  return half == 0 && 2 * b + 1 < p.ncol;
+}
+
+// *p.wide by a vector load, which is waited for with the tile's own
+__device__ __forceinline__ int pair_wide(const FsPair& p) {
+  int lane0 = 0;
+  asm volatile("" : "+v"(lane0));
+  return p.wide[lane0];
+}
+
+// element n of the pair's spectrum, A + i B, from its bins in the two columns
+__device__ __forceinline__ c32 pair_full(int n, int N, c32 A, c32 B, bool two) {
+  A = odd_full(n, N, A);
+  B = two ? odd_full(n, N, B) : c32{0.0f, 0.0f};
+  return {A.x - B.y, A.y + B.x};
+}
+
+// element k of the pair's columns
+__device__ __forceinline__ void pair_output(const FsArgs& a, int64_t col, bool two, int k, c32 v) {
+  float* out = reinterpret_cast<float*>(a.out) + col * a.obs + k;
+  out[0] = v.x * a.scale;
+  if (two) out[a.obs] = -v.y * a.scale;
 }
 
 // element k of transform b, scaled and (inverse) conjugated
 __device__ __forceinline__ void fs_output(const FsArgs& a, int64_t b, int k, c32 v) {
   v = {v.x * a.scale, (a.inverse ? -v.y : v.y) * a.scale};
   if (a.mode == FS_ODD_C2R) {
-    float* out = reinterpret_cast<float*>(a.out);
-    const int64_t c0 = a.pair ? 2 * b : b;
-    out[c0 * a.obs + k] = v.x;
-    if (a.pair && c0 + 1 < a.ncol) out[(c0 + 1) * a.obs + k] = v.y;
+    reinterpret_cast<float*>(a.out)[b * a.obs + k] = v.x;
   } else if (a.mode != FS_ODD_R2C || 2 * k < a.N) {
     a.out[b * a.obs + k] = v;
   }
@@ -381,26 +411,38 @@ __device__ __forceinline__ int64_t xcd_block(int64_t n) {
 // Thread: column c of the block, rows n0 + i dn; a transform's elements are within
 // 2^23 bytes, so one base and 32-bit offsets reach them.  Loads past the edges
 // take the last row or column and are not stored.
-template <int TH>
-__global__ __launch_bounds__(TH, 8) void fs_cols(FsArgs a) {
-  extern __shared__ __align__(16) c32 lds[];  // FS_PER TH elements, the steps, the passes' twiddles
+template <int TH, bool PAIR>
+__device__ __forceinline__ void fs_cols_tile(const FsArgs& a, FsPairOf<PAIR> p, c32* lds, int64_t b, int c0, int half,
+                                             int wide) {
   c32* buf = lds;
   // W_N^{n2 dr i}: with W_N^{n2 n0} of its own, a thread's four-step twiddles
   c32* step = lds + FS_PER * TH;
   c32* tw = step + 16 * FS_PER;
   const int TC = a.T;
   const int lgT = __ffs(TC) - 1;
-  const int tiles = (a.N2 + TC - 1) / TC;
-  const int64_t blk = xcd_block(tiles * a.batch);
-  if (blk < 0) return;
-  const int64_t b = blk / tiles;
-  const int c0 = static_cast<int>(blk % tiles) * TC;
   const int c = static_cast<int>(threadIdx.x) & (TC - 1), r0 = static_cast<int>(threadIdx.x) >> lgT;
   const int dr = TH >> lgT;
   const int col = min(c0 + c, a.N2 - 1);
   // all loads issued before the first LDS store
   c32 v[FS_PER];
-  if (a.mode == FS_C2R) {
+  if constexpr (PAIR) {
+    const bool two = pair_second(p, b, half);  // uniform
+    const c32* A = a.in + (2 * b + half) * a.ibs;
+    const c32* B = A + (two ? a.ibs : 0);
+    c32 w[FS_PER];
+#pragma unroll
+    for (int i = 0; i < FS_PER; ++i) {
+      if (i * dr < a.N1) {
+        const uint32_t k = 8u * static_cast<uint32_t>(odd_bin(col + min(r0 + i * dr, a.N1 - 1) * a.N2, a.N));
+        v[i] = at_byte(A, k);
+        w[i] = at_byte(B, k);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < FS_PER; ++i)
+      if (i * dr < a.N1)
+        v[i] = pair_full(col + min(r0 + i * dr, a.N1 - 1) * a.N2, a.N, v[i], w[i], two && wide == 0);
+  } else if (a.mode == FS_C2R) {
     const c32* X = a.in + b * a.ibs;
     const c32* Xe = X + a.N;
     c32 w[FS_PER];
@@ -437,7 +479,7 @@ __global__ __launch_bounds__(TH, 8) void fs_cols(FsArgs a) {
   __syncthreads();
   fs_dft<TH>(buf, tw, a, a.N1);
   if (c0 + c >= a.N2) return;
-  c32* dst = a.out + b * a.N + c0;
+  c32* dst = a.out + (PAIR ? b + half * a.batch : b) * a.N + c0;
   int k0 = r0;
   asm volatile("" : "+v"(k0));  // keeps the store indices from being computed before the passes
   const c32 w0 = cis_nh(-static_cast<double>((c0 + c) * k0), a.h);
@@ -449,26 +491,39 @@ __global__ __launch_bounds__(TH, 8) void fs_cols(FsArgs a) {
       at_byte(dst, o0 + static_cast<uint32_t>(i) * od) = cmul(at_byte(buf, l0 + 8u * TH * i), cmul(w0, step[i * TC + c]));
 }
 
-// rows: block = (batch b, rows k1 in [r0, r0 + TR)); TR is a power of two.  Rows are
-// interleaved as in fs_cols (element n of row c at n * TR + c), which keeps the
-// passes' LDS accesses as conflict-free as fs_cols's.
-template <int TH>
-__global__ __launch_bounds__(TH, 8) void fs_rows(FsArgs a) {
-  extern __shared__ __align__(16) c32 lds[];  // FS_PER TH elements, the passes' twiddles
-  c32* buf = lds;
-  c32* tw = lds + FS_PER * TH;
-  for (int i = threadIdx.x; i < a.ntw; i += TH) tw[i] = a.tw[i];
-  const int TR = a.T;
-  const int lgT = __ffs(TR) - 1;
-  const int tiles = (a.N1 + TR - 1) / TR;
+template <int TH, bool PAIR>
+__global__ __launch_bounds__(TH, 8) void fs_cols(FsArgs a, FsPairOf<PAIR> p) {
+  extern __shared__ __align__(16) c32 lds[];  // FS_PER TH elements, the steps, the passes' twiddles
+  const int tiles = (a.N2 + a.T - 1) / a.T;
   const int64_t blk = xcd_block(tiles * a.batch);
   if (blk < 0) return;
   const int64_t b = blk / tiles;
-  const int r0 = static_cast<int>(blk % tiles) * TR;
+  const int c0 = static_cast<int>(blk % tiles) * a.T;
+  if constexpr (PAIR) {
+    const int wide = pair_wide(p);
+    fs_cols_tile<TH, true>(a, p, lds, b, c0, 0, wide);
+    if (!pair_second(p, b, 0) || __builtin_amdgcn_readfirstlane(wide) == 0) return;  // uniform
+    __syncthreads();
+    fs_cols_tile<TH, true>(a, p, lds, b, c0, 1, wide);  // a loop over both turns would spill
+  } else {
+    fs_cols_tile<TH, false>(a, p, lds, b, c0, 0, 0);
+  }
+}
+
+// rows: block = (batch b, rows k1 in [r0, r0 + TR)); TR is a power of two.  Rows are
+// interleaved as in fs_cols (element n of row c at n * TR + c), which keeps the
+// passes' LDS accesses as conflict-free as fs_cols's.
+template <int TH, bool PAIR>
+__device__ __forceinline__ void fs_rows_tile(const FsArgs& a, FsPairOf<PAIR> p, c32* lds, int64_t b, int r0, int half,
+                                             int wide) {
+  c32* buf = lds;
+  const c32* tw = lds + FS_PER * TH;
+  const int TR = a.T;
+  const int lgT = __ffs(TR) - 1;
   const int c = static_cast<int>(threadIdx.x) & (TR - 1), n0 = static_cast<int>(threadIdx.x) >> lgT;
   const int dn = TH >> lgT;
   {
-    const c32* src = a.in + b * a.N;
+    const c32* src = a.in + (PAIR ? b + half * a.batch : b) * a.N;
     const int row = min(r0 + c, a.N1 - 1) * a.N2;
     c32 v[FS_PER];
 #pragma unroll
@@ -484,7 +539,13 @@ __global__ __launch_bounds__(TH, 8) void fs_rows(FsArgs a) {
   int k2 = n0;
   asm volatile("" : "+v"(k2));  // keeps the store indices from being computed before the passes
   const uint32_t l0 = 8u * static_cast<uint32_t>(k2 * TR + c);
-  if (a.mode == FS_C2C || a.mode == FS_C2R) {
+  if constexpr (PAIR) {
+    const bool two = wide == 0 && pair_second(p, b, half);
+#pragma unroll
+    for (int i = 0; i < FS_PER; ++i)
+      if (k2 + i * dn < a.N2)
+        pair_output(a, 2 * b + half, two, r0 + c + (k2 + i * dn) * a.N1, at_byte(buf, l0 + 8u * TH * i));
+  } else if (a.mode == FS_C2C || a.mode == FS_C2R) {
     const float sx = a.scale, sy = a.inverse ? -a.scale : a.scale;
     c32* dst = a.out + b * a.obs + r0;
     const uint32_t o0 = 8u * static_cast<uint32_t>(c + k2 * a.N1), od = 8u * static_cast<uint32_t>(dn * a.N1);
@@ -502,11 +563,32 @@ __global__ __launch_bounds__(TH, 8) void fs_rows(FsArgs a) {
   }
 }
 
+template <int TH, bool PAIR>
+__global__ __launch_bounds__(TH, 8) void fs_rows(FsArgs a, FsPairOf<PAIR> p) {
+  extern __shared__ __align__(16) c32 lds[];  // FS_PER TH elements, the passes' twiddles
+  // (their loads are under way during the divisions below)
+  for (int i = threadIdx.x; i < a.ntw; i += TH) lds[FS_PER * TH + i] = a.tw[i];
+  const int tiles = (a.N1 + a.T - 1) / a.T;
+  const int64_t blk = xcd_block(tiles * a.batch);
+  if (blk < 0) return;
+  const int64_t b = blk / tiles;
+  const int r0 = static_cast<int>(blk % tiles) * a.T;
+  if constexpr (PAIR) {
+    const int wide = pair_wide(p);
+    fs_rows_tile<TH, true>(a, p, lds, b, r0, 0, wide);
+    if (!pair_second(p, b, 0) || __builtin_amdgcn_readfirstlane(wide) == 0) return;  // uniform
+    __syncthreads();
+    fs_rows_tile<TH, true>(a, p, lds, b, r0, 1, wide);  // a loop over both turns would spill
+  } else {
+    fs_rows_tile<TH, false>(a, p, lds, b, r0, 0, 0);
+  }
+}
+
 // whole transforms: block = transforms [T blockIdx, T blockIdx + T), element n of
 // transform c at n * T + c; LDS: N * T elements, then the twiddles
-template <int TH>
-__global__ __launch_bounds__(TH, TH == 512 ? 4 : 8) void fs_one(FsArgs a) {
-  extern __shared__ __align__(16) c32 lds[];
+template <bool PAIR>
+__device__ __forceinline__ void fs_one_tile(const FsArgs& a, FsPairOf<PAIR> p, c32* lds, int half, int wide) {
+  constexpr int TH = FS_ONE_TH;
   c32* buf = lds;
   c32* tw = lds + a.N * a.T;
   for (int i = threadIdx.x; i < a.ntw; i += TH) tw[i] = a.tw[i];
@@ -515,37 +597,57 @@ __global__ __launch_bounds__(TH, TH == 512 ? 4 : 8) void fs_one(FsArgs a) {
   const int E = a.N * nt;
   const FsDiv dN = fs_div(a.N);
   {
+    // loads past the last element take it again; one branch on the mode around them
+    // all, so that they are in flight together
     c32 v[FS_PER], w[FS_PER];
+    auto each = [&](auto&& f) {
 #pragma unroll
-    for (int i = 0; i < FS_PER; ++i) {
-      const int e = static_cast<int>(threadIdx.x) + i * TH;
-      const int c = fs_quo(e, dN), n = e - c * a.N;
-      v[i] = w[i] = {0.0f, 0.0f};
-      if (e < E) {
-        if (a.mode == FS_C2R) {
-          const c32* X = a.in + (b0 + c) * a.ibs;
-          v[i] = X[n];
-          w[i] = X[a.N - n];
-        } else {
-          v[i] = fs_input(a, b0 + c, n);
-        }
+      for (int i = 0; i < FS_PER; ++i) {
+        const int e = min(static_cast<int>(threadIdx.x) + i * TH, E - 1);
+        const int c = fs_quo(e, dN), n = e - c * a.N;
+        f(i, b0 + c, n);
       }
+    };
+    if constexpr (PAIR) {
+      each([&](int i, int64_t u, int n) {
+        const c32* A = a.in + min(2 * u + half, p.ncol - 1) * a.ibs + odd_bin(n, a.N);
+        v[i] = A[0];
+        w[i] = A[pair_second(p, u, half) ? a.ibs : 0];
+      });
+      each([&](int i, int64_t u, int n) {
+        v[i] = pair_full(n, a.N, v[i], w[i], wide == 0 && pair_second(p, u, half));
+      });
+    } else if (a.mode == FS_C2R) {
+      each([&](int i, int64_t b, int n) {
+        const c32* X = a.in + b * a.ibs;
+        v[i] = X[n];
+        w[i] = X[a.N - n];
+      });
+      each([&](int i, int64_t, int n) {
+        v[i] = c2r_pack(n, v[i], w[i], cis_nh(-static_cast<double>(n), 0.5 * a.h));
+      });
+    } else if (a.mode == FS_ODD_C2R) {
+      each([&](int i, int64_t b, int n) { v[i] = a.in[b * a.ibs + odd_bin(n, a.N)]; });
+      each([&](int i, int64_t, int n) { v[i] = odd_full(n, a.N, v[i]); });
+    } else if (a.mode == FS_ODD_R2C) {
+      each([&](int i, int64_t b, int n) {
+        v[i] = {reinterpret_cast<const float*>(a.in)[b * a.ibs + n], 0.0f};
+      });
+    } else {
+      each([&](int i, int64_t b, int n) { v[i] = a.in[b * a.ibs + n]; });
     }
 #pragma unroll
     for (int i = 0; i < FS_PER; ++i) {
       const int e = static_cast<int>(threadIdx.x) + i * TH;
       const int c = fs_quo(e, dN), n = e - c * a.N;
-      if (e < E) {
-        if (a.mode == FS_C2R) v[i] = c2r_pack(n, v[i], w[i], cis_nh(-static_cast<double>(n), 0.5 * a.h));
-        buf[n * a.T + c] = {v[i].x, a.inverse ? -v[i].y : v[i].y};
-      }
+      if (e < E) buf[n * a.T + c] = {v[i].x, a.inverse ? -v[i].y : v[i].y};
     }
   }
   __syncthreads();
   fs_dft<TH>(buf, tw, a, a.N);
   int tid = static_cast<int>(threadIdx.x);
   asm volatile("" : "+v"(tid));
-  if (a.mode == FS_R2C) {
+  if (!PAIR && a.mode == FS_R2C) {
     // X[k] = E + W_{2N}^k O, X[N-k] = conj(E - W_{2N}^k O), E = (Z[k] + conj Z[N-k])/2,
     // O = (Z[k] - conj Z[N-k])/(2i)
     const int half = a.N / 2 + 1;
@@ -572,7 +674,29 @@ __global__ __launch_bounds__(TH, TH == 512 ? 4 : 8) void fs_one(FsArgs a) {
   for (int i = 0; i < FS_PER; ++i) {
     const int e = tid + i * TH;
     const int c = fs_quo(e, dN), k = e - c * a.N;
-    if (e < E) fs_output(a, b0 + c, k, buf[k * a.T + c]);
+    if (e < E) {
+      if constexpr (PAIR) {
+        const int64_t u = b0 + c;
+        if (2 * u + half < p.ncol)
+          pair_output(a, 2 * u + half, wide == 0 && pair_second(p, u, half), k, buf[k * a.T + c]);
+      } else {
+        fs_output(a, b0 + c, k, buf[k * a.T + c]);
+      }
+    }
+  }
+}
+
+template <bool PAIR>
+__global__ __launch_bounds__(FS_ONE_TH, 4) void fs_one(FsArgs a, FsPairOf<PAIR> p) {
+  extern __shared__ __align__(16) c32 lds[];
+  if constexpr (PAIR) {
+    const int wide = pair_wide(p);
+    fs_one_tile<true>(a, p, lds, 0, wide);
+    if (__builtin_amdgcn_readfirstlane(wide) == 0) return;  // uniform
+    __syncthreads();
+    fs_one_tile<true>(a, p, lds, 1, wide);
+  } else {
+    fs_one_tile<false>(a, p, lds, 0, 0);
   }
 }
 
@@ -591,17 +715,18 @@ static void fs_passes(FsArgs* a, const std::vector<int>& rad, const c32* tw) {
 }
 
 // `batch` transforms of plan p in mode `mode`; the result is multiplied by
-// scale.  s0: scratch of N * batch elements (four-step only).
+// scale.  s0: scratch of N * batch elements (four-step only).  wide: two real columns
+// a transform (FS_ODD_C2R; batch and s0 count the columns)
 static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void* out, int64_t obs, int64_t batch,
-                  bool inverse, double scale, c32* s0, hipStream_t st, int64_t ncol = 0, bool pair = false) {
+                  bool inverse, double scale, c32* s0, hipStream_t st, const int* wide = nullptr) {
   FsArgs a;
+  const FsPair pr = {batch, wide};
+  if (wide != nullptr) batch = (batch + 1) / 2;
   a.N = static_cast<int>(p->N);
   a.N1 = p->N1;
   a.N2 = p->N2;
   a.inverse = inverse ? 1 : 0;
   a.batch = batch;
-  a.ncol = ncol;
-  a.pair = pair ? 1 : 0;
   a.h = 1.0 / static_cast<double>(p->N);
   const double bytes = 16.0 * static_cast<double>(p->N) * static_cast<double>(batch);
   if (!p->rad0.empty()) {
@@ -618,7 +743,9 @@ static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void*
     fs_passes(&a, p->rad0, p->tw0);
     const size_t lds = (static_cast<size_t>(p->N) * T + a.ntw) * sizeof(c32);
     ProfScope ps(st, "fft_fs_one", bytes);
-    fs_one<512><<<static_cast<unsigned>((batch + T - 1) / T), 512, lds, st>>>(a);
+    const unsigned grid = static_cast<unsigned>((batch + T - 1) / T);
+    if (wide != nullptr) fs_one<true><<<grid, FS_ONE_TH, lds, st>>>(a, pr);
+    else fs_one<false><<<grid, FS_ONE_TH, lds, st>>>(a, {});
     ZDT_CHECK_LAUNCH("fs_one");
     return ZDT_OK;
   }
@@ -645,8 +772,14 @@ static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void*
     fs_passes(&a, p->rad1, p->tw1);
     ProfScope ps(st, mode == FS_C2R ? "fft_fs_cols_c2r" : "fft_fs_cols", bytes);
     const size_t lds = (FS_PER * th + 16 * FS_PER + a.ntw) * sizeof(c32);
-    const auto kern = th == 320 ? fs_cols<320> : th == 512 ? fs_cols<512> : fs_cols<1024>;
-    kern<<<static_cast<unsigned>(grid), th, lds, st>>>(a);
+    const unsigned g = static_cast<unsigned>(grid);
+    if (wide != nullptr) {
+      const auto kern = th == 320 ? fs_cols<320, true> : th == 512 ? fs_cols<512, true> : fs_cols<1024, true>;
+      kern<<<g, th, lds, st>>>(a, pr);
+    } else {
+      const auto kern = th == 320 ? fs_cols<320, false> : th == 512 ? fs_cols<512, false> : fs_cols<1024, false>;
+      kern<<<g, th, lds, st>>>(a, {});
+    }
     ZDT_CHECK_LAUNCH("fs_cols");
   }
   {
@@ -661,8 +794,14 @@ static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void*
     ProfScope ps(st, "fft_fs_rows", bytes);
     const int th = p->N2 * p->TR > 512 * FS_PER ? 1024 : 512;
     const size_t lds = (FS_PER * th + a.ntw) * sizeof(c32);
-    const auto kern = th == 512 ? fs_rows<512> : fs_rows<1024>;
-    kern<<<static_cast<unsigned>(grid), th, lds, st>>>(a);
+    const unsigned g = static_cast<unsigned>(grid);
+    if (wide != nullptr) {
+      const auto kern = th == 512 ? fs_rows<512, true> : fs_rows<1024, true>;
+      kern<<<g, th, lds, st>>>(a, pr);
+    } else {
+      const auto kern = th == 512 ? fs_rows<512, false> : fs_rows<1024, false>;
+      kern<<<g, th, lds, st>>>(a, {});
+    }
     ZDT_CHECK_LAUNCH("fs_rows");
   }
   return ZDT_OK;
@@ -1083,7 +1222,7 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
 }
 
 int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int64_t batch, double scale,
-            void* s0, void* s1, void* s2, hipStream_t st, int maxr, bool pairs) {
+            void* s0, void* s1, void* s2, hipStream_t st, int maxr, const int* wide) {
   if (N % 2 == 0) {
     const int64_t M = N / 2;
     if (ldo % 2 != 0) return fail(ZDT_EINVAL, "c2r: column stride must be even for even N");
@@ -1114,8 +1253,8 @@ int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int6
   const FftPlan* p = nullptr;
   ZDT_TRY(fft_plan_get(N, false, &p, maxr));
   if (fs_has(p))
-    return fs_run(p, FS_ODD_C2R, in, ldi, out, ldo, pairs ? (batch + 1) / 2 : batch, true,
-                  scale / static_cast<double>(N), static_cast<c32*>(s0), st, batch, pairs);
+    return fs_run(p, FS_ODD_C2R, in, ldi, out, ldo, batch, true, scale / static_cast<double>(N),
+                  static_cast<c32*>(s0), st, wide);
   c32* full = static_cast<c32*>(s2);
   hermitian_extend<<<grid_for(N * batch, 256), 256, 0, st>>>(in, ldi, full, N, batch);
   ZDT_CHECK_LAUNCH("hermitian_extend");

@@ -146,6 +146,9 @@ struct zdt_ws {
   // generic path
   c32* F = nullptr;   // Nk x Nt
   c32* Ys = nullptr;  // Nk x Nr
+  // odd Nf: two flags behind Ys, used in turn by the runs (czt_fold, fft_c2r)
+  int* wide = nullptr;
+  int turn = 0;
   void* s[3] = {nullptr, nullptr, nullptr};
   size_t s_bytes = 0;
 
@@ -249,6 +252,9 @@ double out_scale(const zdt_ws* ws) {
 // the chirp-Z can then write past the cache
 int64_t ys_stride(int64_t Nk) { return (Nk + 15) / 16 * 16; }
 
+// bytes of Ys, with the two flags of an odd Nf
+int64_t ys_bytes(int64_t Nf, int64_t Nr) { return ys_stride(Nf / 2 + 1) * Nr * 8 + (Nf % 2 != 0 ? 8 : 0); }
+
 bool use_fast(const zdt_ws* ws) { return ws->fast != nullptr; }
 
 int ensure_stepwise(zdt_ws* ws) {
@@ -292,8 +298,11 @@ int output_impl(zdt_ws* ws, float* dest) {
   if (ws->ys_fout) return fast_output(ws->fout, dest, out_scale(ws), ws->stream);
   if (ws->ys_src == nullptr) return fail(ZDT_ESTATE, "output!: no post-processed spectra (run zdtfdr! or the steps first)");
   ZDT_TRY(ensure_scratch(ws, real_scratch_bytes(ws)));
+  // two rates a transform only for the chirp-Z's own spectra, of which the flag
+  // tells whether one rate's could reach the other's column
+  const int* wide = ws->wide != nullptr && ws->ys_src == ws->Ys ? ws->wide + ws->turn : nullptr;
   return fft_c2r(ws->Nf, ws->ys_src, ws->ys_ld, dest, ws->Nf, ws->Nr, out_scale(ws), ws->s[0], ws->s[1], ws->s[2],
-                 ws->stream, ws->maxr, true);
+                 ws->stream, ws->maxr, wide);
 }
 
 int run_impl(zdt_ws* ws, float r0, int wkind, const float* window, float* dest) {
@@ -332,6 +341,11 @@ int run_impl(zdt_ws* ws, float r0, int wkind, const float* window, float* dest) 
   a.wkind = wkind;
   a.wcustom = window;
   a.scale = 1.0f;
+  a.wide = nullptr;
+  if (ws->wide != nullptr) {
+    ws->turn ^= 1;
+    a.wide = ws->wide + ws->turn;
+  }
   ZDT_TRY(launch_czt(a, ws->stream));
   ws->ys_src = ws->Ys;
   ws->ys_ld = ys_stride(ws->Nk);
@@ -377,7 +391,7 @@ int64_t zdt_workspace_bytes(int64_t Nf, int64_t Nt, int64_t Nr, const int* facto
   if (!(flags & ZDT_FLAG_GENERIC) && fast_out_supported(Nf, Nt, Nr)) return Nk * Nt * 8 + fast_out_bytes(Nf, Nr);
   const int64_t b = std::max(Nt, Nr);
   const int64_t sc = static_cast<int64_t>(fft_real_scratch_elems(Nf, b) * sizeof(c32));
-  return Nk * Nt * 8 + ys_stride(Nk) * Nr * 8 + 3 * sc;
+  return Nk * Nt * 8 + ys_bytes(Nf, Nr) + 3 * sc;
 }
 
 }  // extern "C"
@@ -438,7 +452,11 @@ int create_ws_tuned(const float* spec, int64_t Nf, int64_t Nt, float r0, float d
     } else {
       rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->F), static_cast<size_t>(ws->Nk * Nt) * sizeof(c32));
       if (rc == ZDT_OK)
-        rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->Ys), static_cast<size_t>(ys_stride(ws->Nk) * Nr) * sizeof(c32));
+        rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->Ys), static_cast<size_t>(ys_bytes(Nf, Nr)));
+      if (rc == ZDT_OK && Nf % 2 != 0) {
+        ws->wide = reinterpret_cast<int*>(ws->Ys + ys_stride(ws->Nk) * Nr);
+        rc = launch_set_double(reinterpret_cast<double*>(ws->wide), 0.0, ws->stream);  // both
+      }
       if (rc == ZDT_OK) rc = ensure_scratch(ws, real_scratch_bytes(ws));
     }
     if (rc == ZDT_OK) {

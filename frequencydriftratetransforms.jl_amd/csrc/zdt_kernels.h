@@ -20,12 +20,15 @@ struct CztArgs {
   int64_t ldY;  // Nk x Nr
   int64_t Nk, Nf;
   int Nt, Nr;
+  int wkind;
+  float scale;
+  const float* wcustom;
   double hd;  // dr/(2 Nf): chirp(k,l) = exp(-2 pi i k l^2 hd)
   double hc;  // rc/Nf, rc = r0 + (Nr-1) dr/2 the centre rate
   double hz;  // (r0 - rc)/Nf
-  int wkind;
-  const float* wcustom;
-  float scale;
+  // NULL, or the flag that fft_c2r takes (see czt_fold), one of two in an 8-byte
+  // word; the other is that of the next run
+  int* wide;
 };
 
 // F -> Ys by czt_fold

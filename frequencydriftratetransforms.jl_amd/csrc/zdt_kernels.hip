@@ -65,6 +65,10 @@ __device__ __forceinline__ float window_value(int wkind, const float* wcustom, i
 // kernels this replaced waited for each and reread Ys for every 64 steps past
 // the first (4096 x 16 x 33 11.2 -> 7.5 us, 4096 x 60 x 257 130 -> 23, 2^15 x 177 x
 // 394 611 -> 118, 21609 x 234 x 205 465 -> 66).
+//
+// Odd Nf, whose c2r takes two rates a transform: *a.wide tells that values come
+// near overflow or are not finite, so that the c2r keeps the rates apart;
+// the flag of the run after this one is cleared.
 template <int NB, int NC>
 __global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold(CztArgs a, int tbase, int past) {
   constexpr int BPB = 256 / NC;  // bins per block
@@ -78,10 +82,13 @@ __global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold(CztArgs a, int 
   b.o = static_cast<unsigned>(k);
   b.kd = static_cast<double>(k);
   b.w = window_value(a.wkind, a.wcustom, k, a.Nf) * a.scale;
+  b.wide = a.wide;
   const FoldRates r = {a.Nt, a.Nr, 2.0 * a.hd, a.hc, a.hz};
   const int npair = (a.Nr + 1) / 2;
-  fold_rates<NB, NC>(b, r, threadIdx.x % NC, tbase, group_first(npair, blockIdx.y, gridDim.y),
-                     group_first(npair, blockIdx.y + 1, gridDim.y), tbase > 0, past != 0);
+  fold_rates<NB, NC, true>(b, r, threadIdx.x % NC, tbase, group_first(npair, blockIdx.y, gridDim.y),
+                           group_first(npair, blockIdx.y + 1, gridDim.y), tbase > 0, past != 0);
+  if (a.wide != nullptr && k == 0 && blockIdx.y == 0 && threadIdx.x == 0)
+    *reinterpret_cast<int*>(reinterpret_cast<uintptr_t>(a.wide) ^ 4) = 0;
 }
 
 int launch_czt(const CztArgs& a, hipStream_t st) {
