@@ -8,6 +8,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -163,11 +164,14 @@ struct zdt_ws {
   FastPlan* fout = nullptr;
   c32* Ft = nullptr;  // its input spectrum, Nk x Nt entries in the transposed layout
   bool ys_fout = false;  // last run left its spectra in fout
-  // fftfdr from Ft: its own spectra, for up to rates_cap rates at a time
-  FastPlan* rates = nullptr;
-  int64_t rates_cap = 0;
-  void* Yr = nullptr;  // fftfdr's spectra on the generic path, up to FFTFDR_KEEP with their scratch
-  size_t Yr_bytes = 0;
+  // fftfdr's spectra and scratch, kept for calls on the stream they were made for
+  // (rates_buffer); outgrown ones stay too, for graphs that were captured with them
+  std::mutex rates_mu;
+  hipStream_t rates_stream = nullptr;
+  void* rates = nullptr;
+  size_t rates_bytes = 0;
+  void* rates_old[48] = {};
+  int rates_nold = 0;
 
   bool have_input = false;
   const c32* ys_src = nullptr;  // post-processed spectra for zdt_output
@@ -557,8 +561,8 @@ int zdt_destroy(zdt_ws* ws) {
   for (int i = 0; i < 3; ++i) dev_free(ws->s[i]);
   if (ws->fast) fast_destroy(ws->fast);
   if (ws->fout) fast_destroy(ws->fout);
-  fast_destroy(ws->rates);
-  dev_free(ws->Yr);
+  dev_free(ws->rates);
+  for (int i = 0; i < ws->rates_nold; ++i) dev_free(ws->rates_old[i]);
   delete ws->prof;
   delete ws;
   return ZDT_OK;
@@ -725,6 +729,32 @@ struct AsyncBufs {
 // bytes of spectra and scratch that fftfdr keeps on the generic path
 static constexpr size_t FFTFDR_KEEP = size_t(256) << 20;
 
+// `bytes` for one fftfdr call.  Up to `keep` of them stay with the workspace:
+// allocated and given back by every call they cost a caller that waits for its
+// result 900 us a time.  They serve one stream, whose order keeps a call's kernels
+// from the next one's; calls on another stream, and a capture that finds too few,
+// take theirs from the stream's pool.  A larger buffer is at least twice the one it
+// replaces, so that all of them hold at most twice `keep`.
+static int rates_buffer(zdt_ws* ws, size_t bytes, size_t keep, AsyncBufs& tmp, void** out) {
+  if (bytes > keep || (ws->rates != nullptr && ws->rates_stream != ws->stream)) return tmp.get(out, bytes);
+  if (ws->rates_bytes < bytes) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ws->stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      return tmp.get(out, bytes);
+    }
+    const size_t n = std::min(keep, std::max(bytes, 2 * ws->rates_bytes));
+    void* p = nullptr;
+    ZDT_TRY(dev_alloc(ws, &p, n));
+    if (ws->rates != nullptr) ws->rates_old[ws->rates_nold++] = ws->rates;
+    ws->rates = p;
+    ws->rates_bytes = n;
+    ws->rates_stream = ws->stream;
+  }
+  *out = ws->rates;
+  return ZDT_OK;
+}
+
 int zdt_fftfdr(zdt_ws* ws, const float* rates, int64_t nrates, float* dest) {
   ZDT_TRY(check_ws(ws));
   ProfInstall prof_(ws);
@@ -738,59 +768,33 @@ int zdt_fftfdr(zdt_ws* ws, const float* rates, int64_t nrates, float* dest) {
     if (!std::isfinite(rates[j])) return fail(ZDT_EINVAL, "fftfdr!: rate %lld is not finite", (long long)j);
     rh[static_cast<size_t>(j)] = static_cast<double>(rates[j]) / static_cast<double>(ws->Nf);
   }
+  std::lock_guard<std::mutex> lk(ws->rates_mu);
+  AsyncBufs tmp(ws->stream);
+  void* buf = nullptr;
   if (ws->fout != nullptr) {
-    // The spectra stay with the workspace: allocated and given back by every call
-    // they cost a caller that waits for its result 900 us a time.  2^18 x 16 x 64, whole
-    // calls back to back: 180 us on the generic kernels -> 98 (input 22, czt_rates 25,
-    // k2_c2r 26, k3 29)
-    const int64_t cap = std::min(nrates, fast_rates_chunk(ws->Nf));
-    if (ws->rates_cap < cap) {
-      fast_destroy(ws->rates);
-      ws->rates = nullptr;
-      if (ws->rates_cap > 0) ws->bytes -= fast_out_bytes(ws->Nf, ws->rates_cap);
-      ws->rates_cap = 0;
-      ZDT_TRY(fast_out_create(ws->Nf, cap, ZDT_PRECISION_FP32, &ws->rates));
-      ws->rates_cap = cap;
-      ws->bytes += fast_out_bytes(ws->Nf, cap);
-    }
-    return fast_out_rates(ws->rates, ws->Ft, static_cast<int>(ws->Nt), rh.data(), nrates, dest, ws->stream);
+    // 2^18 x 16 x 64, whole calls back to back: 180 us on the generic kernels -> 98
+    // (input 22, czt_rates 25, k2_c2r 26, k3 29)
+    const int64_t most = fast_rates_chunk(ws->Nf), n = std::min(nrates, most);
+    ZDT_TRY(rates_buffer(ws, fast_rates_bytes(ws->Nf, n), fast_rates_bytes(ws->Nf, most), tmp, &buf));
+    return fast_out_rates(ws->fout, buf, n, ws->Ft, static_cast<int>(ws->Nt), rh.data(), nrates, dest, ws->stream);
   }
   ZDT_TRY(ensure_F_natural(ws));
-  AsyncBufs tmp(ws->stream);
-  void *Y = nullptr, *s0 = nullptr, *s1 = nullptr, *s2 = nullptr;
-  const size_t sc = fft_real_scratch_elems(ws->Nf, nrates) * sizeof(c32);
-  const size_t yb = static_cast<size_t>(ws->Nk * nrates) * sizeof(c32);
-  if (yb + 3 * sc <= FFTFDR_KEEP) {
-    ZDT_TRY(ensure_scratch(ws, sc));
-    if (ws->Yr_bytes < yb) {
-      dev_free(ws->Yr);
-      ws->bytes -= static_cast<int64_t>(ws->Yr_bytes);
-      ws->Yr_bytes = 0;
-      ZDT_TRY(dev_alloc(ws, &ws->Yr, yb));
-      ws->Yr_bytes = yb;
-    }
-    Y = ws->Yr;
-    s0 = ws->s[0];
-    s1 = ws->s[1];
-    s2 = ws->s[2];
-  } else {
-    ZDT_TRY(tmp.get(&Y, yb));
-    ZDT_TRY(tmp.get(&s0, sc));
-    ZDT_TRY(tmp.get(&s1, sc));
-    ZDT_TRY(tmp.get(&s2, sc));
-  }
+  const size_t sc = (fft_real_scratch_elems(ws->Nf, nrates) * sizeof(c32) + 255) / 256 * 256;
+  const size_t yb = (static_cast<size_t>(ws->Nk * nrates) * sizeof(c32) + 255) / 256 * 256;
+  ZDT_TRY(rates_buffer(ws, yb + 3 * sc, FFTFDR_KEEP, tmp, &buf));
+  char* Y = static_cast<char*>(buf);
+  char *s0 = Y + yb, *s1 = s0 + sc, *s2 = s1 + sc;
   CztRatesArgs c;
   c.F = ws->F;
   c.fs = ws->Nk;
-  c.Ys = static_cast<c32*>(Y);
+  c.Ys = reinterpret_cast<c32*>(Y);
   c.ys = ws->Nk;
   c.n = ws->Nk;
   c.logN1 = c.logN2 = 0;
   c.yM = nullptr;
   c.Nt = static_cast<int>(ws->Nt);
   ZDT_TRY(launch_czt_rates(c, rh.data(), nrates, ws->stream));
-  ZDT_TRY(fft_c2r(ws->Nf, static_cast<const c32*>(Y), ws->Nk, dest, ws->Nf, nrates, 1.0, s0, s1, s2, ws->stream,
-                  ws->maxr));
+  ZDT_TRY(fft_c2r(ws->Nf, c.Ys, ws->Nk, dest, ws->Nf, nrates, 1.0, s0, s1, s2, ws->stream, ws->maxr));
   return ZDT_OK;
 }
 

@@ -54,9 +54,11 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
                  double scale, hipStream_t st, double* colmean = nullptr, double* colvar = nullptr);
 
 // fftfdr over a list of rates (rates_over_nf: host, Nr values) from the same Ft, in
-// pieces of the plan's Nr; fast_rates_chunk: the most rates a plan for it needs
+// pieces of n rates, in FP32 whatever p's precision.  buf: fast_rates_bytes(Nf, n) of
+// device memory; fast_rates_chunk: the most rates a piece should have
 int64_t fast_rates_chunk(int64_t Nf);
-int fast_out_rates(FastPlan* p, const c32* F, int Nt, const double* rates_over_nf, int64_t Nr, float* dest,
-                   hipStream_t st);
+size_t fast_rates_bytes(int64_t Nf, int64_t n);
+int fast_out_rates(const FastPlan* p, void* buf, int64_t n, const c32* F, int Nt, const double* rates_over_nf,
+                   int64_t Nr, float* dest, hipStream_t st);
 
 }  // namespace zdt

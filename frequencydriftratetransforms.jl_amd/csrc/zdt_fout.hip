@@ -804,34 +804,45 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
 
 int64_t fast_rates_chunk(int64_t Nf) { return std::max<int64_t>(1, FOUT_CHUNK / (4 * Nf)); }
 
-int fast_out_rates(FastPlan* p, const c32* F, int Nt, const double* rates_over_nf, int64_t Nr, float* dest,
-                   hipStream_t st) {
-  // chunks whose spectra B stay in the last-level cache, as in fast_out_run
-  for (int64_t j0 = 0; j0 < Nr; j0 += p->Nr) {
-    const int64_t n = std::min(p->Nr, Nr - j0);
+size_t fast_rates_bytes(int64_t Nf, int64_t n) { return static_cast<size_t>(n * (Nf + 2)) * sizeof(c32); }
+
+int fast_out_rates(const FastPlan* p, void* buf, int64_t n, const c32* F, int Nt, const double* rates_over_nf,
+                   int64_t Nr, float* dest, hipStream_t st) {
+  // p's shape and tables, buf's spectra
+  FastPlan q = *p;
+  q.precision = ZDT_PRECISION_FP32;
+  q.paired = false;
+  q.smax = nullptr;
+  q.Yc = static_cast<c32*>(buf);
+  q.B = q.Yc + n * q.M;
+  q.yM = q.B + n * q.M;
+  q.yhalf = q.yM + n;
+  // pieces whose spectra B stay in the last-level cache, as in fast_out_run
+  for (int64_t j0 = 0; j0 < Nr; j0 += n) {
+    const int64_t m = std::min(n, Nr - j0);
     CztRatesArgs c;
     c.F = F;
-    c.fs = p->M;
-    c.Ys = p->Yc;
-    c.ys = p->M;
-    c.n = p->M;
-    c.logN1 = p->logN1;
-    c.logN2 = p->logN2;
-    c.yM = p->yM;
+    c.fs = q.M;
+    c.Ys = q.Yc;
+    c.ys = q.M;
+    c.n = q.M;
+    c.logN1 = q.logN1;
+    c.logN2 = q.logN2;
+    c.yM = q.yM;
     c.Nt = Nt;
-    ZDT_TRY(launch_czt_rates(c, rates_over_nf + j0, n, st));
+    ZDT_TRY(launch_czt_rates(c, rates_over_nf + j0, m, st));
     K2cArgs a;
-    a.Yc = p->Yc;
-    a.yM = p->yM;
-    a.B = p->B;
-    a.yhalf = p->yhalf;
-    a.tw1 = p->tw1;
-    a.Nr = static_cast<int>(n);
-    a.M = p->M;
-    a.Nf = p->Nf;
-    a.oscale = static_cast<float>(1.0 / static_cast<double>(p->M));
-    ZDT_TRY(run_k2c(p, a, st));
-    ZDT_TRY(fast_output_part(p, dest + j0 * p->Nf, 0, n, st, false));
+    a.Yc = q.Yc;
+    a.yM = q.yM;
+    a.B = q.B;
+    a.yhalf = q.yhalf;
+    a.tw1 = q.tw1;
+    a.Nr = static_cast<int>(m);
+    a.M = q.M;
+    a.Nf = q.Nf;
+    a.oscale = static_cast<float>(1.0 / static_cast<double>(q.M));
+    ZDT_TRY(run_k2c(&q, a, st));
+    ZDT_TRY(fast_output_part(&q, dest + j0 * q.Nf, 0, m, st, false));
   }
   return ZDT_OK;
 }
