@@ -71,8 +71,11 @@ __global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold_col(CztColArgs 
   b.kd = static_cast<double>(k);
   b.w = fast_window(a.wkind, a.wcustom, k, a.Nf) * a.scale;
   const int npair = (a.r.Nr + 1) / 2;
-  fold_rates<NB, NC>(b, a.r, q, 0, group_first(npair, blockIdx.y, gridDim.y),
-                     group_first(npair, blockIdx.y + 1, gridDim.y), false, a.past != 0);
+  const int jlo = group_first(npair, blockIdx.y, gridDim.y), jhi = group_first(npair, blockIdx.y + 1, gridDim.y);
+  if constexpr (NB == 0)
+    short_rates<false>(b, a.r, jlo, jhi, a.past != 0);
+  else
+    fold_rates<NB, NC>(b, a.r, q, 0, jlo, jhi, false, a.past != 0);
   // the Nyquist bin, a wavefront per rate over all blocks (a block of its own
   // would cost a whole round where the others fill the chip exactly)
   const int lane = threadIdx.x & 63, nw = 4 * gridDim.x * gridDim.y;
@@ -767,7 +770,7 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
   c.r = {Nt, static_cast<int>(p->Nr), static_cast<double>(dr) / nf, rc / nf, (static_cast<double>(r0) - rc) / nf};
   {
     int nb = 0, nc = 0;
-    fold_split(Nt, &nb, &nc);
+    fold_split(Nt, 0, &nb, &nc);
     // (Yc in rate chunks is read past the cache too: see below)
     c.past = fold_past(8 * p->M * p->Nr, nb) || chunked ? 1 : 0;
     const int bpb = 256 / nc;  // bins per block

@@ -85,8 +85,11 @@ __global__ __launch_bounds__(256, NB <= 4 ? 3 : 2) void czt_fold(CztArgs a, int 
   b.wide = a.wide;
   const FoldRates r = {a.Nt, a.Nr, 2.0 * a.hd, a.hc, a.hz};
   const int npair = (a.Nr + 1) / 2;
-  fold_rates<NB, NC, true>(b, r, threadIdx.x % NC, tbase, group_first(npair, blockIdx.y, gridDim.y),
-                           group_first(npair, blockIdx.y + 1, gridDim.y), tbase > 0, past != 0);
+  const int jlo = group_first(npair, blockIdx.y, gridDim.y), jhi = group_first(npair, blockIdx.y + 1, gridDim.y);
+  if constexpr (NB == 0)
+    short_rates<true>(b, r, jlo, jhi, past != 0);
+  else
+    fold_rates<NB, NC, true>(b, r, threadIdx.x % NC, tbase, jlo, jhi, tbase > 0, past != 0);
   if (a.wide != nullptr && k == 0 && blockIdx.y == 0 && threadIdx.x == 0)
     *reinterpret_cast<int*>(reinterpret_cast<uintptr_t>(a.wide) ^ 4) = 0;
 }
@@ -97,7 +100,7 @@ int launch_czt(const CztArgs& a, hipStream_t st) {
   ProfScope ps(st, "czt_fold", 8.0 * static_cast<double>(a.Nk) * (a.Nt + a.Nr));
   for (int tbase = 0; tbase < a.Nt; tbase += FOLD_MAX_NT) {
     int nb = 0, nc = 0;
-    fold_split(a.Nt - tbase, &nb, &nc);
+    fold_split(a.Nt, tbase, &nb, &nc);
     const int per = 256 / nc;
     const int nblk = static_cast<int>((a.Nk + per - 1) / per);
     // (whole cache lines: a 128-byte aligned destination and column stride)
