@@ -164,7 +164,7 @@ struct zdt_ws {
   FastPlan* fout = nullptr;
   c32* Ft = nullptr;  // its input spectrum, Nk x Nt entries in the transposed layout
   bool ys_fout = false;  // last run left its spectra in fout
-  // fftfdr's spectra and scratch, kept for calls on the stream they were made for
+  // fftfdr's and fdshift's spectra and scratch, kept for calls on the stream they were made for
   // (rates_buffer); outgrown ones stay too, for graphs that were captured with them
   std::mutex rates_mu;
   hipStream_t rates_stream = nullptr;
@@ -726,10 +726,10 @@ struct AsyncBufs {
 };
 }  // namespace
 
-// bytes of spectra and scratch that fftfdr keeps on the generic path
+// bytes of spectra and scratch that fftfdr and fdshift keep on the generic path
 static constexpr size_t FFTFDR_KEEP = size_t(256) << 20;
 
-// `bytes` for one fftfdr call.  Up to `keep` of them stay with the workspace:
+// `bytes` for one fftfdr or fdshift call.  Up to `keep` of them stay with the workspace:
 // allocated and given back by every call they cost a caller that waits for its
 // result 900 us a time.  They serve one stream, whose order keeps a call's kernels
 // from the next one's; calls on another stream, and a capture that finds too few,
@@ -752,6 +752,21 @@ static int rates_buffer(zdt_ws* ws, size_t bytes, size_t keep, AsyncBufs& tmp, v
     ws->rates_stream = ws->stream;
   }
   *out = ws->rates;
+  return ZDT_OK;
+}
+
+// n columns of spectra and the c2r's scratch for them, on the generic kernels
+struct ShiftBufs {
+  c32* Y;
+  void* s[3];
+};
+static int shift_bufs(zdt_ws* ws, int64_t n, AsyncBufs& tmp, ShiftBufs* b) {
+  const size_t sc = (fft_real_scratch_elems(ws->Nf, n) * sizeof(c32) + 255) / 256 * 256;
+  const size_t yb = (static_cast<size_t>(ws->Nk * n) * sizeof(c32) + 255) / 256 * 256;
+  void* buf = nullptr;
+  ZDT_TRY(rates_buffer(ws, yb + 3 * sc, FFTFDR_KEEP, tmp, &buf));
+  b->Y = static_cast<c32*>(buf);
+  for (int i = 0; i < 3; ++i) b->s[i] = static_cast<char*>(buf) + yb + i * sc;
   return ZDT_OK;
 }
 
@@ -779,22 +794,19 @@ int zdt_fftfdr(zdt_ws* ws, const float* rates, int64_t nrates, float* dest) {
     return fast_out_rates(ws->fout, buf, n, ws->Ft, static_cast<int>(ws->Nt), rh.data(), nrates, dest, ws->stream);
   }
   ZDT_TRY(ensure_F_natural(ws));
-  const size_t sc = (fft_real_scratch_elems(ws->Nf, nrates) * sizeof(c32) + 255) / 256 * 256;
-  const size_t yb = (static_cast<size_t>(ws->Nk * nrates) * sizeof(c32) + 255) / 256 * 256;
-  ZDT_TRY(rates_buffer(ws, yb + 3 * sc, FFTFDR_KEEP, tmp, &buf));
-  char* Y = static_cast<char*>(buf);
-  char *s0 = Y + yb, *s1 = s0 + sc, *s2 = s1 + sc;
+  ShiftBufs b;
+  ZDT_TRY(shift_bufs(ws, nrates, tmp, &b));
   CztRatesArgs c;
   c.F = ws->F;
   c.fs = ws->Nk;
-  c.Ys = reinterpret_cast<c32*>(Y);
+  c.Ys = b.Y;
   c.ys = ws->Nk;
   c.n = ws->Nk;
   c.logN1 = c.logN2 = 0;
   c.yM = nullptr;
   c.Nt = static_cast<int>(ws->Nt);
   ZDT_TRY(launch_czt_rates(c, rh.data(), nrates, ws->stream));
-  ZDT_TRY(fft_c2r(ws->Nf, c.Ys, ws->Nk, dest, ws->Nf, nrates, 1.0, s0, s1, s2, ws->stream, ws->maxr));
+  ZDT_TRY(fft_c2r(ws->Nf, b.Y, ws->Nk, dest, ws->Nf, nrates, 1.0, b.s[0], b.s[1], b.s[2], ws->stream, ws->maxr));
   return ZDT_OK;
 }
 
@@ -805,17 +817,13 @@ int zdt_fdshift(zdt_ws* ws, float rate, float* dest) {
   ZDT_TRY(set_device(ws));
   if (!ws->have_input) return fail(ZDT_ESTATE, "fdshift!: no input");
   ZDT_TRY(ensure_F_natural(ws));
+  std::lock_guard<std::mutex> lk(ws->rates_mu);
   AsyncBufs tmp(ws->stream);
-  void *Y = nullptr, *s0 = nullptr, *s1 = nullptr, *s2 = nullptr;
-  const size_t sc = fft_real_scratch_elems(ws->Nf, ws->Nt) * sizeof(c32);
-  ZDT_TRY(tmp.get(&Y, static_cast<size_t>(ws->Nk * ws->Nt) * sizeof(c32)));
-  ZDT_TRY(tmp.get(&s0, sc));
-  ZDT_TRY(tmp.get(&s1, sc));
-  ZDT_TRY(tmp.get(&s2, sc));
-  ZDT_TRY(launch_shift_phase(ws->F, ws->Nk, static_cast<c32*>(Y), ws->Nk, ws->Nk, static_cast<int>(ws->Nt),
+  ShiftBufs b;
+  ZDT_TRY(shift_bufs(ws, ws->Nt, tmp, &b));
+  ZDT_TRY(launch_shift_phase(ws->F, ws->Nk, b.Y, ws->Nk, ws->Nk, static_cast<int>(ws->Nt),
                              static_cast<double>(rate) / static_cast<double>(ws->Nf), ws->stream));
-  ZDT_TRY(fft_c2r(ws->Nf, static_cast<const c32*>(Y), ws->Nk, dest, ws->Nf, ws->Nt, 1.0, s0, s1, s2, ws->stream,
-                  ws->maxr));
+  ZDT_TRY(fft_c2r(ws->Nf, b.Y, ws->Nk, dest, ws->Nf, ws->Nt, 1.0, b.s[0], b.s[1], b.s[2], ws->stream, ws->maxr));
   return ZDT_OK;
 }
 

@@ -1,4 +1,4 @@
-"""The spectra that fftfdr keeps with the workspace: captured graphs of the
+"""The spectra that fftfdr and fdshift keep with the workspace: captured graphs of the
 workspace outlive later calls with more rates, and calls on another stream do not
 share them.  Power-of-two lengths (the fused output's kernels) and others (the
 generic ones)."""
@@ -94,6 +94,7 @@ def test_graph_of_fftfdr(F, Nf):
     def between():
         n = next(more)
         F.fftfdr_(F.create_fdr(s, n), ws, rates_of(n, n))
+        F.fdshift(ws, 0.5)
 
     replays(g, dest, want, between)
     assert ws.ws.nbytes - size0 <= 2 * (480 << 20)
@@ -121,3 +122,17 @@ def test_two_streams(F, Nf):
     torch.cuda.synchronize()
     for d, w in zip(dest, want):
         assert torch.equal(d, w)
+
+
+# fdshift! between fftfdr! calls, in the same buffer
+@pytest.mark.parametrize("Nf", [6000, 9375, 1 << 16])
+def test_fdshift_beside_fftfdr(F, Nf):
+    import torch
+    s = spec(Nf, 12, 4)
+    ws, ws2 = F.fftfdr_workspace(s), F.fftfdr_workspace(s)
+    want = F.fdshift(ws2, 1.25)
+    for n in (3, 90, 5):
+        fdr = F.fftfdr(ws, rates_of(n, n))
+        sh = F.fdshift(ws, 1.25)
+        assert torch.equal(sh, want)
+        assert torch.equal(fdr, F.fftfdr(F.fftfdr_workspace(s), rates_of(n, n)))
