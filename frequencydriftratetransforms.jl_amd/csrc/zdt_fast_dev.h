@@ -281,41 +281,6 @@ __device__ __forceinline__ void cf_stage2(c32 (&y)[R1], const c32* ex, int c, in
   }
 }
 
-// The column FFT with the exchange taken in two halves, the real parts and
-// then the imaginary ones, through one plane of floats: half the LDS, so that
-// two blocks share a CU and one computes while the other waits for memory.
-template <int R1>
-struct CH {
-  static constexpr int N2 = 32 * R1;
-  static constexpr int THREADS = 16 * R1;
-  static constexpr int PITCH = R1 * 16 + 16;  // floats per m' slab ([r][c] + pad)
-  static constexpr int LDS = 32 * PITCH;
-  static constexpr int MPER = 32 / R1;
-};
-
-// x (rows r + R1 m, already transformed over m and twiddled) -> y[h][r'] for
-// m' = r + R1 h: the exchanged rows r' of slab m'
-template <int R1>
-__device__ __forceinline__ void ch_exchange(const c32 (&x)[32], c32 (&y)[32], float* ex, int r, int c) {
-  using C = CH<R1>;
-#pragma unroll
-  for (int m = 0; m < 32; ++m) ex[m * C::PITCH + r * 16 + c] = x[m].x;
-  __syncthreads();
-#pragma unroll
-  for (int h = 0; h < C::MPER; ++h)
-#pragma unroll
-    for (int q = 0; q < R1; ++q) y[h * R1 + q].x = ex[(r + R1 * h) * C::PITCH + q * 16 + c];
-  __syncthreads();
-#pragma unroll
-  for (int m = 0; m < 32; ++m) ex[m * C::PITCH + r * 16 + c] = x[m].y;
-  __syncthreads();
-#pragma unroll
-  for (int h = 0; h < C::MPER; ++h)
-#pragma unroll
-    for (int q = 0; q < R1; ++q) y[h * R1 + q].y = ex[(r + R1 * h) * C::PITCH + q * 16 + c];
-  __syncthreads();
-}
-
 template <int N>
 __device__ __forceinline__ void cf_load_twiddles(c32* twl, const c32* __restrict__ tw, int nthreads) {
   for (int i = threadIdx.x; i < N; i += nthreads) twl[i] = tw[i];
