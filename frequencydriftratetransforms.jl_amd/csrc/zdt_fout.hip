@@ -805,6 +805,9 @@ int fast_out_run(FastPlan* p, const c32* F, int Nt, float r0, float dr, int wkin
   return ZDT_OK;
 }
 
+// Each piece reads F again: 64 rates of 16 steps in one piece take 1171 us where
+// 14 at a time take 1387 (2^22), 595 against 640 (2^21), and 128 rates 572 against 551
+// (2^20).  Above 2^20 the bound is for the memory kept, 470 MB.
 int64_t fast_rates_chunk(int64_t Nf) { return std::max<int64_t>(1, FOUT_CHUNK / (4 * Nf)); }
 
 size_t fast_rates_bytes(int64_t Nf, int64_t n) { return static_cast<size_t>(n * (Nf + 2)) * sizeof(c32); }
