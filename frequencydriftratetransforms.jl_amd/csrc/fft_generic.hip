@@ -164,7 +164,7 @@ static int pow2_floor(int64_t x) {
 // (us): Nf = 10^6, 129 rates (1.03 GB through fs_cols, as much through fs_rows)
 // c2r columns 403 -> 305, rows 374 -> 278; r2c columns 59 -> 40.  Odd Nf = 99225, 77
 // rates, two columns a transform instead of a zero imaginary part: 86 + 70 + 40
-// for filling in the Hermitian half and taking the real part -> 44 + 43.  Nf =
+// for filling in the Hermitian half and taking the real part -> 39 + 42.  Nf =
 // 4096, 33 rates: six launches of 5 to 6 -> two, 17 together (fs_one).  Of that, 8
 // elements a thread and 1024 threads: c2r columns 318 -> 305; 32-bit offsets and
 // wave-uniform strides in place of an index per access (112 -> 76 vector
