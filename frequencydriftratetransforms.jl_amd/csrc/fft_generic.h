@@ -48,10 +48,10 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
 
 // Complex-to-real inverse: the normalized inverse (1/N) times `scale`; the imaginary
 // parts of the DC and (even N) Nyquist bins are ignored.  wide: NULL, or a device
-// flag: while it is 0, odd N transforms two columns as the real and imaginary part
+// word: while it is 0, odd N transforms two columns as the real and imaginary part
 // of one, whose values must then be finite and below 2^96 (else one column's reach
 // the other).
 int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int64_t batch, double scale,
-            void* s0, void* s1, void* s2, hipStream_t st, int maxr = 16, const int* wide = nullptr);
+            void* s0, void* s1, void* s2, hipStream_t st, int maxr = 16, const int64_t* wide = nullptr);
 
 }  // namespace zdt

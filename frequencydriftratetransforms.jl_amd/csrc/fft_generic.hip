@@ -207,7 +207,7 @@ struct FsArgs {
 // 16 bytes more of arguments cost a 6 to 9 us kernel 0.2 us
 struct FsPair {
   int64_t ncol;
-  const int* wide;  // not 0: one column a transform after all
+  const int64_t* wide;  // not 0: one column a transform after all
 };
 struct FsNoPair {};
 template <bool PAIR>
@@ -368,7 +368,7 @@ __device__ __forceinline__ bool pair_second(const FsPair& p, int64_t b, int half
 __device__ __forceinline__ int pair_wide(const FsPair& p) {
   int lane0 = 0;
   asm volatile("" : "+v"(lane0));
-  return p.wide[lane0];
+  return p.wide[lane0] != 0 ? 1 : 0;
 }
 
 // element n of the pair's spectrum, A + i B, from its bins in the two columns
@@ -718,7 +718,7 @@ static void fs_passes(FsArgs* a, const std::vector<int>& rad, const c32* tw) {
 // scale.  s0: scratch of N * batch elements (four-step only).  wide: two real columns
 // a transform (FS_ODD_C2R; batch and s0 count the columns)
 static int fs_run(const FftPlan* p, int mode, const void* in, int64_t ibs, void* out, int64_t obs, int64_t batch,
-                  bool inverse, double scale, c32* s0, hipStream_t st, const int* wide = nullptr) {
+                  bool inverse, double scale, c32* s0, hipStream_t st, const int64_t* wide = nullptr) {
   FsArgs a;
   const FsPair pr = {batch, wide};
   if (wide != nullptr) batch = (batch + 1) / 2;
@@ -1239,7 +1239,7 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
 }
 
 int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int64_t batch, double scale,
-            void* s0, void* s1, void* s2, hipStream_t st, int maxr, const int* wide) {
+            void* s0, void* s1, void* s2, hipStream_t st, int maxr, const int64_t* wide) {
   if (N % 2 == 0) {
     const int64_t M = N / 2;
     if (ldo % 2 != 0) return fail(ZDT_EINVAL, "c2r: column stride must be even for even N");

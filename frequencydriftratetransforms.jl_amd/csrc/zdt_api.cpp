@@ -302,9 +302,10 @@ int output_impl(zdt_ws* ws, float* dest) {
   if (ws->ys_fout) return fast_output(ws->fout, dest, out_scale(ws), ws->stream);
   if (ws->ys_src == nullptr) return fail(ZDT_ESTATE, "output!: no post-processed spectra (run zdtfdr! or the steps first)");
   ZDT_TRY(ensure_scratch(ws, real_scratch_bytes(ws)));
-  // two rates a transform only for the chirp-Z's own spectra, of which the flag
-  // tells whether one rate's could reach the other's column
-  const int* wide = ws->wide != nullptr && ws->ys_src == ws->Ys ? ws->wide + ws->turn : nullptr;
+  // two rates a transform only for the chirp-Z's own spectra, of which the flags
+  // tell whether one rate's could reach the other's column.  Both: the last run may
+  // have been a captured one's replay, which this workspace's turn does not follow
+  const int64_t* wide = ws->ys_src == ws->Ys ? reinterpret_cast<const int64_t*>(ws->wide) : nullptr;
   return fft_c2r(ws->Nf, ws->ys_src, ws->ys_ld, dest, ws->Nf, ws->Nr, out_scale(ws), ws->s[0], ws->s[1], ws->s[2],
                  ws->stream, ws->maxr, wide);
 }

@@ -26,8 +26,8 @@ struct CztArgs {
   double hd;  // dr/(2 Nf): chirp(k,l) = exp(-2 pi i k l^2 hd)
   double hc;  // rc/Nf, rc = r0 + (Nr-1) dr/2 the centre rate
   double hz;  // (r0 - rc)/Nf
-  // NULL, or the flag that fft_c2r takes (see czt_fold), one of two in an 8-byte
-  // word; the other is that of the next run
+  // NULL, or the run's half of the word that fft_c2r takes (see czt_fold); the other
+  // half is the next run's
   int* wide;
 };
 

@@ -58,6 +58,49 @@ def test_large_values(F, Nf, Nr):
             assert np.array_equal(run(F, ws, s), good)
 
 
+# a captured run, replayed after other runs have moved on to the other flag
+@pytest.mark.parametrize("Nf", LENGTHS)
+@pytest.mark.parametrize("others", [0, 1, 2])
+def test_overflow_in_a_replay(F, Nf, others):
+    import torch
+    n = np.arange(Nf)
+    x = 1.9e38 / (Nf / 2) * np.cos(2 * np.pi * ((Nf // 2 * n) % Nf) / Nf)
+    big = np.asfortranarray(np.stack([x, -x], axis=1).astype(np.float32))
+    s = synth.spectrogram(Nf, 2, [(Nf * 0.4, 0.5, 25.0)], seed=5)
+    ws = F.ZDTWorkspace(s, 0.0, 1.0, 4)
+    st = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ws.set_stream(st.cuda_stream)
+
+    def run_on(spec):  # on the workspace's stream, which torch's own does not wait for
+        d = F.create_fdr(spec, 4)
+        torch.cuda.synchronize()
+        F.zdtfdr_(d, ws, spec)
+        torch.cuda.synchronize()
+        return d.cpu().numpy()
+
+    s, big = (torch.from_numpy(np.ascontiguousarray(v.T)).cuda().t() for v in (s, big))
+    good = run_on(s)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        F.zdtfdr_(ws)
+    for spec in (big, s, big, s):
+        for _ in range(others):
+            run_on(s)
+        F.input_(ws, spec)
+        torch.cuda.synchronize()
+        g.replay()
+        out = F.create_fdr(s, 4)
+        torch.cuda.synchronize()
+        F.output_(out, ws)
+        torch.cuda.synchronize()
+        out = out.cpu().numpy()
+        if spec is s:
+            assert np.max(np.abs(out - good)) <= 2e-6 * np.max(np.abs(good))
+        else:
+            assert np.isfinite(out[:, 0::2]).all() and not np.isfinite(out[:, 1]).all()
+
+
 @pytest.mark.parametrize("Nf", LENGTHS)
 def test_bad_column_of_Y(F, Nf):
     import torch
