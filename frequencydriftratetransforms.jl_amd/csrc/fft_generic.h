@@ -53,5 +53,8 @@ int fft_r2c(int64_t N, const float* in, int64_t ldi, c32* out, int64_t ldo, int6
 // the other).
 int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int64_t batch, double scale,
             void* s0, void* s1, void* s2, hipStream_t st, int maxr = 16, const int64_t* wide = nullptr);
+// *wide = 0 (a kernel of this file's, which a new workspace's r2c loads anyway: one of
+// another file costs its first use 100 us)
+int fft_clear_wide(int64_t* wide, hipStream_t st);
 
 }  // namespace zdt

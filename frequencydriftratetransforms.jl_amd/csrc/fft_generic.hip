@@ -1281,4 +1281,12 @@ int fft_c2r(int64_t N, const c32* in, int64_t ldi, float* out, int64_t ldo, int6
   return ZDT_OK;
 }
 
+__global__ void clear_wide(int64_t* wide) { *wide = 0; }
+
+int fft_clear_wide(int64_t* wide, hipStream_t st) {
+  clear_wide<<<1, 1, 0, st>>>(wide);
+  ZDT_CHECK_LAUNCH("clear_wide");
+  return ZDT_OK;
+}
+
 }  // namespace zdt

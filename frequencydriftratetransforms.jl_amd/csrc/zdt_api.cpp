@@ -460,7 +460,7 @@ int create_ws_tuned(const float* spec, int64_t Nf, int64_t Nt, float r0, float d
         rc = dev_alloc(ws, reinterpret_cast<void**>(&ws->Ys), static_cast<size_t>(ys_bytes(Nf, Nr)));
       if (rc == ZDT_OK && Nf % 2 != 0) {
         ws->wide = reinterpret_cast<int*>(ws->Ys + ys_stride(ws->Nk) * Nr);
-        rc = launch_set_double(reinterpret_cast<double*>(ws->wide), 0.0, ws->stream);  // both
+        rc = fft_clear_wide(reinterpret_cast<int64_t*>(ws->wide), ws->stream);
       }
       if (rc == ZDT_OK) rc = ensure_scratch(ws, real_scratch_bytes(ws));
     }
